@@ -16,7 +16,7 @@ PKG_DIR = os.path.dirname(os.path.abspath(__file__))
 REPO_DIR = os.path.dirname(PKG_DIR)
 CSRC = os.path.join(PKG_DIR, "csrc")
 # one object per translation unit, compiled in parallel, then linked
-SOURCES = [os.path.join(CSRC, f) for f in ("ma_attn.hip", "encoder_layer.hip")]
+SOURCES = [os.path.join(CSRC, f) for f in ("ma_attn.hip", "flash_attn.hip", "encoder_layer.hip")]
 LIB = os.path.join(PKG_DIR, "libma_attn.so")
 BUILD_DIR = os.path.join(PKG_DIR, "_build")
 ARCH = os.environ.get("MA_ATTN_ARCH", "gfx950")

@@ -1,0 +1,177 @@
+// flash_attn.hip -- launches of the banded MFMA kernels (flash_kernel.h).
+#include "flash_attn.h"
+
+#include <algorithm>
+#include <cmath>
+
+#include "flash_kernel.h"
+#include "host_common.h"
+
+namespace ma_flash {
+
+using namespace ma_dev;
+
+namespace {
+
+bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
+int64_t elt_of(const ma_attn_desc* d) { return d->dtype == MA_ATTN_F32 ? 4 : 2; }
+
+// The band a descriptor maps to, clipped to the sequence.
+struct Band {
+  int64_t left, right, dil, nr;
+};
+bool band_of(const ma_attn_desc* d, Band* b) {
+  if (d->pattern == MA_ATTN_DENSE) {
+    *b = Band{d->seq_len, d->causal ? 0 : d->seq_len, 1, d->seq_len};
+    return true;
+  }
+  if (d->pattern != MA_ATTN_SLIDING || d->left < 0 || d->right < 0) return false;
+  const int64_t nr = (d->seq_len + d->dilation - 1) / d->dilation;
+  *b = Band{std::min(d->left, nr), std::min(d->right, nr), d->dilation, nr};
+  return true;
+}
+
+FlArgs args_of(const ma_attn_desc* d) {
+  Band b;
+  band_of(d, &b);
+  FlArgs a{};
+  a.N = d->seq_len;
+  a.H = (int32_t)d->num_heads;
+  a.D = (int32_t)d->head_dim;
+  a.left = (int32_t)b.left;
+  a.right = (int32_t)b.right;
+  a.dil = (int32_t)b.dil;
+  a.tok_bytes = (uint32_t)(b.dil * d->num_heads * d->head_dim * elt_of(d));
+  a.scale = d->scale > 0.0f ? d->scale : 1.0f / std::sqrt(static_cast<float>(d->head_dim));
+  a.scale_log2 = a.scale * 1.4426950408889634f;
+  // rows that see more of the sequence the later they are run first
+  a.desc = b.left >= b.nr && b.right < b.nr;
+  return a;
+}
+
+template <typename T, int ND, int NQ, int NW, int KB, bool DB, int OCC>
+int run_fwd(const ma_attn_desc* d, FlArgs a, hipStream_t st) {
+  Band b;
+  band_of(d, &b);
+  constexpr int QT = 16 * NQ * NW;
+  constexpr size_t shm = (size_t)(DB ? 2 : 1) * 2 * FlStage<T, ND, KB, NW>::kMat;
+  auto kern = &flash_fwd_kernel<T, ND, NQ, NW, KB, DB, OCC>;
+  if (ma_host::reserve_lds(reinterpret_cast<const void*>(kern), shm, st)) return 1;
+  a.tiles = (int32_t)((b.nr + QT - 1) / QT);
+  const int64_t wgs = d->batch * d->num_heads * b.dil * a.tiles;
+  ma_host::launch(true, kern, dim3((unsigned)wgs), dim3(64 * NW), (uint32_t)shm, st, a);
+  return 0;
+}
+
+// One query group per wave, 4 waves, 64-key blocks in one buffer: measured
+// best of 1 or 2 groups, 4 or 8 waves, 32- or 64-key blocks and one or two
+// buffers at head_dim 32 and 128 (causal 128-key window, bf16, head_dim 128,
+// 8 heads, 32768 rows: 83 us against 87-104; two-sided 64-key window, head_dim
+// 32, 4 x 8 heads, 8191 rows: f16 26 us against 28-31, f32 43 us against
+// 43-70).  float32 above head_dim 64 takes 32-key blocks (three planes of 64
+// rows would leave one workgroup per CU, or spill).
+template <typename T, int ND>
+int fwd_nd(const ma_attn_desc* d, const FlArgs& a, hipStream_t st) {
+  constexpr bool f32 = sizeof(T) == 4;
+  if constexpr (f32 && ND > 2)
+    return run_fwd<T, ND, 1, 4, 32, false, 2>(d, a, st);
+  else
+    return run_fwd<T, ND, 1, 4, 64, false, f32 ? 2 : 3>(d, a, st);
+}
+
+template <typename T>
+int fwd_t(const ma_attn_desc* d, const FlArgs& a, hipStream_t st) {
+  switch ((d->head_dim + 31) / 32) {
+    case 1: return fwd_nd<T, 1>(d, a, st);
+    case 2: return fwd_nd<T, 2>(d, a, st);
+    case 3: return fwd_nd<T, 3>(d, a, st);
+    default: return fwd_nd<T, 4>(d, a, st);
+  }
+}
+
+template <typename T, int ND, int NQ, int NWQ, int NWK, int KB, int OCC>
+int run_bwd(const ma_attn_desc* d, FlArgs a, hipStream_t st) {
+  Band b;
+  band_of(d, &b);
+  constexpr int QT = 16 * NQ * NWQ, KT = 16 * NWK;
+  constexpr size_t shm_q = 2 * FlStage<T, ND, KB, NWQ>::kMat;
+  constexpr size_t shm_k = 2 * FlStage<T, ND, KB, NWK>::kMat + 2 * KB * sizeof(float);
+  auto kq = &flash_dq_kernel<T, ND, NQ, NWQ, KB, OCC, false>;
+  auto kk = &flash_dkv_kernel<T, ND, NWK, KB, OCC>;
+  if (ma_host::reserve_lds(reinterpret_cast<const void*>(kq), shm_q, st) ||
+      ma_host::reserve_lds(reinterpret_cast<const void*>(kk), shm_k, st))
+    return 1;
+  const int64_t streams = d->batch * d->num_heads * b.dil;
+  a.tiles = (int32_t)((b.nr + QT - 1) / QT);
+  ma_host::launch(false, kq, dim3((unsigned)(streams * a.tiles)), dim3(64 * NWQ), (uint32_t)shm_q, st, a);
+  a.tiles = (int32_t)((b.nr + KT - 1) / KT);
+  a.desc = 0;  // key tiles: the first see the most queries
+  ma_host::launch(true, kk, dim3((unsigned)(streams * a.tiles)), dim3(64 * NWK), (uint32_t)shm_k, st, a);
+  return 0;
+}
+
+// 4 waves and 64-row blocks (float32 above head_dim 64: 32-row): measured best
+// of 4 or 8 waves and 32- or 64-row blocks (causal 128-key window, bf16,
+// head_dim 128, 2 x 8 heads, 4096 rows: 74 us against 79-88).
+template <typename T, int ND>
+int bwd_nd(const ma_attn_desc* d, const FlArgs& a, hipStream_t st) {
+  constexpr int KB = sizeof(T) == 4 && ND > 2 ? 32 : 64;
+  return run_bwd<T, ND, 1, 4, 4, KB, 2>(d, a, st);
+}
+
+template <typename T>
+int bwd_t(const ma_attn_desc* d, const FlArgs& a, hipStream_t st) {
+  switch ((d->head_dim + 31) / 32) {
+    case 1: return bwd_nd<T, 1>(d, a, st);
+    case 2: return bwd_nd<T, 2>(d, a, st);
+    case 3: return bwd_nd<T, 3>(d, a, st);
+    default: return bwd_nd<T, 4>(d, a, st);
+  }
+}
+
+}  // namespace
+
+bool applies(const ma_attn_desc* d, const void* const* ptrs, int n) {
+  Band b;
+  if (!band_of(d, &b) || d->head_dim < 8 || d->head_dim > 128 || d->head_dim % 8 != 0) return false;
+  for (int i = 0; i < n; ++i)
+    if (!aligned16(ptrs[i])) return false;
+  const int64_t tb = b.dil * d->num_heads * d->head_dim * elt_of(d);
+  // every byte offset a workgroup forms, and the 16-row tiles' ids
+  return (b.nr + 512) * tb < (1LL << 31) && b.nr < (1LL << 29) &&
+         d->batch * d->num_heads * b.dil * ((b.nr + 15) / 16) <= (int64_t)INT32_MAX;
+}
+
+int forward(const ma_attn_desc* d, const void* q, const void* k, const void* v, void* o, float* lse,
+            hipStream_t st) {
+  FlArgs a = args_of(d);
+  a.q = q;
+  a.k = k;
+  a.v = v;
+  a.o = o;
+  a.lse = lse;
+  switch (d->dtype) {
+    case MA_ATTN_F32: return fwd_t<float>(d, a, st);
+    case MA_ATTN_BF16: return fwd_t<__bf16>(d, a, st);
+    default: return fwd_t<_Float16>(d, a, st);
+  }
+}
+
+int backward(const ma_attn_desc* d, const void* const* ptrs, float* stats, hipStream_t st) {
+  FlArgs a = args_of(d);
+  a.q = ptrs[0];
+  a.k = ptrs[1];
+  a.v = ptrs[2];
+  a.dout = ptrs[3];
+  a.o = const_cast<void*>(ptrs[4]);
+  a.dk = const_cast<void*>(ptrs[5]);
+  a.dv = const_cast<void*>(ptrs[6]);
+  a.stats = stats;
+  switch (d->dtype) {
+    case MA_ATTN_F32: return bwd_t<float>(d, a, st);
+    case MA_ATTN_BF16: return bwd_t<__bf16>(d, a, st);
+    default: return bwd_t<_Float16>(d, a, st);
+  }
+}
+
+}  // namespace ma_flash

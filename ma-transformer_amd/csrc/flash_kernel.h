@@ -1,0 +1,993 @@
+// flash_kernel.h -- banded attention, forward and backward, for head_dims 8 to
+// 128 (a multiple of 8) on 16x16x32 MFMA: windows [i-left, i+right] of any
+// dilation, dense and causal rows (bands as wide as the sequence).
+//
+// float32 is computed on the bf16 matrix cores.  x = x0 + x1 + x2 with x0, x1,
+// x2 the successive bf16 roundings of what is left (24 bits in all, float32's
+// exponent range), and a product takes the six partial products whose bf16
+// planes p, p' have p + p' <= 2, smallest first; the three left out are below
+// 2^-26 of it.  Six 16x16x32 MFMAs take 6/16 of the time of the sixteen
+// 16x16x4 fp32 MFMAs they replace, and 64-term dot products came out closer to
+// 64-bit ones (relative error 4.6e-8 against 1.44e-7 on normal data; 7.7e-8
+// against 1.24e-7 on data spread over e^(+-9)): each MFMA rounds once per 32
+// terms instead of once per term.
+//
+// 16-bit inputs multiply exactly (one plane).  Probabilities and dS are float32
+// and enter their products as a 16-bit value plus its 16-bit remainder (two
+// MFMAs, 16 or more significant bits), so nothing but the stored results is
+// rounded to 16 bits.
+//
+// Operand layouts (lane = 16 g + c).  Row operand: lane (c, g) holds row c at
+// head_dim 32 j + 8 g .. +7 for each j (one 16-byte LDS read, or registers).
+// rows . rows^T of 16 x 16 lands with lane (c, g) holding column c of rows
+// 4 g .. 4 g + 3, which is the B operand of the products with the other
+// matrix's transpose; that transpose is read from the LDS rows by the
+// transpose read (tr_read), two 16-row sub-tiles per MFMA.  A lane ends with
+// head_dim 32 h + 8 g .. +7 of its column for each h.
+//
+// LDS rows are 64 ND + 32 bytes (ND = ceil(head_dim / 32)): the 32-byte pad
+// keeps a transpose read's four rows on disjoint banks.  Columns from head_dim
+// to 32 ND read as zero and are not stored.
+#pragma once
+
+#include "device_common.h"
+
+namespace ma_dev {
+
+struct FlArgs {
+  const void* q;
+  const void* k;
+  const void* v;
+  const void* dout;
+  void* o;          // forward: O; backward: dQ
+  void* dk;
+  void* dv;
+  const void* fo;   // backward from saved statistics: the forward's O
+  float* lse;       // forward: optional statistics out; backward from saved statistics: in ([B*N*H])
+  float* stats;     // backward: {lse2, delta} per row, [B*N*H][2]
+  int64_t N;
+  int32_t H, D, left, right, dil;
+  int32_t tiles;      // tiles of the longest residue class
+  int32_t desc;       // 1: the last tile first (causal rows: longest first)
+  uint32_t tok_bytes; // bytes between consecutive rows of a residue class
+  float scale, scale_log2;
+};
+
+// Element type of the MFMA operands and the number of planes of an input.
+template <typename T>
+struct FlElt {
+  using E = T;
+  static constexpr int NP = 1;
+  static constexpr int NPB = 2;  // planes of a probability or dS operand
+};
+template <>
+struct FlElt<float> {
+  using E = __bf16;
+  static constexpr int NP = 3;
+  static constexpr int NPB = 3;
+};
+
+template <typename E>
+__device__ __forceinline__ float fl_lo(uint32_t w) {
+  if constexpr (__is_same(E, __bf16))
+    return __uint_as_float(w << 16);
+  else
+    return static_cast<float>(__builtin_bit_cast(E, (uint16_t)(w & 0xffffu)));
+}
+template <typename E>
+__device__ __forceinline__ float fl_hi(uint32_t w) {
+  if constexpr (__is_same(E, __bf16))
+    return __uint_as_float(w & 0xffff0000u);
+  else
+    return static_cast<float>(__builtin_bit_cast(E, (uint16_t)(w >> 16)));
+}
+
+// Planes of two values: w[p] holds plane p of both.
+template <typename E, int NPL>
+__device__ __forceinline__ void fl_split2(float x, float y, uint32_t (&w)[NPL]) {
+#pragma unroll
+  for (int p = 0; p < NPL; ++p) {
+    w[p] = Mma<E>::pack2(x, y);
+    if (p + 1 < NPL) {
+      x -= fl_lo<E>(w[p]);
+      y -= fl_hi<E>(w[p]);
+    }
+  }
+}
+
+// The three bf16 planes of 8 floats.  A value that rounds to a bf16 infinity
+// (above 3.39e38, or an infinity itself) is clamped to bf16's largest in its
+// first planes, so that its planes still add up to it.
+__device__ __forceinline__ void fl_split8(const uint4& a, const uint4& b, uint4 (&o)[3]) {
+  float x[8] = {__uint_as_float(a.x), __uint_as_float(a.y), __uint_as_float(a.z), __uint_as_float(a.w),
+                __uint_as_float(b.x), __uint_as_float(b.y), __uint_as_float(b.z), __uint_as_float(b.w)};
+  constexpr float kBig = 3.3895313892515355e38f;  // bf16's largest finite value
+  const float mx = fmaxf(fmaxf(fmaxf(fabsf(x[0]), fabsf(x[1])), fmaxf(fabsf(x[2]), fabsf(x[3]))),
+                         fmaxf(fmaxf(fabsf(x[4]), fabsf(x[5])), fmaxf(fabsf(x[6]), fabsf(x[7]))));
+  uint32_t w[3][4];
+  if (__builtin_expect(__builtin_amdgcn_ballot_w64(mx > kBig) == 0, 1)) {  // NaNs pass: fmaxf skips them
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      uint32_t t[3];
+      fl_split2<__bf16, 3>(x[2 * i], x[2 * i + 1], t);
+      w[0][i] = t[0];
+      w[1][i] = t[1];
+      w[2][i] = t[2];
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      float y = x[2 * i], z = x[2 * i + 1];
+#pragma unroll
+      for (int p = 0; p < 3; ++p) {
+        const float cy = p < 2 && fabsf(y) > kBig ? copysignf(kBig, y) : y;
+        const float cz = p < 2 && fabsf(z) > kBig ? copysignf(kBig, z) : z;
+        w[p][i] = Mma<__bf16>::pack2(cy, cz);
+        y -= fl_lo<__bf16>(w[p][i]);
+        z -= fl_hi<__bf16>(w[p][i]);
+      }
+    }
+  }
+#pragma unroll
+  for (int p = 0; p < 3; ++p) o[p] = make_uint4(w[p][0], w[p][1], w[p][2], w[p][3]);
+}
+
+// ---------------------------------------------------------------- operands
+
+template <int ND>
+constexpr int fl_rs() {
+  return 64 * ND + 32;  // bytes per LDS row of one plane
+}
+
+// A register row operand: row c at head_dim 32 j + 8 g .. +7, per plane.
+template <typename T, int ND>
+struct FlFrag {
+  static constexpr int NP = FlElt<T>::NP;
+  uint4 r[NP][ND];
+  // `row`: byte offset of the row (kOob or past the range: zeros)
+  __device__ __forceinline__ void load(__amdgpu_buffer_rsrc_t rs, uint32_t row, int D, int g) {
+#pragma unroll
+    for (int j = 0; j < ND; ++j) {
+      const int d = 32 * j + 8 * g;
+      const uint32_t off = d < D ? row + (uint32_t)(d * sizeof(T)) : kOob;
+      if constexpr (NP == 1) {
+        r[0][j] = bload16(rs, off);
+      } else {
+        const uint4 a = bload16(rs, off), b = bload16(rs, off + 16);
+        uint4 s[3];
+        fl_split8(a, b, s);
+#pragma unroll
+        for (int p = 0; p < 3; ++p) r[p][j] = s[p];
+      }
+    }
+  }
+};
+
+// R rows of one matrix on their way to LDS: 8-element units, a thread's unit i
+// is number tid + threads * i in row order.
+template <typename T, int ND, int R, int NW>
+struct FlStage {
+  static constexpr int kUnits = R * 4 * ND, kThr = 64 * NW;
+  static constexpr int NU = (kUnits + kThr - 1) / kThr;
+  static constexpr bool kEven = kUnits % kThr == 0;
+  static constexpr int NP = FlElt<T>::NP;
+  static constexpr int RS = fl_rs<ND>();
+  static constexpr int kPlane = R * RS, kMat = NP * kPlane;
+  uint4 r[NU][sizeof(T) == 4 ? 2 : 1];
+  __device__ __forceinline__ void load(__amdgpu_buffer_rsrc_t rs, int row0, int tid, uint32_t tb, int D) {
+#pragma unroll
+    for (int i = 0; i < NU; ++i) {
+      const int u = tid + kThr * i, row = u / (4 * ND), col = u % (4 * ND);
+      const bool ok = (kEven || u < kUnits) && 8 * col < D;
+      const uint32_t off = ok ? (uint32_t)(row0 + row) * tb + (uint32_t)(8 * col * sizeof(T)) : kOob;
+      r[i][0] = bload16(rs, off);
+      if constexpr (sizeof(T) == 4) r[i][1] = bload16(rs, off + 16);
+    }
+  }
+  __device__ __forceinline__ void store(uint8_t* m, int tid) const {
+#pragma unroll
+    for (int i = 0; i < NU; ++i) {
+      const int u = tid + kThr * i, row = u / (4 * ND), col = u % (4 * ND);
+      if (!kEven && u >= kUnits) continue;
+      uint8_t* p = m + row * RS + 16 * col;
+      if constexpr (sizeof(T) == 2) {
+        *reinterpret_cast<uint4*>(p) = r[i][0];
+      } else {
+        uint4 s[3];
+        fl_split8(r[i][0], r[i][1], s);
+#pragma unroll
+        for (int q = 0; q < 3; ++q) *reinterpret_cast<uint4*>(p + q * kPlane) = s[q];
+      }
+    }
+  }
+};
+
+// z[n] = 16 LDS rows (at p, the lane's address in plane 0) . frags[n]^T.
+template <typename T, int ND, int PL, int NF>
+__device__ __forceinline__ void fl_rowdot(const uint8_t* p, const FlFrag<T, ND> (&f)[NF], f32x4 (&z)[NF]) {
+  using E = typename FlElt<T>::E;
+#pragma unroll
+  for (int n = 0; n < NF; ++n) z[n] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  if constexpr (FlElt<T>::NP == 1) {
+#pragma unroll
+    for (int j = 0; j < ND; ++j) {
+      const uint4 a = *reinterpret_cast<const uint4*>(p + 64 * j);
+#pragma unroll
+      for (int n = 0; n < NF; ++n) z[n] = Mma<E>::x32(a, f[n].r[0][j], z[n]);
+    }
+  } else {
+    // LDS planes 2, 1, 0 against register planes with p + p' <= 2, smallest first
+#pragma unroll
+    for (int s = 2; s >= 0; --s)
+#pragma unroll
+      for (int pa = s; pa >= 0; --pa)
+#pragma unroll
+        for (int j = 0; j < ND; ++j) {
+          const uint4 a = *reinterpret_cast<const uint4*>(p + pa * PL + 64 * j);
+#pragma unroll
+          for (int n = 0; n < NF; ++n) z[n] = Mma<E>::x32(a, f[n].r[s - pa][j], z[n]);
+        }
+  }
+}
+
+// B operand planes of two sub-tiles' values (4 per lane each).
+template <typename T>
+struct FlB {
+  static constexpr int NPB = FlElt<T>::NPB;
+  uint4 b[NPB];
+  __device__ __forceinline__ void set(const float (&p0)[4], const float (&p1)[4]) {
+    using E = typename FlElt<T>::E;
+    uint32_t w[4][NPB];
+    fl_split2<E, NPB>(p0[0], p0[1], w[0]);
+    fl_split2<E, NPB>(p0[2], p0[3], w[1]);
+    fl_split2<E, NPB>(p1[0], p1[1], w[2]);
+    fl_split2<E, NPB>(p1[2], p1[3], w[3]);
+#pragma unroll
+    for (int p = 0; p < NPB; ++p) b[p] = make_uint4(w[0][p], w[1][p], w[2][p], w[3][p]);
+  }
+};
+
+// acc[n] += M^T B[n]^T over two 16-row sub-tiles of M: m0, m1 the lane's
+// transpose-read addresses (fl_tr_lane) in their plane 0.
+template <int ND>
+__device__ __forceinline__ uint32_t fl_tr_lane(int c, int g) {
+  return (uint32_t)((4 * g + (c >> 2)) * fl_rs<ND>() + 16 * (c & 3));
+}
+template <typename T, int ND, int PL, int NF>
+__device__ __forceinline__ void fl_trmul(const uint8_t* m0, const uint8_t* m1, const FlB<T> (&b)[NF],
+                                         f32x4 (&acc)[NF][2 * ND]) {
+  using E = typename FlElt<T>::E;
+#pragma unroll
+  for (int dt = 0; dt < 2 * ND; ++dt) {
+    const int o = 64 * (dt >> 1) + 8 * (dt & 1);
+    if constexpr (FlElt<T>::NP == 1) {
+      const uint2 a0 = tr_read(m0 + o), a1 = tr_read(m1 + o);
+      const uint4 a = make_uint4(a0.x, a0.y, a1.x, a1.y);
+#pragma unroll
+      for (int n = 0; n < NF; ++n) {
+        acc[n][dt] = Mma<E>::x32(a, b[n].b[1], acc[n][dt]);  // the remainders, then the values
+        acc[n][dt] = Mma<E>::x32(a, b[n].b[0], acc[n][dt]);
+      }
+    } else {
+      uint4 a[3];
+#pragma unroll
+      for (int p = 0; p < 3; ++p) {
+        const uint2 a0 = tr_read(m0 + p * PL + o), a1 = tr_read(m1 + p * PL + o);
+        a[p] = make_uint4(a0.x, a0.y, a1.x, a1.y);
+      }
+#pragma unroll
+      for (int s = 2; s >= 0; --s)
+#pragma unroll
+        for (int pa = s; pa >= 0; --pa)
+#pragma unroll
+          for (int n = 0; n < NF; ++n) acc[n][dt] = Mma<E>::x32(a[pa], b[n].b[s - pa], acc[n][dt]);
+    }
+  }
+}
+
+// A finished row: acc * s at head_dim 32 h + 8 g .. +7.
+template <typename T, int ND>
+__device__ __forceinline__ void fl_store(const f32x4 (&acc)[2 * ND], float s, __amdgpu_buffer_rsrc_t rs,
+                                         uint32_t row, int D, int g) {
+#pragma unroll
+  for (int h = 0; h < ND; ++h) {
+    const int d = 32 * h + 8 * g;
+    const uint32_t off = d < D ? row + (uint32_t)(d * sizeof(T)) : kOob;
+    const f32x4 x = acc[2 * h] * s, y = acc[2 * h + 1] * s;
+    if constexpr (sizeof(T) == 4) {
+      bstore16(rs, off, __builtin_bit_cast(uint4, x));
+      bstore16(rs, off + 16, __builtin_bit_cast(uint4, y));
+    } else {
+      bstore16(rs, off, make_uint4(Mma<T>::pack2(x[0], x[1]), Mma<T>::pack2(x[2], x[3]), Mma<T>::pack2(y[0], y[1]),
+                                   Mma<T>::pack2(y[2], y[3])));
+    }
+  }
+}
+
+// Whether any of the lane's sums is an infinity or NaN (0 * x is NaN then).
+template <int ND>
+__device__ __forceinline__ bool fl_bad(const f32x4 (&acc)[2 * ND]) {
+  float t = 0.0f;
+#pragma unroll
+  for (int i = 0; i < 2 * ND; ++i)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) t = fmaf(acc[i][r], 0.0f, t);
+  return t != 0.0f;  // true for NaN
+}
+
+// The (batch, head, residue class) stream and tile of a workgroup.
+struct FlPos {
+  int tile, rho, h, b, Nr;
+  int64_t base;  // elements of the stream's first row
+  uint32_t nrec;
+};
+__device__ __forceinline__ FlPos fl_pos(const FlArgs& a, int elt) {
+  FlPos p;
+  int lin = xcd_row_order(blockIdx.x, gridDim.x);
+  p.tile = lin % a.tiles;
+  if (a.desc) p.tile = a.tiles - 1 - p.tile;
+  lin /= a.tiles;
+  p.rho = lin % a.dil;
+  lin /= a.dil;
+  p.h = lin % a.H;
+  p.b = lin / a.H;
+  p.Nr = (int)((a.N - p.rho + a.dil - 1) / a.dil);
+  p.base = (((int64_t)p.b * a.N + p.rho) * a.H + p.h) * a.D;
+  p.nrec = p.Nr > 0 ? (uint32_t)(p.Nr - 1) * a.tok_bytes + (uint32_t)(a.D * elt) : 0u;
+  return p;
+}
+
+__device__ __forceinline__ float fl_wave_sum(float x) {
+#pragma unroll
+  for (int m = 32; m >= 1; m >>= 1) x += __shfl_xor(x, m, 64);
+  return x;
+}
+
+template <typename T>
+__device__ __forceinline__ float fl_at(const T* p, int64_t row, int64_t rs, int d, int D) {
+  return d < D ? static_cast<float>(p[row * rs + d]) : 0.0f;
+}
+
+// ---------------------------------------------------------------- forward
+//
+// One workgroup (NW waves) per 16 NQ NW queries of one stream; a wave holds
+// NQ groups of 16 queries, so that every K and V operand it reads from LDS
+// feeds NQ MFMAs.  Key blocks of KB rows go through LDS (DB: two buffers, the
+// next block's loads in flight while this one computes; otherwise one buffer,
+// refilled between two barriers), softmax online in registers, rescaled only
+// when a row's maximum rose.  16-key sub-tiles outside every window of the
+// wave are skipped.
+//
+// A row whose sums come out infinite or NaN is computed again key by key
+// (fl_fwd_row): a masked key's probability is 0, but 0 times an infinity or
+// NaN in its V row would reach queries that do not attend it.
+template <typename T, int NC>
+__device__ __forceinline__ void fl_fwd_row(const FlArgs& a, const FlPos& ps, int i, int lane) {
+  const int64_t rs = (int64_t)a.dil * a.H * a.D;
+  const T* q = static_cast<const T*>(a.q) + ps.base;
+  const T* k = static_cast<const T*>(a.k) + ps.base;
+  const T* v = static_cast<const T*>(a.v) + ps.base;
+  T* o = static_cast<T*>(a.o) + ps.base;
+  float qd[NC], acc[NC];
+#pragma unroll
+  for (int c = 0; c < NC; ++c) {
+    qd[c] = fl_at(q, i, rs, lane + 64 * c, a.D);
+    acc[c] = 0.0f;
+  }
+  float m = -INFINITY, l = 0.0f;
+  const int j0 = max(0, i - a.left), j1 = min(ps.Nr - 1, i + a.right);
+  for (int j = j0; j <= j1; ++j) {
+    float s = 0.0f;
+#pragma unroll
+    for (int c = 0; c < NC; ++c) s = fmaf(qd[c], fl_at(k, j, rs, lane + 64 * c, a.D), s);
+    s = fl_wave_sum(s) * a.scale;
+    const float mn = fmaxf(m, s);
+    const float mu = mn == -INFINITY ? 0.0f : mn;
+    const float corr = expf(m - mu), p = expf(s - mu);
+    l = fmaf(l, corr, p);
+#pragma unroll
+    for (int c = 0; c < NC; ++c) acc[c] = fmaf(p, fl_at(v, j, rs, lane + 64 * c, a.D), acc[c] * corr);
+    m = mn;
+  }
+  const float inv = l != 0.0f ? 1.0f / l : 0.0f;
+#pragma unroll
+  for (int c = 0; c < NC; ++c)
+    if (lane + 64 * c < a.D) o[i * rs + lane + 64 * c] = static_cast<T>(acc[c] * inv);
+}
+
+template <typename T, int ND, int NQ, int NW, int KB, bool DB, int OCC>
+__global__ __launch_bounds__(64 * NW, OCC) void flash_fwd_kernel(FlArgs a) {
+  extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+  using St = FlStage<T, ND, KB, NW>;
+  constexpr int RS = St::RS, PL = St::kPlane, MAT = St::kMat, BUF = 2 * MAT;
+  constexpr int NU = KB / 16;
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int c = lane & 15, g = lane >> 4;
+  const FlPos ps = fl_pos(a, sizeof(T));
+  const int Nr = ps.Nr, L = a.left, R = a.right, D = a.D;
+  const int q0 = ps.tile * (16 * NQ * NW);
+  if (q0 >= Nr) return;  // uniform per workgroup, before any barrier
+  const uint32_t tb = a.tok_bytes;
+  const __amdgpu_buffer_rsrc_t Qr = make_rsrc(static_cast<const T*>(a.q) + ps.base, ps.nrec);
+  const __amdgpu_buffer_rsrc_t Kr = make_rsrc(static_cast<const T*>(a.k) + ps.base, ps.nrec);
+  const __amdgpu_buffer_rsrc_t Vr = make_rsrc(static_cast<const T*>(a.v) + ps.base, ps.nrec);
+  const __amdgpu_buffer_rsrc_t Or = make_rsrc(static_cast<T*>(a.o) + ps.base, ps.nrec);
+
+  const int qa = q0 + 16 * NQ * wv;  // the wave's first query
+  const int k0 = max(0, q0 - L) & ~15;
+  const int kend = min(Nr, q0 + 16 * NQ * NW + R);
+  const int nb = (kend - k0 + KB - 1) / KB;
+
+  St ks, vs;
+  ks.load(Kr, k0, tid, tb, D);
+  vs.load(Vr, k0, tid, tb, D);
+  FlFrag<T, ND> qf[NQ];
+#pragma unroll
+  for (int n = 0; n < NQ; ++n) qf[n].load(Qr, (uint32_t)(qa + 16 * n + c) * tb, D, g);
+  const uint32_t kl = (uint32_t)(c * RS + 16 * g), vl = (uint32_t)MAT + fl_tr_lane<ND>(c, g);
+
+  float m_run[NQ], l_run[NQ];
+  f32x4 acc[NQ][2 * ND];
+#pragma unroll
+  for (int n = 0; n < NQ; ++n) {
+    m_run[n] = -INFINITY;
+    l_run[n] = 0.0f;
+#pragma unroll
+    for (int d = 0; d < 2 * ND; ++d) acc[n][d] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  }
+  const float sl2 = a.scale_log2;
+  ks.store(lds, tid);
+  vs.store(lds + MAT, tid);
+  __syncthreads();
+
+  for (int e = 0; e < nb; ++e) {
+    if (e + 1 < nb) {
+      ks.load(Kr, k0 + (e + 1) * KB, tid, tb, D);
+      vs.load(Vr, k0 + (e + 1) * KB, tid, tb, D);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    const uint8_t* buf = lds + (DB && (e & 1) ? BUF : 0);
+    const int key0 = k0 + e * KB;
+    // sub-tiles [u0, u1] of the block meet some window of the wave
+    const int u0 = max(0, (qa - L - key0) >> 4);
+    const int u1 = qa < Nr ? min(NU - 1, (min(qa + 16 * NQ - 1 + R, Nr - 1) - key0) >> 4) : -1;
+    if (u0 <= u1) {  // wave-uniform
+      f32x4 sc[NU][NQ];
+      float mx[NQ];
+#pragma unroll
+      for (int n = 0; n < NQ; ++n) mx[n] = -INFINITY;
+#pragma unroll
+      for (int u = 0; u < NU; ++u) {
+        if (u >= u0 && u <= u1) {
+          fl_rowdot<T, ND, PL, NQ>(buf + u * 16 * RS + kl, qf, sc[u]);
+          const int key = key0 + 16 * u;
+#pragma unroll
+          for (int n = 0; n < NQ; ++n) {
+            const int rel = key - (qa + 16 * n);  // key - query offsets span rel -+ 15
+            if (rel - 15 < -L || rel + 15 > R || key + 15 >= Nr) {
+              const int x = rel + 4 * g - c, hi = min(R, Nr - 1 - (qa + 16 * n) - c);
+#pragma unroll
+              for (int r = 0; r < 4; ++r) sc[u][n][r] = x + r >= -L && x + r <= hi ? sc[u][n][r] : -INFINITY;
+            }
+          }
+        } else {
+#pragma unroll
+          for (int n = 0; n < NQ; ++n) sc[u][n] = f32x4{-INFINITY, -INFINITY, -INFINITY, -INFINITY};
+        }
+#pragma unroll
+        for (int n = 0; n < NQ; ++n)
+          mx[n] = fmaxf(mx[n], fmaxf(fmaxf(sc[u][n][0], sc[u][n][1]), fmaxf(sc[u][n][2], sc[u][n][3])));
+      }
+      float mu[NQ];
+      bool rose = false;
+#pragma unroll
+      for (int n = 0; n < NQ; ++n) {
+        mx[n] = fmaxf(m_run[n], col_max(mx[n]));
+        mu[n] = mx[n] == -INFINITY ? 0.0f : mx[n] * sl2;
+        rose = rose || mx[n] != m_run[n];
+      }
+      if (__builtin_amdgcn_ballot_w64(rose) != 0) {
+#pragma unroll
+        for (int n = 0; n < NQ; ++n) {
+          const float corr = __builtin_amdgcn_exp2f(m_run[n] * sl2 - mu[n]);  // 0 on a row's first block
+          l_run[n] *= corr;
+#pragma unroll
+          for (int d = 0; d < 2 * ND; ++d) acc[n][d] *= corr;
+          m_run[n] = mx[n];
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < NU; u += 2) {
+        if (u + 1 < u0 || u > u1) continue;  // wave-uniform
+        FlB<T> pb[NQ];
+#pragma unroll
+        for (int n = 0; n < NQ; ++n) {
+          float p0[4], p1[4];
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            p0[r] = __builtin_amdgcn_exp2f(fmaf(sc[u][n][r], sl2, -mu[n]));
+            p1[r] = __builtin_amdgcn_exp2f(fmaf(sc[u + 1][n][r], sl2, -mu[n]));
+            l_run[n] += p0[r] + p1[r];
+          }
+          pb[n].set(p0, p1);
+        }
+        fl_trmul<T, ND, PL, NQ>(buf + u * 16 * RS + vl, buf + (u + 1) * 16 * RS + vl, pb, acc);
+      }
+    }
+    if constexpr (DB) {
+      if (e + 1 < nb) {
+        uint8_t* nx = lds + (e & 1 ? 0 : BUF);
+        ks.store(nx, tid);
+        vs.store(nx + MAT, tid);
+      }
+      __syncthreads();
+    } else if (e + 1 < nb) {
+      __syncthreads();
+      ks.store(lds, tid);
+      vs.store(lds + MAT, tid);
+      __syncthreads();
+    }
+  }
+
+  if (qa >= Nr) return;  // no barrier below
+#pragma unroll
+  for (int n = 0; n < NQ; ++n) {
+    const float l_tot = col_sum(l_run[n]);
+    const float inv = l_tot != 0.0f ? 1.0f / l_tot : 0.0f;
+    const int i = qa + 16 * n + c;
+    // bit r of each lane group: row r is left to fl_fwd_row
+    const uint64_t bad = __builtin_amdgcn_ballot_w64(i < Nr && (fl_bad<ND>(acc[n]) || !(l_tot < INFINITY)));
+    const bool own_bad = (bad >> c & 0x0001000100010001ull) != 0;
+    fl_store<T, ND>(acc[n], inv, Or, own_bad ? kOob : (uint32_t)i * tb, D, g);
+    if (a.lse && g == 0 && i < Nr)
+      a.lse[((int64_t)ps.b * a.N + ps.rho + (int64_t)a.dil * i) * a.H + ps.h] =
+          l_tot > 0.0f ? m_run[n] * sl2 + __log2f(l_tot) : 0.0f;
+    if (__builtin_expect(bad != 0, 0)) {
+      for (int r = 0; r < 16; ++r)
+        if (bad >> r & 0x0001000100010001ull) fl_fwd_row<T, (ND + 1) / 2>(a, ps, qa + 16 * n + r, lane);
+    }
+  }
+}
+
+// ---------------------------------------------------------------- backward
+//
+// Two launches: dQ (and each row's statistics) by query tiles, then dK and dV
+// by key tiles.  With p_ij = 2^(s_ij sl2 - lse2_i), dp_ij = dO_i . V_j,
+// delta_i = sum_j p_ij dp_ij and ds_ij = p_ij (dp_ij - delta_i):
+// dQ_i = scale sum_j ds_ij K_j, dK_j = scale sum_i ds_ij Q_i,
+// dV_j = sum_i p_ij dO_i.  Each output row has one writer.
+//
+// As in the forward, a row whose sums come out infinite or NaN is computed
+// again over its own set alone.
+template <typename T, int NC>
+__device__ __forceinline__ void fl_dq_row(const FlArgs& a, const FlPos& ps, int i, float lse2, float dlt, int lane) {
+  const int64_t rs = (int64_t)a.dil * a.H * a.D;
+  const T* q = static_cast<const T*>(a.q) + ps.base;
+  const T* k = static_cast<const T*>(a.k) + ps.base;
+  const T* v = static_cast<const T*>(a.v) + ps.base;
+  const T* go = static_cast<const T*>(a.dout) + ps.base;
+  T* dq = static_cast<T*>(a.o) + ps.base;
+  float qd[NC], gd[NC], acc[NC];
+#pragma unroll
+  for (int c = 0; c < NC; ++c) {
+    qd[c] = fl_at(q, i, rs, lane + 64 * c, a.D);
+    gd[c] = fl_at(go, i, rs, lane + 64 * c, a.D);
+    acc[c] = 0.0f;
+  }
+  const int j0 = max(0, i - a.left), j1 = min(ps.Nr - 1, i + a.right);
+  for (int j = j0; j <= j1; ++j) {
+    float s = 0.0f, dp = 0.0f;
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+      s = fmaf(qd[c], fl_at(k, j, rs, lane + 64 * c, a.D), s);
+      dp = fmaf(gd[c], fl_at(v, j, rs, lane + 64 * c, a.D), dp);
+    }
+    s = fl_wave_sum(s);
+    dp = fl_wave_sum(dp);
+    const float ds = __builtin_amdgcn_exp2f(fmaf(s, a.scale_log2, -lse2)) * (dp - dlt);
+#pragma unroll
+    for (int c = 0; c < NC; ++c) acc[c] = fmaf(ds, fl_at(k, j, rs, lane + 64 * c, a.D), acc[c]);
+  }
+#pragma unroll
+  for (int c = 0; c < NC; ++c)
+    if (lane + 64 * c < a.D) dq[i * rs + lane + 64 * c] = static_cast<T>(acc[c] * a.scale);
+}
+
+template <typename T, int NC>
+__device__ __forceinline__ void fl_dkv_row(const FlArgs& a, const FlPos& ps, int j, int lane) {
+  const int64_t rs = (int64_t)a.dil * a.H * a.D;
+  const T* q = static_cast<const T*>(a.q) + ps.base;
+  const T* k = static_cast<const T*>(a.k) + ps.base;
+  const T* v = static_cast<const T*>(a.v) + ps.base;
+  const T* go = static_cast<const T*>(a.dout) + ps.base;
+  float kd[NC], vd[NC], dk[NC], dv[NC];
+#pragma unroll
+  for (int c = 0; c < NC; ++c) {
+    kd[c] = fl_at(k, j, rs, lane + 64 * c, a.D);
+    vd[c] = fl_at(v, j, rs, lane + 64 * c, a.D);
+    dk[c] = dv[c] = 0.0f;
+  }
+  const int i0 = max(0, j - a.right), i1 = min(ps.Nr - 1, j + a.left);
+  for (int i = i0; i <= i1; ++i) {
+    const int64_t row = ((int64_t)ps.b * a.N + ps.rho + (int64_t)a.dil * i) * a.H + ps.h;
+    float s = 0.0f, dp = 0.0f, qd[NC], gd[NC];
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+      qd[c] = fl_at(q, i, rs, lane + 64 * c, a.D);
+      gd[c] = fl_at(go, i, rs, lane + 64 * c, a.D);
+      s = fmaf(qd[c], kd[c], s);
+      dp = fmaf(gd[c], vd[c], dp);
+    }
+    s = fl_wave_sum(s);
+    dp = fl_wave_sum(dp);
+    const float p = __builtin_amdgcn_exp2f(fmaf(s, a.scale_log2, -a.stats[2 * row]));
+    const float ds = p * (dp - a.stats[2 * row + 1]);
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+      dv[c] = fmaf(p, gd[c], dv[c]);
+      dk[c] = fmaf(ds, qd[c], dk[c]);
+    }
+  }
+  T* ok = static_cast<T*>(a.dk) + ps.base;
+  T* ov = static_cast<T*>(a.dv) + ps.base;
+#pragma unroll
+  for (int c = 0; c < NC; ++c)
+    if (lane + 64 * c < a.D) {
+      ok[j * rs + lane + 64 * c] = static_cast<T>(dk[c] * a.scale);
+      ov[j * rs + lane + 64 * c] = static_cast<T>(dv[c]);
+    }
+}
+
+// dQ of 16 NQ NW queries.  Pass 1 over the key blocks: the online softmax's
+// maximum, sum and sum of e dp.  Pass 2, backwards over the same blocks (the
+// last one is still in LDS): p, ds, dQ^T += K^T ds^T.  SAVED: the forward's
+// statistics are read and delta = dO . O, so only the second pass runs.
+template <typename T, int ND, int NQ, int NW, int KB, int OCC, bool SAVED>
+__global__ __launch_bounds__(64 * NW, OCC) void flash_dq_kernel(FlArgs a) {
+  extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+  using St = FlStage<T, ND, KB, NW>;
+  constexpr int RS = St::RS, PL = St::kPlane, MAT = St::kMat;
+  constexpr int NU = KB / 16;
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int c = lane & 15, g = lane >> 4;
+  const FlPos ps = fl_pos(a, sizeof(T));
+  const int Nr = ps.Nr, L = a.left, R = a.right, D = a.D;
+  const int q0 = ps.tile * (16 * NQ * NW);
+  if (q0 >= Nr) return;  // uniform per workgroup, before any barrier
+  const uint32_t tb = a.tok_bytes;
+  const __amdgpu_buffer_rsrc_t Qr = make_rsrc(static_cast<const T*>(a.q) + ps.base, ps.nrec);
+  const __amdgpu_buffer_rsrc_t Gr = make_rsrc(static_cast<const T*>(a.dout) + ps.base, ps.nrec);
+  const __amdgpu_buffer_rsrc_t Kr = make_rsrc(static_cast<const T*>(a.k) + ps.base, ps.nrec);
+  const __amdgpu_buffer_rsrc_t Vr = make_rsrc(static_cast<const T*>(a.v) + ps.base, ps.nrec);
+  const __amdgpu_buffer_rsrc_t Or = make_rsrc(static_cast<T*>(a.o) + ps.base, ps.nrec);
+
+  const int qa = q0 + 16 * NQ * wv;
+  const int k0 = max(0, q0 - L) & ~15;
+  const int kend = min(Nr, q0 + 16 * NQ * NW + R);
+  const int nb = (kend - k0 + KB - 1) / KB;
+  const int steps = SAVED ? nb : 2 * nb;
+  auto block_at = [&](int e) { return !SAVED && e < nb ? e : steps - 1 - e; };
+
+  St ks, vs;
+  ks.load(Kr, k0 + block_at(0) * KB, tid, tb, D);
+  vs.load(Vr, k0 + block_at(0) * KB, tid, tb, D);
+  FlFrag<T, ND> qf[NQ], gf[NQ];
+  float m[NQ], l[NQ], dl[NQ];  // pass 1: maximum, sum, sum of e dp; then mu, 1/sum, delta
+  const float sl2 = a.scale_log2;
+#pragma unroll
+  for (int n = 0; n < NQ; ++n) {
+    const uint32_t row = (uint32_t)(qa + 16 * n + c) * tb;
+    qf[n].load(Qr, row, D, g);
+    gf[n].load(Gr, row, D, g);
+    m[n] = -INFINITY;
+    l[n] = dl[n] = 0.0f;
+    if constexpr (SAVED) {
+      const __amdgpu_buffer_rsrc_t Fr = make_rsrc(static_cast<const T*>(a.fo) + ps.base, ps.nrec);
+      FlFrag<T, ND> of;
+      of.load(Fr, row, D, g);
+      using E = typename FlElt<T>::E;
+      float d = 0.0f;
+#pragma unroll
+      for (int j = 0; j < ND; ++j)
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+          float x0 = 0.0f, x1 = 0.0f, y0 = 0.0f, y1 = 0.0f;  // planes add up exactly, smallest first
+#pragma unroll
+          for (int p = FlElt<T>::NP - 1; p >= 0; --p) {
+            const uint32_t gw = reinterpret_cast<const uint32_t*>(&gf[n].r[p][j])[w];
+            const uint32_t ow = reinterpret_cast<const uint32_t*>(&of.r[p][j])[w];
+            x0 += fl_lo<E>(gw);
+            x1 += fl_hi<E>(gw);
+            y0 += fl_lo<E>(ow);
+            y1 += fl_hi<E>(ow);
+          }
+          d = fmaf(x0, y0, d);
+          d = fmaf(x1, y1, d);
+        }
+      dl[n] = col_sum(d);
+      const int i = qa + 16 * n + c;
+      m[n] = i < Nr ? a.lse[((int64_t)ps.b * a.N + ps.rho + (int64_t)a.dil * i) * a.H + ps.h] : 0.0f;
+      l[n] = 1.0f;
+    }
+  }
+  const uint32_t rl = (uint32_t)(c * RS + 16 * g), tl = fl_tr_lane<ND>(c, g);
+  f32x4 acc[NQ][2 * ND];
+#pragma unroll
+  for (int n = 0; n < NQ; ++n)
+#pragma unroll
+    for (int d = 0; d < 2 * ND; ++d) acc[n][d] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  ks.store(lds, tid);
+  vs.store(lds + MAT, tid);
+  __syncthreads();
+
+  // S and dP of sub-tile u of the block at key0, pairs outside the band
+  // masked (their V row may hold anything: dP 0)
+  auto scores = [&](int u, int key0, f32x4 (&sc)[NQ], f32x4 (&dp)[NQ]) {
+    fl_rowdot<T, ND, PL, NQ>(lds + u * 16 * RS + rl, qf, sc);
+    fl_rowdot<T, ND, PL, NQ>(lds + MAT + u * 16 * RS + rl, gf, dp);
+    const int key = key0 + 16 * u;
+#pragma unroll
+    for (int n = 0; n < NQ; ++n) {
+      const int rel = key - (qa + 16 * n);
+      if (rel - 15 < -L || rel + 15 > R || key + 15 >= Nr) {
+        const int x = rel + 4 * g - c, hi = min(R, Nr - 1 - (qa + 16 * n) - c);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const bool in = x + r >= -L && x + r <= hi;
+          sc[n][r] = in ? sc[n][r] : -INFINITY;
+          dp[n][r] = in ? dp[n][r] : 0.0f;
+        }
+      }
+    }
+  };
+
+  for (int e = 0; e < steps; ++e) {
+    const bool turn = !SAVED && e == nb - 1;  // the next step works on the same block
+    const bool more = e + 1 < steps && !turn;
+    if (more) {
+      ks.load(Kr, k0 + block_at(e + 1) * KB, tid, tb, D);
+      vs.load(Vr, k0 + block_at(e + 1) * KB, tid, tb, D);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    const int key0 = k0 + block_at(e) * KB;
+    const int u0 = max(0, (qa - L - key0) >> 4);
+    const int u1 = qa < Nr ? min(NU - 1, (min(qa + 16 * NQ - 1 + R, Nr - 1) - key0) >> 4) : -1;
+    if (!SAVED && e < nb) {
+#pragma unroll
+      for (int u = 0; u < NU; ++u) {
+        if (u < u0 || u > u1) continue;  // wave-uniform
+        f32x4 sc[NQ], dp[NQ];
+        scores(u, key0, sc, dp);
+#pragma unroll
+        for (int n = 0; n < NQ; ++n) {
+          const float mn =
+              fmaxf(m[n], col_max(fmaxf(fmaxf(sc[n][0], sc[n][1]), fmaxf(sc[n][2], sc[n][3]))));
+          const float mu = mn == -INFINITY ? 0.0f : mn * sl2;
+          const float corr = __builtin_amdgcn_exp2f(m[n] * sl2 - mu);
+          l[n] *= corr;
+          dl[n] *= corr;
+          m[n] = mn;
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const float p = __builtin_amdgcn_exp2f(fmaf(sc[n][r], sl2, -mu));
+            l[n] += p;
+            dl[n] = fmaf(p, dp[n][r], dl[n]);
+          }
+        }
+      }
+      if (e == nb - 1) {
+#pragma unroll
+        for (int n = 0; n < NQ; ++n) {
+          const float lt = col_sum(l[n]), dt = col_sum(dl[n]);
+          const float mu = m[n] == -INFINITY ? 0.0f : m[n] * sl2;
+          l[n] = lt != 0.0f ? 1.0f / lt : 0.0f;
+          dl[n] = dt * l[n];
+          const int i = qa + 16 * n + c;
+          if (g == 0 && i < Nr) {
+            const int64_t row = ((int64_t)ps.b * a.N + ps.rho + (int64_t)a.dil * i) * a.H + ps.h;
+            *reinterpret_cast<f32x2*>(a.stats + 2 * row) = f32x2{lt != 0.0f ? mu + __log2f(lt) : 0.0f, dl[n]};
+          }
+          m[n] = mu;
+        }
+      }
+    } else {
+#pragma unroll
+      for (int u = 0; u < NU; u += 2) {
+        if (u + 1 < u0 || u > u1) continue;  // wave-uniform
+        f32x4 sc[2][NQ], dp[2][NQ];
+#pragma unroll
+        for (int w = 0; w < 2; ++w) {
+          if (u + w >= u0 && u + w <= u1)
+            scores(u + w, key0, sc[w], dp[w]);
+          else
+#pragma unroll
+            for (int n = 0; n < NQ; ++n) {
+              sc[w][n] = f32x4{-INFINITY, -INFINITY, -INFINITY, -INFINITY};
+              dp[w][n] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+            }
+        }
+        FlB<T> db[NQ];
+#pragma unroll
+        for (int n = 0; n < NQ; ++n) {
+          float ds[2][4];
+#pragma unroll
+          for (int w = 0; w < 2; ++w)
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+              ds[w][r] = __builtin_amdgcn_exp2f(fmaf(sc[w][n][r], sl2, -m[n])) * l[n] * (dp[w][n][r] - dl[n]);
+          db[n].set(ds[0], ds[1]);
+        }
+        fl_trmul<T, ND, PL, NQ>(lds + u * 16 * RS + tl, lds + (u + 1) * 16 * RS + tl, db, acc);
+      }
+    }
+    if (more) {
+      __syncthreads();
+      ks.store(lds, tid);
+      vs.store(lds + MAT, tid);
+      __syncthreads();
+    }
+  }
+
+  if (qa >= Nr) return;  // no barrier below
+#pragma unroll
+  for (int n = 0; n < NQ; ++n) {
+    const int i = qa + 16 * n + c;
+    if constexpr (SAVED) {  // the dK, dV kernel reads {lse2, delta}
+      if (g == 0 && i < Nr) {
+        const int64_t row = ((int64_t)ps.b * a.N + ps.rho + (int64_t)a.dil * i) * a.H + ps.h;
+        *reinterpret_cast<f32x2*>(a.stats + 2 * row) = f32x2{m[n], dl[n]};
+      }
+    }
+    const uint64_t bad = __builtin_amdgcn_ballot_w64(i < Nr && fl_bad<ND>(acc[n]));
+    const bool own_bad = (bad >> c & 0x0001000100010001ull) != 0;
+    fl_store<T, ND>(acc[n], a.scale, Or, own_bad ? kOob : (uint32_t)i * tb, D, g);
+    if (__builtin_expect(bad != 0, 0)) {
+      for (int r = 0; r < 16; ++r)
+        if (bad >> r & 0x0001000100010001ull) {
+          const float mu = __shfl(m[n], r, 64), inv = __shfl(l[n], r, 64), dd = __shfl(dl[n], r, 64);
+          fl_dq_row<T, (ND + 1) / 2>(a, ps, qa + 16 * n + r, mu - __log2f(inv), dd, lane);
+        }
+    }
+  }
+}
+
+// dK, dV of 16 NW keys: a wave holds 16 keys' K and V rows as register
+// operands; blocks of QB query rows (Q, dO and their statistics) go through
+// LDS.  S and dP land with lane (c, g) holding queries 4 g .. 4 g + 3 of key c.
+template <typename T, int ND, int NW, int QB, int OCC>
+__global__ __launch_bounds__(64 * NW, OCC) void flash_dkv_kernel(FlArgs a) {
+  extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+  using St = FlStage<T, ND, QB, NW>;
+  constexpr int RS = St::RS, PL = St::kPlane, MAT = St::kMat;
+  constexpr int NU = QB / 16;
+  float* lst = reinterpret_cast<float*>(lds + 2 * MAT);  // QB lse2, then QB delta
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int c = lane & 15, g = lane >> 4;
+  const FlPos ps = fl_pos(a, sizeof(T));
+  const int Nr = ps.Nr, L = a.left, R = a.right, D = a.D;
+  const int j0 = ps.tile * (16 * NW);
+  if (j0 >= Nr) return;  // uniform per workgroup, before any barrier
+  const uint32_t tb = a.tok_bytes;
+  const __amdgpu_buffer_rsrc_t Qr = make_rsrc(static_cast<const T*>(a.q) + ps.base, ps.nrec);
+  const __amdgpu_buffer_rsrc_t Gr = make_rsrc(static_cast<const T*>(a.dout) + ps.base, ps.nrec);
+  const __amdgpu_buffer_rsrc_t Kr = make_rsrc(static_cast<const T*>(a.k) + ps.base, ps.nrec);
+  const __amdgpu_buffer_rsrc_t Vr = make_rsrc(static_cast<const T*>(a.v) + ps.base, ps.nrec);
+  const __amdgpu_buffer_rsrc_t dKr = make_rsrc(static_cast<T*>(a.dk) + ps.base, ps.nrec);
+  const __amdgpu_buffer_rsrc_t dVr = make_rsrc(static_cast<T*>(a.dv) + ps.base, ps.nrec);
+
+  const int ja = j0 + 16 * wv;  // the wave's first key
+  const int i0 = max(0, j0 - R) & ~15;
+  const int iend = min(Nr, j0 + 16 * NW + L);
+  const int nb = (iend - i0 + QB - 1) / QB;
+
+  St qs, gs;
+  f32x2 st;
+  auto load_stats = [&](int r0) {  // threads 0 .. QB-1; rows past the end get p = 0
+    const int i = r0 + tid;
+    st = f32x2{INFINITY, 0.0f};
+    if (tid < QB && i < Nr)
+      st = *reinterpret_cast<const f32x2*>(a.stats +
+                                           2 * (((int64_t)ps.b * a.N + ps.rho + (int64_t)a.dil * i) * a.H + ps.h));
+  };
+  auto store_stats = [&]() {
+    if (tid < QB) {
+      lst[tid] = st[0];
+      lst[QB + tid] = st[1];
+    }
+  };
+  qs.load(Qr, i0, tid, tb, D);
+  gs.load(Gr, i0, tid, tb, D);
+  load_stats(i0);
+  FlFrag<T, ND> kf[1], vf[1];
+  kf[0].load(Kr, (uint32_t)(ja + c) * tb, D, g);
+  vf[0].load(Vr, (uint32_t)(ja + c) * tb, D, g);
+  const uint32_t rl = (uint32_t)(c * RS + 16 * g), tl = fl_tr_lane<ND>(c, g);
+  const float sl2 = a.scale_log2;
+  f32x4 ak[1][2 * ND], av[1][2 * ND];
+#pragma unroll
+  for (int d = 0; d < 2 * ND; ++d) ak[0][d] = av[0][d] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  qs.store(lds, tid);
+  gs.store(lds + MAT, tid);
+  store_stats();
+  __syncthreads();
+
+  for (int e = 0; e < nb; ++e) {
+    const bool more = e + 1 < nb;
+    if (more) {
+      qs.load(Qr, i0 + (e + 1) * QB, tid, tb, D);
+      gs.load(Gr, i0 + (e + 1) * QB, tid, tb, D);
+      load_stats(i0 + (e + 1) * QB);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    const int r0 = i0 + e * QB;
+    // query sub-tiles [u0, u1] see some key of the wave: i in [ja - R, ja + 15 + L]
+    const int u0 = max(0, (ja - R - r0) >> 4);
+    const int u1 = ja < Nr ? min(NU - 1, (min(ja + 15 + L, Nr - 1) - r0) >> 4) : -1;
+#pragma unroll
+    for (int u = 0; u < NU; u += 2) {
+      if (u + 1 < u0 || u > u1) continue;  // wave-uniform
+      float p[2][4], ds[2][4];
+#pragma unroll
+      for (int w = 0; w < 2; ++w) {
+        if (u + w >= u0 && u + w <= u1) {
+          f32x4 sc[1], dp[1];
+          fl_rowdot<T, ND, PL, 1>(lds + (u + w) * 16 * RS + rl, kf, sc);
+          fl_rowdot<T, ND, PL, 1>(lds + MAT + (u + w) * 16 * RS + rl, vf, dp);
+          const int qb = r0 + 16 * (u + w);
+          const int rel = ja - qb;  // key - query offsets span rel -+ 15
+          const f32x4 ls = *reinterpret_cast<const f32x4*>(lst + 16 * (u + w) + 4 * g);
+          const f32x4 dt = *reinterpret_cast<const f32x4*>(lst + QB + 16 * (u + w) + 4 * g);
+          if (rel - 15 < -L || rel + 15 > R) {
+            const int x = rel + c - 4 * g;  // key - query of element 0
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+              const bool in = x - r >= -L && x - r <= R;
+              sc[0][r] = in ? sc[0][r] : -INFINITY;
+              dp[0][r] = in ? dp[0][r] : dt[r];
+            }
+          }
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            p[w][r] = __builtin_amdgcn_exp2f(fmaf(sc[0][r], sl2, -ls[r]));
+            ds[w][r] = p[w][r] * (dp[0][r] - dt[r]);
+          }
+        } else {
+#pragma unroll
+          for (int r = 0; r < 4; ++r) p[w][r] = ds[w][r] = 0.0f;
+        }
+      }
+      FlB<T> b[1];
+      b[0].set(p[0], p[1]);
+      fl_trmul<T, ND, PL, 1>(lds + MAT + u * 16 * RS + tl, lds + MAT + (u + 1) * 16 * RS + tl, b, av);
+      b[0].set(ds[0], ds[1]);
+      fl_trmul<T, ND, PL, 1>(lds + u * 16 * RS + tl, lds + (u + 1) * 16 * RS + tl, b, ak);
+    }
+    if (more) {
+      __syncthreads();
+      qs.store(lds, tid);
+      gs.store(lds + MAT, tid);
+      store_stats();
+      __syncthreads();
+    }
+  }
+
+  if (ja >= Nr) return;  // no barrier below
+  const int j = ja + c;
+  const uint64_t bad = __builtin_amdgcn_ballot_w64(j < Nr && (fl_bad<ND>(ak[0]) || fl_bad<ND>(av[0])));
+  const bool own_bad = (bad >> c & 0x0001000100010001ull) != 0;
+  const uint32_t row = own_bad ? kOob : (uint32_t)j * tb;
+  fl_store<T, ND>(ak[0], a.scale, dKr, row, D, g);
+  fl_store<T, ND>(av[0], 1.0f, dVr, row, D, g);
+  if (__builtin_expect(bad != 0, 0)) {
+    for (int r = 0; r < 16; ++r)
+      if (bad >> r & 0x0001000100010001ull) fl_dkv_row<T, (ND + 1) / 2>(a, ps, ja + r, lane);
+  }
+}
+
+}  // namespace ma_dev

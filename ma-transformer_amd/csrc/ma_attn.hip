@@ -40,6 +40,8 @@
 #include "../../include/ma_attn.h"
 #include "../../include/ma_features.h"
 #include "device_common.h"
+#include "flash_attn.h"
+#include "host_common.h"
 #include "pattern.h"
 #include "stream_kernel.h"
 #include "block_kernel.h"
@@ -56,9 +58,11 @@
 // the stream's device (hipGetSymbolAddress, once per device).
 static __device__ __align__(256) unsigned char scratch[MA_ATTN_NOALLOC_SCRATCH_BYTES];
 
-namespace {
+// The library's one error channel, shared with the other translation units
+// (ma_attn_last_error() reads it).
+static thread_local std::string g_last_error;
 
-thread_local std::string g_last_error;
+namespace ma_host {
 
 int fail(const char* fmt, ...) {
   char buf[512];
@@ -70,17 +74,22 @@ int fail(const char* fmt, ...) {
   return 1;
 }
 
-}  // namespace
-
-// The library's one error channel, shared with the other translation units
-// (ma_attn_last_error() reads it).
-namespace ma_host {
 void clear_error() { g_last_error.clear(); }
 int set_error(const char* msg) {
   g_last_error = msg;
   return 1;
 }
+
+thread_local hipEvent_t g_ev_start = nullptr;
+thread_local hipEvent_t g_ev_stop = nullptr;
+
 }  // namespace ma_host
+
+using ma_host::fail;
+using ma_host::g_ev_start;
+using ma_host::g_ev_stop;
+using ma_host::launch;
+using ma_host::reserve_lds;
 
 namespace {
 
@@ -121,8 +130,10 @@ int stream_device(hipStream_t st, int* dev) {
   return 0;
 }
 
-// Raises a kernel's dynamic-LDS limit to `shm` bytes once per (kernel,
-// device), with that device current; safe from any number of threads.
+}  // namespace
+
+namespace ma_host {
+
 int reserve_lds(const void* kern, size_t shm, hipStream_t st) {
   int dev = 0;
   if (stream_device(st, &dev)) return 1;
@@ -140,28 +151,11 @@ int reserve_lds(const void* kern, size_t shm, hipStream_t st) {
   return 0;
 }
 
+}  // namespace ma_host
+
+namespace {
+
 using namespace ma_dev;
-
-// ------------------------------------------------------------------ launches
-//
-// Events of the current ma_attn_*_timed call (null otherwise): the call's
-// first kernel takes the start event and its last kernel the stop event, so
-// they bracket the kernels' own execution (hipExtLaunchKernel stamps them on
-// the dispatch packets; no extra queue packets).
-thread_local hipEvent_t g_ev_start = nullptr;
-thread_local hipEvent_t g_ev_stop = nullptr;
-
-template <typename F, typename... Args>
-void launch(bool last, F kernel, dim3 grid, dim3 block, uint32_t shm, hipStream_t st, Args... args) {
-  hipEvent_t e0 = g_ev_start, e1 = last ? g_ev_stop : nullptr;
-  if (e0 || e1) {
-    g_ev_start = nullptr;
-    if (last) g_ev_stop = nullptr;
-    hipExtLaunchKernelGGL(kernel, grid, block, shm, st, e0, e1, 0u, args...);
-  } else {
-    hipLaunchKernelGGL(kernel, grid, block, shm, st, args...);
-  }
-}
 
 // ------------------------------------------------------------------ element access
 
@@ -2138,6 +2132,17 @@ int ma_attn_forward_noalloc(const ma_attn_desc* desc, const void* q, const void*
 
 namespace {
 
+// Bands at head_dims other than 64 (8 to 128, a multiple of 8) on the MFMA
+// kernels of flash_kernel.h, in both directions; head_dim 64 has kernels of its
+// own.  At head_dim 128 in bf16 the row kernels took 2740 us for a causal
+// 128-key window over 8 heads of 32768 rows, these take 83 us (backward over
+// 2 x 8 heads of 4096 rows: 3017 -> 74 us); at head_dim 32 the narrow kernel
+// took 174 us for a two-sided 64-key window over 4 x 8 heads of 8191 rows (f16),
+// these 26 us, and 10.4 against 9.0 us on 4 heads of 1024 rows of 16.
+bool flash_route(const ma_attn_desc* d, const void* const* ptrs, int n) {
+  return d->head_dim != kHeadDim && ma_flash::applies(d, ptrs, n);
+}
+
 // lse: optional per-row softmax statistics (ma_attn_forward_lse), written by
 // the block-row, tiled and Longformer stream kernels; other kernels refuse
 // it.
@@ -2154,7 +2159,10 @@ int forward_launch(const ma_attn_desc* desc, const void* q, const void* k, const
       !(stream && desc->pattern == MA_ATTN_LONGFORMER && desc->num_global > 0))
     return fail("ma_attn_forward_lse: these kernels write no statistics (block-sparse, dense, Longformer "
                 "with 1 to 16 global tokens and index sets with a tile plan do, at head_dim 64)");
-  if (stream) {
+  const bool flash = !want_rows && !want_band && flash_route(desc, qkvo, 4);
+  if (flash) {
+    rc = ma_flash::forward(desc, q, k, v, o, lse, st);
+  } else if (stream) {
     rc = launch_stream(desc, q, k, v, o, lse, workspace, workspace_bytes, st);
   } else if (block) {
     rc = launch_block(desc, q, k, v, o, lse, st);
@@ -2289,6 +2297,13 @@ int ma_attn_backward(const ma_attn_desc* desc, const void* q, const void* k, con
          : desc->dtype == MA_ATTN_F16
              ? launch_tiles_bwd<HalfPath<_Float16>>(desc, ptrs, workspace, st, nullptr, nullptr)
              : launch_tiles_bwd<F32BwdPath>(desc, ptrs, workspace, st, nullptr, nullptr);
+    if (rc) return rc;
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return fail("ma_attn_backward: kernel launch failed: %s", hipGetErrorString(e));
+    return 0;
+  }
+  if (!g_opt.force_rows && flash_route(desc, ptrs, 7)) {
+    rc = ma_flash::backward(desc, ptrs, reinterpret_cast<float*>(stats), st);
     if (rc) return rc;
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return fail("ma_attn_backward: kernel launch failed: %s", hipGetErrorString(e));

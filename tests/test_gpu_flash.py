@@ -1,0 +1,96 @@
+"""Bands at head_dims 8 to 128 on the MFMA kernels of flash_kernel.h, forward
+and backward, against the oracle.
+
+Lengths around the 16-row sub-tiles and 64-row tiles and blocks, head_dims
+around the 32-column steps (padded columns, odd multiples of 8), windows
+narrower and wider than a block, dilations and dense rows.  Tolerances: the
+parity suites' (forward 1e-5 in fp32, gradients per check_grad); 16-bit forward
+rows are rounded once from fp32 sums, so they lie within one unit of the last
+place (2^-8 bf16, 2^-11 f16) plus 1e-4 for the rounding boundary.
+"""
+import numpy as np
+import pytest
+import torch
+
+from conftest import check_grad, qkv, randn
+
+pytestmark = pytest.mark.gpu
+
+DTYPES = [torch.float32, torch.bfloat16, torch.float16]
+
+# N, D, left, right, dilation; left None: dense, causal when right == 0
+SHAPES = [
+    (1, 8, 3, 3, 1), (63, 16, 63, 0, 1), (64, 128, 127, 0, 1), (65, 32, 32, 31, 1), (130, 40, 5, 70, 1),
+    (257, 96, 100, 17, 2), (300, 120, 200, 0, 3), (191, 72, 0, 64, 1), (513, 24, 16, 15, 1),
+    (129, 128, None, 0, 1), (200, 80, None, 1, 1), (321, 32, None, 0, 1),
+]
+
+
+@pytest.fixture(scope="module")
+def ext():
+    if not torch.cuda.is_available():
+        pytest.skip("no HIP device")
+    import sparse_attention_cuda
+    return sparse_attention_cuda
+
+
+def _spec(oracle, shape, left, right, dil):
+    if left is None:
+        return oracle.Spec(*shape, pattern="dense", causal=right == 0)
+    return oracle.Spec(*shape, pattern="sliding", left=left, right=right, dilation=dil)
+
+
+@pytest.mark.parametrize("N,D,left,right,dil", SHAPES)
+@pytest.mark.parametrize("dtype", DTYPES)
+def test_flash_against_oracle(ext, oracle, N, D, left, right, dil, dtype):
+    shape = (2, N, 3, D)
+    arrs = [*qkv(shape, 8000 + N + D), randn(shape, 8100 + N)]
+    q, k, v, g = (torch.from_numpy(a).to(dtype).cuda() for a in arrs)
+    up = [t.float().cpu().numpy() for t in (q, k, v, g)]
+    spec = _spec(oracle, shape, left, right, dil)
+    if left is None:
+        y, grads = ext.dense_forward(q, k, v, right == 0), ext.dense_backward(q, k, v, g, right == 0)
+    else:
+        y, grads = ext.sliding_forward(q, k, v, left, right, dil), ext.sliding_backward(q, k, v, g, left, right, dil)
+    ref = oracle.forward(spec, *up[:3])
+    ulp = {torch.float32: 0.0, torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}[dtype]
+    err = np.abs(y.float().cpu().numpy() - ref)
+    assert (err <= (1e-5 if dtype == torch.float32 else 1e-4) + ulp * np.abs(ref)).all(), float(err.max())
+    for name, a, b in zip("qkv", grads, oracle.backward(spec, *up)):
+        check_grad("d" + name, a.float().cpu().numpy(), b, dtype == torch.float32)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("bad", [float("nan"), float("inf")])
+def test_flash_keeps_bad_values_to_their_rows(ext, dtype, bad):
+    """An infinity or NaN in one key's V row reaches the queries that attend
+    it and no other: the rest of the output, and the dK, dV rows that none of
+    those queries attends, are as without it."""
+    N, left, right, key = 200, 20, 7, 90
+    arrs = [*qkv((1, N, 2, 96), 8300), randn((1, N, 2, 96), 8304)]
+    q, k, v, g = (torch.from_numpy(a).to(dtype).cuda() for a in arrs)
+    v2 = v.clone()
+    v2[0, key, 1, 5] = bad
+    y, y2 = (ext.sliding_forward(q, k, x, left, right) for x in (v, v2))
+    sees = torch.zeros(N, dtype=torch.bool, device="cuda")
+    sees[key - right:key + left + 1] = True  # query i attends [i - left, i + right]
+    assert not torch.isfinite(y2[0, sees, 1, 5]).any()
+    tol = 1e-5 if dtype == torch.float32 else 1e-2
+    torch.testing.assert_close(y2[0, ~sees], y[0, ~sees], rtol=tol, atol=tol)
+    torch.testing.assert_close(y2[0, :, 0], y[0, :, 0], rtol=0, atol=0)  # the other head: untouched
+    d1, d2 = (ext.sliding_backward(q, k, x, g, left, right) for x in (v, v2))
+    far = torch.ones(N, dtype=torch.bool, device="cuda")
+    far[key - right - left:key + left + right + 1] = False
+    torch.testing.assert_close(d2[0][0, ~sees], d1[0][0, ~sees], rtol=tol, atol=tol)
+    for a, b in zip(d2[1:], d1[1:]):
+        torch.testing.assert_close(a[0, far], b[0, far], rtol=tol, atol=tol)
+
+
+def test_flash_float32_extremes(ext):
+    """float32 values near the largest finite one (above bf16's) and tiny ones
+    pass through the three-plane products: one attended key gives O = V."""
+    v = torch.tensor([3.4e38, -3.39e38, 1e-30, 3.0e38, -1e-20, 1.5, 3.3895314e38, -3.4028234e38], device="cuda")
+    q = torch.zeros(1, 70, 1, 8, device="cuda")
+    V = v.repeat(1, 70, 1, 1)
+    o = ext.sliding_forward(q, q, V, 0, 0)
+    torch.testing.assert_close(o, V, rtol=2e-7, atol=0)
