@@ -70,13 +70,54 @@ int run_fwd(const ma_attn_desc* d, FlArgs a, hipStream_t st) {
 // 32, 4 x 8 heads, 8191 rows: f16 26 us against 28-31, f32 43 us against
 // 43-70).  float32 above head_dim 64 takes 32-key blocks (three planes of 64
 // rows would leave one workgroup per CU, or spill).
+// Causal rows, the longest and the shortest tile of a stream in one workgroup.
+template <typename T, int ND, int NW, int KB>
+int run_pair(const ma_attn_desc* d, FlArgs a, hipStream_t st) {
+  Band b;
+  band_of(d, &b);
+  constexpr int QT = 16 * NW;
+  constexpr size_t shm = 2 * FlStage<T, ND, KB, NW>::kMat;
+  auto kern = &flash_pair_fwd_kernel<T, ND, 1, NW, KB, FlElt<T>::NPB>;
+  if (ma_host::reserve_lds(reinterpret_cast<const void*>(kern), shm, st)) return 1;
+  a.desc = 0;
+  a.tiles = (int32_t)((b.nr + QT - 1) / QT);
+  const int64_t wgs = d->batch * d->num_heads * b.dil * a.tiles;
+  ma_host::launch(true, kern, dim3((unsigned)wgs), dim3(64 * NW), (uint32_t)shm, st, a);
+  return 0;
+}
+
+// One query group per wave, 4 waves, 64-key blocks in one buffer: measured
+// best of 1 or 2 groups, 4 or 8 waves, 32- or 64-key blocks and one or two
+// buffers at head_dim 32 and 128 (causal 128-key window, bf16, head_dim 128,
+// 8 heads, 32768 rows: 83 us against 87-104; two-sided 64-key window, head_dim
+// 32, 4 x 8 heads, 8191 rows: f16 26 us against 28-31, f32 43 us against
+// 43-70).  float32 above head_dim 64 takes 32-key blocks (three planes of 64
+// rows would leave one workgroup per CU, or spill).
+//
+// Causal rows whose 128-row tiles are at most one per CU run in pairs, longest
+// with shortest (float32, head_dim 64, 8 heads of 4000 rows: 136 us against
+// 173 unpaired; above one tile per CU the scheduler evens the tiles out: 8000
+// rows 415 us unpaired, 442 paired).
+//
+// float32 at head_dim 33 to 64 splits every staged row into three planes, so 8
+// waves share a block once there are workgroups enough for every CU (two-sided
+// 129-key window, 8 heads of 32768 rows: 82 us against 102 with 4 waves; 2
+// heads of 600 rows: 14.7 against 11.8), and two query groups per wave pay on
+// very long rows (causal, 8 heads of 16384 rows: 1275 us against 1387; 8000
+// rows: 558 against 415).
 template <typename T, int ND>
 int fwd_nd(const ma_attn_desc* d, const FlArgs& a, hipStream_t st) {
   constexpr bool f32 = sizeof(T) == 4;
-  if constexpr (f32 && ND > 2)
-    return run_fwd<T, ND, 1, 4, 32, false, 2>(d, a, st);
-  else
-    return run_fwd<T, ND, 1, 4, 64, false, f32 ? 2 : 3>(d, a, st);
+  constexpr int KB = f32 && ND > 2 ? 32 : 64;
+  Band b;
+  band_of(d, &b);
+  const int64_t tiles128 = d->batch * d->num_heads * b.dil * ((b.nr + 127) / 128);
+  if (a.desc && tiles128 <= 256) return run_pair<T, ND, 8, KB>(d, a, st);
+  if constexpr (f32 && ND == 2) {
+    if (b.left >= b.nr && tiles128 >= 1024) return run_fwd<T, ND, 2, 8, KB, false, 2>(d, a, st);
+    if (tiles128 >= 256) return run_fwd<T, ND, 1, 8, KB, false, 2>(d, a, st);
+  }
+  return run_fwd<T, ND, 1, 4, KB, false, f32 ? 2 : 3>(d, a, st);
 }
 
 template <typename T>
@@ -89,14 +130,14 @@ int fwd_t(const ma_attn_desc* d, const FlArgs& a, hipStream_t st) {
   }
 }
 
-template <typename T, int ND, int NQ, int NWQ, int NWK, int KB, int OCC>
+template <typename T, int ND, int NQ, int NWQ, int NWK, int KB, int OCC, bool SAVED>
 int run_bwd(const ma_attn_desc* d, FlArgs a, hipStream_t st) {
   Band b;
   band_of(d, &b);
   constexpr int QT = 16 * NQ * NWQ, KT = 16 * NWK;
   constexpr size_t shm_q = 2 * FlStage<T, ND, KB, NWQ>::kMat;
   constexpr size_t shm_k = 2 * FlStage<T, ND, KB, NWK>::kMat + 2 * KB * sizeof(float);
-  auto kq = &flash_dq_kernel<T, ND, NQ, NWQ, KB, OCC, false>;
+  auto kq = &flash_dq_kernel<T, ND, NQ, NWQ, KB, OCC, SAVED>;
   auto kk = &flash_dkv_kernel<T, ND, NWK, KB, OCC>;
   if (ma_host::reserve_lds(reinterpret_cast<const void*>(kq), shm_q, st) ||
       ma_host::reserve_lds(reinterpret_cast<const void*>(kk), shm_k, st))
@@ -116,7 +157,9 @@ int run_bwd(const ma_attn_desc* d, FlArgs a, hipStream_t st) {
 template <typename T, int ND>
 int bwd_nd(const ma_attn_desc* d, const FlArgs& a, hipStream_t st) {
   constexpr int KB = sizeof(T) == 4 && ND > 2 ? 32 : 64;
-  return run_bwd<T, ND, 1, 4, 4, KB, 2>(d, a, st);
+  if constexpr (sizeof(T) == 4 && ND == 2)  // saved statistics: head_dim 64
+    if (a.fo) return run_bwd<T, ND, 1, 4, 4, KB, 2, true>(d, a, st);
+  return run_bwd<T, ND, 1, 4, 4, KB, 2, false>(d, a, st);
 }
 
 template <typename T>
@@ -157,7 +200,8 @@ int forward(const ma_attn_desc* d, const void* q, const void* k, const void* v, 
   }
 }
 
-int backward(const ma_attn_desc* d, const void* const* ptrs, float* stats, hipStream_t st) {
+int backward(const ma_attn_desc* d, const void* const* ptrs, float* stats, const void* fo, const float* lse,
+             hipStream_t st) {
   FlArgs a = args_of(d);
   a.q = ptrs[0];
   a.k = ptrs[1];
@@ -167,6 +211,8 @@ int backward(const ma_attn_desc* d, const void* const* ptrs, float* stats, hipSt
   a.dk = const_cast<void*>(ptrs[5]);
   a.dv = const_cast<void*>(ptrs[6]);
   a.stats = stats;
+  a.fo = fo;
+  a.lse = const_cast<float*>(lse);
   switch (d->dtype) {
     case MA_ATTN_F32: return bwd_t<float>(d, a, st);
     case MA_ATTN_BF16: return bwd_t<__bf16>(d, a, st);

@@ -231,9 +231,8 @@ __device__ __forceinline__ void fl_rowdot(const uint8_t* p, const FlFrag<T, ND> 
 }
 
 // B operand planes of two sub-tiles' values (4 per lane each).
-template <typename T>
+template <typename T, int NPB = FlElt<T>::NPB>
 struct FlB {
-  static constexpr int NPB = FlElt<T>::NPB;
   uint4 b[NPB];
   __device__ __forceinline__ void set(const float (&p0)[4], const float (&p1)[4]) {
     using E = typename FlElt<T>::E;
@@ -253,8 +252,8 @@ template <int ND>
 __device__ __forceinline__ uint32_t fl_tr_lane(int c, int g) {
   return (uint32_t)((4 * g + (c >> 2)) * fl_rs<ND>() + 16 * (c & 3));
 }
-template <typename T, int ND, int PL, int NF>
-__device__ __forceinline__ void fl_trmul(const uint8_t* m0, const uint8_t* m1, const FlB<T> (&b)[NF],
+template <typename T, int ND, int PL, int NF, int NPB = FlElt<T>::NPB>
+__device__ __forceinline__ void fl_trmul(const uint8_t* m0, const uint8_t* m1, const FlB<T, NPB> (&b)[NF],
                                          f32x4 (&acc)[NF][2 * ND]) {
   using E = typename FlElt<T>::E;
 #pragma unroll
@@ -265,8 +264,8 @@ __device__ __forceinline__ void fl_trmul(const uint8_t* m0, const uint8_t* m1, c
       const uint4 a = make_uint4(a0.x, a0.y, a1.x, a1.y);
 #pragma unroll
       for (int n = 0; n < NF; ++n) {
-        acc[n][dt] = Mma<E>::x32(a, b[n].b[1], acc[n][dt]);  // the remainders, then the values
-        acc[n][dt] = Mma<E>::x32(a, b[n].b[0], acc[n][dt]);
+#pragma unroll
+        for (int p = NPB - 1; p >= 0; --p) acc[n][dt] = Mma<E>::x32(a, b[n].b[p], acc[n][dt]);  // remainders first
       }
     } else {
       uint4 a[3];
@@ -395,6 +394,8 @@ __device__ __forceinline__ void fl_fwd_row(const FlArgs& a, const FlPos& ps, int
     if (lane + 64 * c < a.D) o[i * rs + lane + 64 * c] = static_cast<T>(acc[c] * inv);
 }
 
+constexpr float kSlack = 8.0f;
+
 template <typename T, int ND, int NQ, int NW, int KB, bool DB, int OCC>
 __global__ __launch_bounds__(64 * NW, OCC) void flash_fwd_kernel(FlArgs a) {
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
@@ -455,7 +456,7 @@ __global__ __launch_bounds__(64 * NW, OCC) void flash_fwd_kernel(FlArgs a) {
     const int u1 = qa < Nr ? min(NU - 1, (min(qa + 16 * NQ - 1 + R, Nr - 1) - key0) >> 4) : -1;
     if (u0 <= u1) {  // wave-uniform
       f32x4 sc[NU][NQ];
-      float mx[NQ];
+      float mx[NQ], mu[NQ];
 #pragma unroll
       for (int n = 0; n < NQ; ++n) mx[n] = -INFINITY;
 #pragma unroll
@@ -476,17 +477,21 @@ __global__ __launch_bounds__(64 * NW, OCC) void flash_fwd_kernel(FlArgs a) {
 #pragma unroll
           for (int n = 0; n < NQ; ++n) sc[u][n] = f32x4{-INFINITY, -INFINITY, -INFINITY, -INFINITY};
         }
+      }
+#pragma unroll
+      for (int u = 0; u < NU; ++u)
 #pragma unroll
         for (int n = 0; n < NQ; ++n)
           mx[n] = fmaxf(mx[n], fmaxf(fmaxf(sc[u][n][0], sc[u][n][1]), fmaxf(sc[u][n][2], sc[u][n][3])));
-      }
-      float mu[NQ];
       bool rose = false;
 #pragma unroll
       for (int n = 0; n < NQ; ++n) {
-        mx[n] = fmaxf(m_run[n], col_max(mx[n]));
+        // a maximum up to 2^kSlack times the running one (in weights) keeps it
+        mx[n] = col_max(mx[n]);
+        const bool up = !(mx[n] * sl2 <= fmaf(m_run[n], sl2, kSlack));
+        mx[n] = up ? fmaxf(m_run[n], mx[n]) : m_run[n];
         mu[n] = mx[n] == -INFINITY ? 0.0f : mx[n] * sl2;
-        rose = rose || mx[n] != m_run[n];
+        rose = rose || up;
       }
       if (__builtin_amdgcn_ballot_w64(rose) != 0) {
 #pragma unroll
@@ -538,6 +543,218 @@ __global__ __launch_bounds__(64 * NW, OCC) void flash_fwd_kernel(FlArgs a) {
     const float inv = l_tot != 0.0f ? 1.0f / l_tot : 0.0f;
     const int i = qa + 16 * n + c;
     // bit r of each lane group: row r is left to fl_fwd_row
+    const uint64_t bad = __builtin_amdgcn_ballot_w64(i < Nr && (fl_bad<ND>(acc[n]) || !(l_tot < INFINITY)));
+    const bool own_bad = (bad >> c & 0x0001000100010001ull) != 0;
+    fl_store<T, ND>(acc[n], inv, Or, own_bad ? kOob : (uint32_t)i * tb, D, g);
+    if (a.lse && g == 0 && i < Nr)
+      a.lse[((int64_t)ps.b * a.N + ps.rho + (int64_t)a.dil * i) * a.H + ps.h] =
+          l_tot > 0.0f ? m_run[n] * sl2 + __log2f(l_tot) : 0.0f;
+    if (__builtin_expect(bad != 0, 0)) {
+      for (int r = 0; r < 16; ++r)
+        if (bad >> r & 0x0001000100010001ull) fl_fwd_row<T, (ND + 1) / 2>(a, ps, qa + 16 * n + r, lane);
+    }
+  }
+}
+
+// ---------------------------------------------------------------- forward, paired tiles
+//
+// Causal (and other one-sided, sequence-wide) rows on few tiles: a launch lasts
+// as long as its longest row of blocks.  The first half of the waves takes tile
+// p, the second half tile T - 1 - p, so that every workgroup has the same
+// number of (wave, block) products and each SIMD holds a wave of either tile;
+// both walk the key blocks from 0 and share them.  The long tile's wave is
+// alone on its SIMD for most of them, so a block's two halves overlap: while
+// block e's scores turn into probabilities (VALU), the products of block e + 1
+// with the queries run on the matrix cores.  K is therefore one block ahead of
+// V in LDS (one buffer each, refilled between two barriers from loads issued a
+// block earlier).  float32, head_dim 64, 8 heads of 4096 rows: 138 us, against
+// 170-190 us unpaired and 214 us on the fp32 matrix cores.
+//
+// NPB: planes of a probability.
+__device__ __forceinline__ float fl_max(float a, float b) { return __builtin_elementwise_maximum(a, b); }
+
+template <typename T, int ND, int NQ, int NW, int KB, int NPB>
+__global__ __launch_bounds__(64 * NW, 2) void flash_pair_fwd_kernel(FlArgs a) {
+  extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+  using St = FlStage<T, ND, KB, NW>;
+  constexpr int RS = St::RS, PL = St::kPlane, MAT = St::kMat;
+  constexpr int NU = KB / 16;
+  constexpr int QT = 16 * NQ * NW;
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int c = lane & 15, g = lane >> 4;
+  const FlPos ps = fl_pos(a, sizeof(T));
+  const int Nr = ps.Nr, L = a.left, R = a.right, D = a.D;
+  constexpr int HT = QT / 2;
+  const int T2 = (Nr + HT - 1) / HT, lo = ps.tile, hi = T2 - 1 - ps.tile;
+  if (lo > hi) return;  // uniform per workgroup, before any barrier
+  const bool second = wv >= NW / 2;
+  int qa = (second ? hi : lo) * HT + 16 * NQ * (wv % (NW / 2));  // the wave's first query
+  if (second && lo == hi) qa = Nr;  // the middle tile of an odd count: one half is enough
+  const int qmin = lo * HT, qmax = hi * HT + HT - 1;
+  const uint32_t tb = a.tok_bytes;
+  const __amdgpu_buffer_rsrc_t Qr = make_rsrc(static_cast<const T*>(a.q) + ps.base, ps.nrec);
+  const __amdgpu_buffer_rsrc_t Kr = make_rsrc(static_cast<const T*>(a.k) + ps.base, ps.nrec);
+  const __amdgpu_buffer_rsrc_t Vr = make_rsrc(static_cast<const T*>(a.v) + ps.base, ps.nrec);
+  const __amdgpu_buffer_rsrc_t Or = make_rsrc(static_cast<T*>(a.o) + ps.base, ps.nrec);
+  const int k0 = max(0, qmin - L) & ~15;
+  const int kend = min(Nr, qmax + R + 1);
+  const int nb = (kend - k0 + KB - 1) / KB;
+
+  St ks, vs;
+  ks.load(Kr, k0, tid, tb, D);
+  FlFrag<T, ND> qf[NQ];
+#pragma unroll
+  for (int n = 0; n < NQ; ++n) qf[n].load(Qr, (uint32_t)(qa + 16 * n + c) * tb, D, g);
+  const uint32_t kl = (uint32_t)(c * RS + 16 * g), vl = (uint32_t)MAT + fl_tr_lane<ND>(c, g);
+  float m_run[NQ], l_run[NQ];
+  f32x4 acc[NQ][2 * ND];
+#pragma unroll
+  for (int n = 0; n < NQ; ++n) {
+    m_run[n] = -INFINITY;
+    l_run[n] = 0.0f;
+#pragma unroll
+    for (int d = 0; d < 2 * ND; ++d) acc[n][d] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  }
+  const float sl2 = a.scale_log2;
+
+  // block e holds a pair of the wave's band / only pairs of it
+  auto live = [&](int e) {
+    const int key0 = k0 + e * KB;
+    return e < nb && qa < Nr && key0 + KB - 1 >= qa - L && key0 <= min(qa + 16 * NQ - 1 + R, Nr - 1);
+  };
+  auto full = [&](int e) {
+    const int key0 = k0 + e * KB;
+    return e < nb && qa < Nr && key0 >= qa + 16 * NQ - 1 - L && key0 + KB - 1 <= min(qa + R, Nr - 1);
+  };
+  auto products = [&](f32x4 (&sc)[NU][NQ]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < NU; ++u) fl_rowdot<T, ND, PL, NQ>(lds + u * 16 * RS + kl, qf, sc[u]);
+  };
+  auto masks = [&](int e, f32x4 (&sc)[NU][NQ]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int n = 0; n < NQ; ++n) {
+      const int i = qa + 16 * n + c, x = k0 + e * KB + 4 * g - i;  // key - query of element 0
+      const int hi = min(R, Nr - 1 - i);
+#pragma unroll
+      for (int u = 0; u < NU; ++u)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int d = x + 16 * u + r;
+          sc[u][n][r] = d >= -L && d <= hi ? sc[u][n][r] : -INFINITY;
+        }
+    }
+  };
+  // the online softmax of a block's scores: a row's maximum moves only when
+  // some score's weight would pass 2^kSlack times the largest so far
+  auto weights = [&](f32x4 (&sc)[NU][NQ], float (&mu)[NQ]) __attribute__((always_inline)) {
+    bool rose = false;
+    float mn[NQ];
+#pragma unroll
+    for (int n = 0; n < NQ; ++n) {
+      float mx = fl_max(fl_max(sc[0][n][0], sc[0][n][1]), fl_max(sc[0][n][2], sc[0][n][3]));
+#pragma unroll
+      for (int u = 1; u < NU; ++u)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) mx = fl_max(mx, sc[u][n][r]);
+      mx = col_max(mx);
+      const bool up = !(mx * sl2 <= fmaf(m_run[n], sl2, kSlack));
+      mn[n] = up ? fmaxf(m_run[n], mx) : m_run[n];
+      mu[n] = mn[n] == -INFINITY ? 0.0f : mn[n] * sl2;
+      rose = rose || up;
+    }
+    if (__builtin_amdgcn_ballot_w64(rose) != 0) {
+#pragma unroll
+      for (int n = 0; n < NQ; ++n) {
+        const float corr = __builtin_amdgcn_exp2f(m_run[n] * sl2 - mu[n]);  // 0 on a row's first block
+        l_run[n] *= corr;
+#pragma unroll
+        for (int d = 0; d < 2 * ND; ++d) acc[n][d] *= corr;
+        m_run[n] = mn[n];
+      }
+    }
+  };
+  auto apply = [&](f32x4 (&sc)[NU][NQ], const float (&mu)[NQ], FlB<T, NPB> (&pb)[NU / 2][NQ])
+                   __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < NU; u += 2)
+#pragma unroll
+      for (int n = 0; n < NQ; ++n) {
+        float p0[4], p1[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          p0[r] = __builtin_amdgcn_exp2f(fmaf(sc[u][n][r], sl2, -mu[n]));
+          p1[r] = __builtin_amdgcn_exp2f(fmaf(sc[u + 1][n][r], sl2, -mu[n]));
+          l_run[n] += p0[r] + p1[r];
+        }
+        pb[u / 2][n].set(p0, p1);
+      }
+  };
+  auto values = [&](const FlB<T, NPB> (&pb)[NU / 2][NQ]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < NU; u += 2)
+      fl_trmul<T, ND, PL, NQ, NPB>(lds + u * 16 * RS + vl, lds + (u + 1) * 16 * RS + vl, pb[u / 2], acc);
+  };
+
+  f32x4 sa[NU][NQ], sb[NU][NQ];
+  ks.store(lds, tid);
+  __syncthreads();
+  ks.load(Kr, k0 + KB, tid, tb, D);
+  vs.load(Vr, k0, tid, tb, D);
+  if (live(0)) {
+    products(sa);
+    masks(0, sa);
+  }
+  __syncthreads();
+  ks.store(lds, tid);
+  vs.store(lds + MAT, tid);
+  __syncthreads();
+
+  auto step = [&](int e, f32x4 (&cur)[NU][NQ], f32x4 (&nxt)[NU][NQ]) __attribute__((always_inline)) {
+    ks.load(Kr, k0 + (e + 2) * KB, tid, tb, D);
+    vs.load(Vr, k0 + (e + 1) * KB, tid, tb, D);
+    __builtin_amdgcn_sched_barrier(0);
+    const bool lv = live(e);
+    if (lv && full(e + 1)) {  // wave-uniform
+      float mu[NQ];
+      FlB<T, NPB> pb[NU / 2][NQ];
+      weights(cur, mu);
+      products(nxt);
+      apply(cur, mu, pb);
+      values(pb);
+    } else {
+      if (lv) {
+        float mu[NQ];
+        FlB<T, NPB> pb[NU / 2][NQ];
+        weights(cur, mu);
+        apply(cur, mu, pb);
+        values(pb);
+      }
+      if (live(e + 1)) {
+        products(nxt);
+        masks(e + 1, nxt);
+      }
+    }
+    if (e + 1 < nb) {
+      __syncthreads();
+      ks.store(lds, tid);
+      vs.store(lds + MAT, tid);
+      __syncthreads();
+    }
+  };
+  for (int e = 0; e < nb; e += 2) {
+    step(e, sa, sb);
+    if (e + 1 >= nb) break;
+    step(e + 1, sb, sa);
+  }
+
+  if (qa >= Nr) return;  // no barrier below
+#pragma unroll
+  for (int n = 0; n < NQ; ++n) {
+    const float l_tot = col_sum(l_run[n]);
+    const float inv = l_tot != 0.0f ? 1.0f / l_tot : 0.0f;
+    const int i = qa + 16 * n + c;
     const uint64_t bad = __builtin_amdgcn_ballot_w64(i < Nr && (fl_bad<ND>(acc[n]) || !(l_tot < INFINITY)));
     const bool own_bad = (bad >> c & 0x0001000100010001ull) != 0;
     fl_store<T, ND>(acc[n], inv, Or, own_bad ? kOob : (uint32_t)i * tb, D, g);

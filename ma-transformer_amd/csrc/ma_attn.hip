@@ -1620,6 +1620,38 @@ bool bwd_mfma_applies(const ma_attn_desc* d, const void* const* ptrs) {
          d->batch * d->num_heads * dil * tiles <= (int64_t)INT32_MAX;
 }
 
+// Bands that meet at most two 64-row blocks in both directions (on the stream
+// kernels' shifted grids, whose blocks start at row -16*(ceil(L/16) & 3) for
+// keys and -16*(ceil(R/16) & 3) for queries).
+bool bwd_two_blocks(int64_t L, int64_t R) {
+  const int64_t obq = -16 * (((L + 15) / 16) & 3), obkv = -16 * (((R + 15) / 16) & 3);
+  return ma::floordiv64(63 + R - obq, 64) - ma::floordiv64(-L - obq, 64) + 1 <= 2 &&
+         ma::floordiv64(63 + L - obkv, 64) - ma::floordiv64(-R - obkv, 64) + 1 <= 2;
+}
+
+// Whether a band runs on the MFMA kernels of flash_kernel.h.
+//
+// Head_dims other than 64 (8 to 128, a multiple of 8): in both directions.  In
+// bf16 at head_dim 128 the row kernels took 2740 us for a causal 128-key window
+// over 8 heads of 32768 rows, these take 83 us (backward over 2 x 8 heads of
+// 4096 rows: 3017 -> 74 us); at head_dim 32 the narrow kernel took 174 us for a
+// two-sided 64-key window over 4 x 8 heads of 8191 rows (f16), these 26 us, and
+// 10.4 against 9.0 us on 4 heads of 1024 rows of 16.
+//
+// float32 at head_dim 64: dense rows, windows of more than 65 keys forward, and
+// windows past two 64-row blocks backward; shorter ones stay on the stream
+// kernels, which read every row once and keep a tile's scores in registers
+// (8 heads of 32768 rows, stream / these: [i-63, i] forward 65 / 62 us,
+// backward 234 / 263; [i-100, i] 114 / 80 and 466 / 344; [i-64, i+64] 121 / 82
+// and 490 / 361; dense causal, 8 heads of 4000 rows: 211 / 136 and 924 / 594).
+bool flash_route(const ma_attn_desc* d, const void* const* ptrs, int n, bool backward) {
+  if (!ma_flash::applies(d, ptrs, n)) return false;
+  if (d->head_dim != kHeadDim) return true;
+  if (d->dtype != MA_ATTN_F32) return false;
+  if (d->pattern == MA_ATTN_DENSE) return true;
+  return backward ? !bwd_two_blocks(d->left, d->right) : d->left + d->right > 64;
+}
+
 // The fused backward's chunks of a stream's tiles, fitted to one round of the
 // resident workgroups (two per CU).
 void fused_chunks(BwdArgs& a, int64_t streams) {
@@ -1664,11 +1696,7 @@ int launch_backward_mfma(const ma_attn_desc* d, const void* const* ptrs, float* 
   const size_t shm_q = 2 * (size_t)PairLds<P>::kBytes, shm_kv = 2 * ((size_t)PairLds<P>::kBytes + 512);
   // Bands that meet at most two 64-row blocks in both directions stream a
   // chunk of tiles per workgroup; wider bands take one workgroup per tile.
-  // The stream kernels' blocks start at row -16*(ceil(L/16) & 3) (keys) and
-  // -16*(ceil(R/16) & 3) (queries), which fits [i-32, i+31] in two.
-  const int64_t obq = -16 * (((L + 15) / 16) & 3), obkv = -16 * (((R + 15) / 16) & 3);
-  const bool chunked = ma::floordiv64(63 + R - obq, 64) - ma::floordiv64(-L - obq, 64) + 1 <= 2 &&
-                       ma::floordiv64(63 + L - obkv, 64) - ma::floordiv64(-R - obkv, 64) + 1 <= 2;
+  const bool chunked = bwd_two_blocks(L, R);
   // fixed-window instantiations: causal 64 (also per residue class of a dilated window)
   // and [i-32, i+31] (cfg 2)
   const bool no_fixed = g_opt.bwd_no_fixed;
@@ -2132,17 +2160,6 @@ int ma_attn_forward_noalloc(const ma_attn_desc* desc, const void* q, const void*
 
 namespace {
 
-// Bands at head_dims other than 64 (8 to 128, a multiple of 8) on the MFMA
-// kernels of flash_kernel.h, in both directions; head_dim 64 has kernels of its
-// own.  At head_dim 128 in bf16 the row kernels took 2740 us for a causal
-// 128-key window over 8 heads of 32768 rows, these take 83 us (backward over
-// 2 x 8 heads of 4096 rows: 3017 -> 74 us); at head_dim 32 the narrow kernel
-// took 174 us for a two-sided 64-key window over 4 x 8 heads of 8191 rows (f16),
-// these 26 us, and 10.4 against 9.0 us on 4 heads of 1024 rows of 16.
-bool flash_route(const ma_attn_desc* d, const void* const* ptrs, int n) {
-  return d->head_dim != kHeadDim && ma_flash::applies(d, ptrs, n);
-}
-
 // lse: optional per-row softmax statistics (ma_attn_forward_lse), written by
 // the block-row, tiled and Longformer stream kernels; other kernels refuse
 // it.
@@ -2153,13 +2170,13 @@ int forward_launch(const ma_attn_desc* desc, const void* q, const void* k, const
   int rc;
   const bool want_rows = g_opt.force_rows;
   const bool want_band = g_opt.force_band;
-  const bool stream = !want_rows && !want_band && stream_applies(desc, q, k, v, o);
+  const bool flash = !want_rows && !want_band && flash_route(desc, qkvo, 4, false);
+  const bool stream = !flash && !want_rows && !want_band && stream_applies(desc, q, k, v, o);
   const bool block = !stream && !want_rows && block_applies(desc, q, k, v, o);
   if (lse && !block && !tiles_apply(desc, qkvo, 4) &&
       !(stream && desc->pattern == MA_ATTN_LONGFORMER && desc->num_global > 0))
     return fail("ma_attn_forward_lse: these kernels write no statistics (block-sparse, dense, Longformer "
                 "with 1 to 16 global tokens and index sets with a tile plan do, at head_dim 64)");
-  const bool flash = !want_rows && !want_band && flash_route(desc, qkvo, 4);
   if (flash) {
     rc = ma_flash::forward(desc, q, k, v, o, lse, st);
   } else if (stream) {
@@ -2302,8 +2319,8 @@ int ma_attn_backward(const ma_attn_desc* desc, const void* q, const void* k, con
     if (e != hipSuccess) return fail("ma_attn_backward: kernel launch failed: %s", hipGetErrorString(e));
     return 0;
   }
-  if (!g_opt.force_rows && flash_route(desc, ptrs, 7)) {
-    rc = ma_flash::backward(desc, ptrs, reinterpret_cast<float*>(stats), st);
+  if (!g_opt.force_rows && flash_route(desc, ptrs, 7, true)) {
+    rc = ma_flash::backward(desc, ptrs, reinterpret_cast<float*>(stats), nullptr, nullptr, st);
     if (rc) return rc;
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return fail("ma_attn_backward: kernel launch failed: %s", hipGetErrorString(e));
@@ -2388,10 +2405,12 @@ int ma_attn_backward_saved(const ma_attn_desc* desc, const void* q, const void* 
                : desc->dtype == MA_ATTN_F16
                    ? launch_tiles_bwd<HalfPath<_Float16>>(desc, ptrs, workspace, st, o, lse)
                    : launch_tiles_bwd<F32BwdPath>(desc, ptrs, workspace, st, o, lse))
-            : (desc->dtype == MA_ATTN_BF16 ? launch_backward_mfma<HalfPath<__bf16>>(desc, ptrs, sf, st, o, lse)
-               : desc->dtype == MA_ATTN_F16
-                   ? launch_backward_mfma<HalfPath<_Float16>>(desc, ptrs, sf, st, o, lse)
-                   : launch_backward_mfma<F32BwdPath>(desc, ptrs, sf, st, o, lse));
+      : flash_route(desc, ptrs, 8, true)
+          ? ma_flash::backward(desc, ptrs, sf, o, lse, st)
+          : (desc->dtype == MA_ATTN_BF16 ? launch_backward_mfma<HalfPath<__bf16>>(desc, ptrs, sf, st, o, lse)
+             : desc->dtype == MA_ATTN_F16
+                 ? launch_backward_mfma<HalfPath<_Float16>>(desc, ptrs, sf, st, o, lse)
+                 : launch_backward_mfma<F32BwdPath>(desc, ptrs, sf, st, o, lse));
   if (rc) return rc;
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return fail("ma_attn_backward_saved: kernel launch failed: %s", hipGetErrorString(e));

@@ -22,7 +22,11 @@ DTYPES = [torch.float32, torch.bfloat16, torch.float16]
 SHAPES = [
     (1, 8, 3, 3, 1), (63, 16, 63, 0, 1), (64, 128, 127, 0, 1), (65, 32, 32, 31, 1), (130, 40, 5, 70, 1),
     (257, 96, 100, 17, 2), (300, 120, 200, 0, 3), (191, 72, 0, 64, 1), (513, 24, 16, 15, 1),
-    (129, 128, None, 0, 1), (200, 80, None, 1, 1), (321, 32, None, 0, 1),
+    (129, 128, None, 0, 1), (200, 80, None, 1, 1), (321, 32, None, 0, 1), (450, 128, None, 0, 1),
+    # head_dim 64 (float32 on these kernels): windows past the stream kernels', causal rows in pairs of
+    # tiles (an odd tile count, a ragged last one), dense rows
+    (129, 64, 64, 64, 1), (700, 64, 100, 0, 2), (260, 64, 0, 127, 1), (64, 64, None, 0, 1), (65, 64, None, 0, 1),
+    (330, 64, None, 0, 1), (257, 64, None, 1, 1),
 ]
 
 
@@ -40,8 +44,11 @@ def _spec(oracle, shape, left, right, dil):
     return oracle.Spec(*shape, pattern="sliding", left=left, right=right, dilation=dil)
 
 
-@pytest.mark.parametrize("N,D,left,right,dil", SHAPES)
-@pytest.mark.parametrize("dtype", DTYPES)
+# head_dim 64 in 16 bits runs on other kernels
+CASES = [(*s, dt) for s in SHAPES for dt in DTYPES if s[1] != 64 or dt == torch.float32]
+
+
+@pytest.mark.parametrize("N,D,left,right,dil,dtype", CASES)
 def test_flash_against_oracle(ext, oracle, N, D, left, right, dil, dtype):
     shape = (2, N, 3, D)
     arrs = [*qkv(shape, 8000 + N + D), randn(shape, 8100 + N)]
@@ -58,6 +65,37 @@ def test_flash_against_oracle(ext, oracle, N, D, left, right, dil, dtype):
     assert (err <= (1e-5 if dtype == torch.float32 else 1e-4) + ulp * np.abs(ref)).all(), float(err.max())
     for name, a, b in zip("qkv", grads, oracle.backward(spec, *up)):
         check_grad("d" + name, a.float().cpu().numpy(), b, dtype == torch.float32)
+
+
+@pytest.mark.parametrize("N,H,causal", [(4200, 8, True), (9000, 16, True), (3000, 16, False)])
+def test_flash_dense_grids(ext, oracle, N, H, causal):
+    """float32 dense rows at head_dim 64 where the tiles pass one per CU (no
+    pairs, 8 waves) and four per CU (two query groups per wave): sampled rows
+    against the oracle."""
+    shape = (1, N, H, 64)
+    q, k, v = (torch.from_numpy(a).cuda() for a in qkv(shape, 8500 + N))
+    y = ext.dense_forward(q, k, v, causal).cpu().numpy()
+    up = [t.cpu().numpy()[:, :, [0, H - 1]] for t in (q, k, v)]
+    ref = oracle.forward(oracle.Spec(1, N, 2, 64, pattern="dense", causal=causal), *up)
+    assert float(np.abs(y[:, :, [0, H - 1]] - ref).max()) <= 1e-5
+
+
+@pytest.mark.parametrize("N,causal", [(300, True), (257, False), (65, True)])
+def test_flash_saved_statistics(ext, oracle, N, causal):
+    """float32 dense training pair at head_dim 64: the forward's statistics
+    against a float64 log-sum-exp, and the gradients from them."""
+    shape = (2, N, 3, 64)
+    arrs = [*qkv(shape, 8600 + N), randn(shape, 8610 + N)]
+    q, k, v, g = (torch.from_numpy(a).cuda() for a in arrs)
+    out, lse = ext.dense_forward(q, k, v, causal, return_lse=True)
+    s = torch.einsum("bihd,bjhd->bihj", q.double().cpu(), k.double().cpu()) / 8.0
+    if causal:
+        s = s.masked_fill(torch.arange(N)[None, :] > torch.arange(N)[:, None, None], float("-inf"))
+    ref = torch.logsumexp(s, -1) / np.log(2.0)
+    assert float((lse.double().cpu() - ref).abs().max()) <= 4e-6
+    got = ext.dense_backward(q, k, v, g, causal, out=out, lse=lse)
+    for name, a, b in zip("qkv", got, oracle.backward(oracle.Spec(*shape, pattern="dense", causal=causal), *arrs)):
+        check_grad("d" + name, a.cpu().numpy(), b, True)
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
