@@ -67,6 +67,45 @@ typedef struct ma_encoder_layer {
 int ma_encoder_layer_forward(const ma_encoder_layer* layer, const float* src, const float* attn,
                              float* out, void* stream);
 
+/*
+ * The whole forecasting model in one launch, eval mode: the reference's
+ * TransformerModel.forward (src/model.py:74-92).
+ *
+ *   x   = (src encoder_weight^T + encoder_bias) * sqrt(d_model) + pos[b]
+ *   x   = layer(x) for every layer (as ma_encoder_layer_forward without attn)
+ *   out = x[:, -1] decoder_weight^T + decoder_bias
+ *
+ * A workgroup keeps one sequence's activations in LDS from the input to the
+ * prediction.  Everything is float32; src is [batch, seq_len, input_dim], pos
+ * [batch, d_model] (the positional table's first `batch` rows, which the
+ * reference adds per batch entry), out [batch].  layers: HOST array of
+ * num_layers descriptors, each with this batch, seq_len and d_model.
+ * d_model in {16, 32, 64, 128}; 1 to MA_ENCODER_MAX_LAYERS layers; sequences up
+ * to ma_encoder_model_max_seq(d_model).  Pointers, return codes and asynchrony
+ * as ma_encoder_layer_forward (src, encoder_weight and decoder_bias need only
+ * 4-byte alignment); out must not overlap src.
+ */
+#define MA_ENCODER_MAX_LAYERS 8
+
+typedef struct ma_encoder_model {
+  int64_t batch;
+  int64_t seq_len;
+  int64_t input_dim;
+  int64_t d_model;
+  int64_t num_layers;
+  const ma_encoder_layer* layers;
+  const float* encoder_weight; /* [d_model, input_dim] */
+  const float* encoder_bias;   /* [d_model] */
+  const float* pos;            /* [batch, d_model] */
+  const float* decoder_weight; /* [1, d_model] */
+  const float* decoder_bias;   /* [1] */
+} ma_encoder_model;
+
+int ma_encoder_model_forward(const ma_encoder_model* model, const float* src, float* out, void* stream);
+
+/* The longest sequence ma_encoder_model_forward takes at d_model (0: none). */
+int64_t ma_encoder_model_max_seq(int64_t d_model);
+
 #ifdef __cplusplus
 }
 #endif

@@ -85,6 +85,27 @@ class EncoderLayer(ctypes.Structure):
     ]
 
 
+class EncoderModel(ctypes.Structure):
+    """Mirror of ``ma_encoder_model`` (include/ma_encoder.h)."""
+
+    _fields_ = [
+        ("batch", ctypes.c_int64),
+        ("seq_len", ctypes.c_int64),
+        ("input_dim", ctypes.c_int64),
+        ("d_model", ctypes.c_int64),
+        ("num_layers", ctypes.c_int64),
+        ("layers", ctypes.POINTER(EncoderLayer)),
+        ("encoder_weight", ctypes.c_void_p),
+        ("encoder_bias", ctypes.c_void_p),
+        ("pos", ctypes.c_void_p),
+        ("decoder_weight", ctypes.c_void_p),
+        ("decoder_bias", ctypes.c_void_p),
+    ]
+
+
+ENCODER_MAX_LAYERS = 8  # MA_ENCODER_MAX_LAYERS
+
+
 def _open():
     if not os.path.exists(LIB_PATH):
         raise ImportError(
@@ -136,6 +157,10 @@ def _open():
     lib.ma_attn_forward_noalloc.argtypes = [ctypes.POINTER(Desc)] + [ctypes.c_void_p] * 5
     lib.ma_encoder_layer_forward.restype = ctypes.c_int
     lib.ma_encoder_layer_forward.argtypes = [ctypes.POINTER(EncoderLayer)] + [ctypes.c_void_p] * 4
+    lib.ma_encoder_model_forward.restype = ctypes.c_int
+    lib.ma_encoder_model_forward.argtypes = [ctypes.POINTER(EncoderModel)] + [ctypes.c_void_p] * 3
+    lib.ma_encoder_model_max_seq.restype = ctypes.c_int64
+    lib.ma_encoder_model_max_seq.argtypes = [ctypes.c_int64]
     lib.ma_attn_tile_plan.restype = ctypes.c_int
     lib.ma_attn_tile_plan.argtypes = [ctypes.c_int64, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int64,
                                       ctypes.POINTER(TileHeader), ctypes.c_void_p, ctypes.c_size_t]
@@ -343,6 +368,12 @@ def encoder_layer_forward_raw(layer: EncoderLayer, src_ptr: int, attn_ptr: int, 
         raise RuntimeError(last_error())
 
 
+def encoder_model_forward_raw(model: EncoderModel, src_ptr: int, out_ptr: int, stream: int = 0) -> None:
+    """ma_encoder_model_forward.  Raises RuntimeError on rejection."""
+    if LIB.ma_encoder_model_forward(ctypes.byref(model), src_ptr, out_ptr, stream or None) != 0:
+        raise RuntimeError(last_error())
+
+
 def copy_probe_raw(desc: Desc, q_ptr: int, k_ptr: int, v_ptr: int, o_ptr: int, stream: int = 0,
                    events=None) -> None:
     """ma_attn_copy_probe(_timed): a forward kernel's traffic without its arithmetic
@@ -378,5 +409,6 @@ def default_scale(D: int) -> float:
 
 
 __all__ = ["LIB", "Desc", "make_desc", "forward_raw", "forward_noalloc_raw", "validate", "workspace_size",
-           "block_table", "row_keys", "pattern_csr", "copy_probe_raw", "backward_copy_probe_raw", "tile_plan", "tile_header_of", "TileHeader", "reload_options", "last_error", "EncoderLayer", "encoder_layer_forward_raw", "DTYPES", "default_scale",
+           "block_table", "row_keys", "pattern_csr", "copy_probe_raw", "backward_copy_probe_raw", "tile_plan", "tile_header_of", "TileHeader", "reload_options", "last_error", "EncoderLayer", "encoder_layer_forward_raw", "EncoderModel",
+           "encoder_model_forward_raw", "ENCODER_MAX_LAYERS", "DTYPES", "default_scale",
            "SLIDING", "DENSE", "BLOCK_SPARSE", "LONGFORMER", "INDEX_SET", "F32", "BF16", "F16"]

@@ -18,6 +18,10 @@ LayerNorm1, linear1, ReLU, linear2, residual and LayerNorm2 without
 intermediate tensors.  It applies to float32 device inputs when the layer is
 in eval mode (dropout the identity) and no gradient is being recorded; a call
 that records gradients, or a training-mode call, runs the operations above.
+A whole model of such layers, with sequences short enough for one workgroup's
+LDS, runs as one launch (ma_encoder_model_forward) from the input to the
+prediction; anything that would observe the modules in between (hooks,
+subclasses, tracing, autocast, tensor subclasses) keeps the layer calls.
 """
 from __future__ import annotations
 
@@ -141,6 +145,80 @@ class CustomTransformerEncoderLayer(nn.Module):
         return self.norm2(src + self.dropout2(ff))
 
 
+def _plain(module: nn.Module, cls) -> bool:
+    """Whether calling `module` runs cls.forward and nothing else."""
+    return (type(module) is cls and "forward" not in module.__dict__
+            and not (module._forward_hooks or module._forward_pre_hooks))
+
+
+def _linear_params(lin: nn.Linear):
+    return lin._parameters.get("weight"), lin._parameters.get("bias")
+
+
+def _model_launch(model: "TransformerModel", src: torch.Tensor):
+    """model(src) as one launch, or None when the call needs its modules:
+    gradients, training-mode dropout, other types, hooks, a width, depth or
+    length the kernel does not take."""
+    import torch.nn.modules.module as _m
+    if type(src) is not torch.Tensor or not src.is_cuda or src.dtype != torch.float32 or src.dim() != 3:
+        return None
+    if _m._global_forward_hooks or _m._global_forward_pre_hooks or torch.is_autocast_enabled("cuda") or \
+            torch.jit.is_tracing() or torch.compiler.is_compiling() or torch._C._len_torch_dispatch_stack() or \
+            torch._C._len_torch_function_stack() or torch._C._functorch.peek_interpreter_stack() is not None:
+        return None
+    mods = model._modules
+    enc, pos, dec, layers = mods["encoder"], mods["pos_encoder"], mods["decoder"], mods["encoder_layers"]
+    D = model.model_dim
+    B, S, I = src.shape
+    if D not in _FUSED_WIDTHS or B == 0 or S == 0 or not (_plain(enc, nn.Linear) and _plain(dec, nn.Linear)
+                                                         and _plain(pos, PositionalEncoding)):
+        return None
+    blocks = list(layers._modules.values())
+    grad = torch.is_grad_enabled()
+    params = [*_linear_params(enc), *_linear_params(dec)]
+    windows = []
+    for layer in blocks:
+        if not (_plain(layer, CustomTransformerEncoderLayer) and layer.fused):
+            return None
+        sub = layer._modules
+        attn = sub["self_attn"]
+        if not (type(attn) is SparseAttention and attn.use_ma_core):
+            return None
+        if layer.training and any(sub[n].p > 0 for n in ("dropout", "dropout1", "dropout2")):
+            return None
+        l1, l2, n1, n2 = sub["linear1"], sub["linear2"], sub["norm1"], sub["norm2"]
+        if (l1.in_features, l1.out_features) != (D, 4 * D) or n1.eps != n2.eps:
+            return None
+        for m in (n1, l1, l2, n2):
+            params += _linear_params(m)
+        windows.append((int(attn.window_size), float(n1.eps)))
+    pe = pos._buffers["pe"]
+    if pe.dtype != torch.float32 or pe.device != src.device or pe.shape[0] < B or not pe.is_contiguous() or \
+            pe.data_ptr() % 16:
+        return None
+    ptrs = []
+    for p in params:
+        if p is None or p.device != src.device or p.dtype != torch.float32 or not p.is_contiguous() or \
+                (grad and p.requires_grad):
+            return None
+        ptrs.append(p.data_ptr())
+    if (grad and src.requires_grad) or enc.in_features != I or any(p % 16 for p in ptrs[1:3] + ptrs[4:]):
+        return None
+    import ma_attn as _ma
+    if len(blocks) < 1 or len(blocks) > _ma.ENCODER_MAX_LAYERS or S > _ma.LIB.ma_encoder_model_max_seq(D):
+        return None
+    from sparse_attention_cuda import _on_device
+    descs = (_ma.EncoderLayer * len(blocks))()
+    for i, (w, eps) in enumerate(windows):
+        descs[i] = _ma.EncoderLayer(B, S, D, 4 * D, w, eps, 0, *ptrs[4 + 8 * i:12 + 8 * i])
+    M = _ma.EncoderModel(B, S, I, D, len(blocks), descs, ptrs[0], ptrs[1], pe.data_ptr(), ptrs[2], ptrs[3])
+    src = src.contiguous()
+    out = torch.empty((B, 1), dtype=torch.float32, device=src.device)
+    _on_device(src.get_device(),
+               lambda stream: _ma.encoder_model_forward_raw(M, src.data_ptr(), out.data_ptr(), stream))
+    return out
+
+
 class TransformerModel(nn.Module):
     """[batch, seq_len, input_dim] -> [batch, 1] (reference model.py:54-92).
 
@@ -151,6 +229,7 @@ class TransformerModel(nn.Module):
                  fallback_training=True, fused_layers=False):
         super().__init__()
         self.model_dim = model_dim
+        self.fused_layers = bool(fused_layers)
         self.encoder = nn.Linear(input_dim, model_dim)
         self.pos_encoder = PositionalEncoding(model_dim)
         self.encoder_layers = nn.ModuleList([
@@ -168,6 +247,10 @@ class TransformerModel(nn.Module):
         self.decoder.weight.data.uniform_(-r, r)
 
     def forward(self, src):
+        if self.__dict__.get("fused_layers"):  # absent from models pickled before it existed
+            out = _model_launch(self, src)
+            if out is not None:
+                return out
         x = self.pos_encoder(self.encoder(src) * math.sqrt(self.model_dim))
         for layer in self.encoder_layers:
             x = layer(x)

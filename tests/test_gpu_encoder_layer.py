@@ -197,3 +197,54 @@ def test_fused_model_other_width_runs_its_operations(model_mod):
         ext.forward = orig
     assert calls["n"] == 4  # two layers, each through the attention entry point, twice
     assert torch.equal(y_fused, y_plain)
+
+
+@pytest.mark.parametrize("d,layers", [(16, 1), (32, 6), (64, 4), (128, 3)])
+@pytest.mark.parametrize("B,S", [(1, 1), (64, 10), (3, 16), (5, 17), (2, 33), (7, 48), (257, 10), (1030, 7),
+                                 (600, 31), (5000, 1)])
+def test_model_launch_matches_layers(model_mod, d, layers, B, S):
+    """The whole model as one launch (sequences around the 16-token tiles, up
+    to the longest it takes) against the same model layer by layer, and its
+    float64 evaluation."""
+    torch.manual_seed(11 + d + S)
+    m = model_mod.TransformerModel(5, d, 2, layers, fused_layers=True).cuda().eval()
+    src = torch.randn(B, S, 5, device="cuda")
+    with torch.no_grad():
+        one = model_mod._model_launch(m, src)
+        assert one is not None and torch.equal(one, m(src))
+        x = m.pos_encoder(m.encoder(src) * d ** 0.5)
+        y = x.double().cpu()
+        for layer in m.encoder_layers:
+            x = layer(x)
+            y = _ref64(layer, y, 3)
+        by_layer = m.decoder(x[:, -1, :])
+        ref = y[:, -1] @ m.decoder.weight.double().cpu().T + m.decoder.bias.double().cpu()
+    assert (one - by_layer).abs().max().item() <= TOL
+    assert (one.double().cpu() - ref).abs().max().item() <= TOL
+
+
+def test_model_launch_leaves_observed_modules_alone(model_mod):
+    """Hooks, gradients, autocast, training-mode dropout, other types and long
+    sequences keep the layer-by-layer forward."""
+    m = model_mod.TransformerModel(5, 64, 2, 2, fused_layers=True).cuda().eval()
+    src = torch.randn(2, 10, 5, device="cuda")
+    take = model_mod._model_launch
+    with torch.no_grad():
+        assert take(m, src) is not None
+        seen = []
+        handle = m.encoder_layers[0].register_forward_hook(lambda *a: seen.append(1))
+        y = m(src)
+        assert seen == [1]
+        handle.remove()
+        assert (m(src) - y).abs().max().item() <= TOL
+        assert take(m, src.double()) is None and take(m, src.cpu()) is None
+        assert take(m, torch.randn(1, 65, 5, device="cuda")) is None
+        with torch.autocast("cuda"):
+            assert take(m, src) is None
+        m.encoder_layers[1].norm1.eps = 1e-3
+        assert take(m, src) is None
+        m.encoder_layers[1].norm1.eps = 1e-5
+        m.train()
+        assert take(m, src) is None
+        m.eval()
+    assert take(m, src) is None  # parameters record gradients
