@@ -68,7 +68,9 @@ int run_fwd(const ma_attn_desc* d, FlArgs a, hipStream_t st) {
 // buffers at head_dim 32 and 128 (causal 128-key window, bf16, head_dim 128,
 // 8 heads, 32768 rows: 83 us against 87-104; two-sided 64-key window, head_dim
 // 32, 4 x 8 heads, 8191 rows: f16 26 us against 28-31, f32 43 us against
-// 43-70).  float32 above head_dim 64 takes 32-key blocks (three planes of 64
+// 43-70).  16-bit windows of at most 128 keys at head_dim 32 take 128-key
+// blocks: a 64-query tile of a 64-key window is then one block (22 us against
+// 24 on the f16 window above).  float32 above head_dim 64 takes 32-key blocks (three planes of 64
 // rows would leave one workgroup per CU, or spill).
 // Causal rows, the longest and the shortest tile of a stream in one workgroup.
 template <typename T, int ND, int NW, int KB>
@@ -91,7 +93,9 @@ int run_pair(const ma_attn_desc* d, FlArgs a, hipStream_t st) {
 // buffers at head_dim 32 and 128 (causal 128-key window, bf16, head_dim 128,
 // 8 heads, 32768 rows: 83 us against 87-104; two-sided 64-key window, head_dim
 // 32, 4 x 8 heads, 8191 rows: f16 26 us against 28-31, f32 43 us against
-// 43-70).  float32 above head_dim 64 takes 32-key blocks (three planes of 64
+// 43-70).  16-bit windows of at most 128 keys at head_dim 32 take 128-key
+// blocks: a 64-query tile of a 64-key window is then one block (22 us against
+// 24 on the f16 window above).  float32 above head_dim 64 takes 32-key blocks (three planes of 64
 // rows would leave one workgroup per CU, or spill).
 //
 // Causal rows whose 128-row tiles are at most one per CU run in pairs, longest
@@ -117,6 +121,8 @@ int fwd_nd(const ma_attn_desc* d, const FlArgs& a, hipStream_t st) {
     if (b.left >= b.nr && tiles128 >= 1024) return run_fwd<T, ND, 2, 8, KB, false, 2>(d, a, st);
     if (tiles128 >= 256) return run_fwd<T, ND, 1, 8, KB, false, 2>(d, a, st);
   }
+  if constexpr (!f32 && ND == 1)
+    if (b.left + b.right < 128) return run_fwd<T, ND, 1, 4, 128, false, 3>(d, a, st);
   return run_fwd<T, ND, 1, 4, KB, false, f32 ? 2 : 3>(d, a, st);
 }
 
