@@ -19,7 +19,7 @@ int forward(const ma_attn_desc* d, const void* q, const void* k, const void* v, 
 
 // Launches the backward (ptrs: q, k, v, dout, dq, dk, dv); stats: 2 floats per
 // row of workspace.  fo, lse: the forward's O and statistics
-// (ma_attn_backward_saved; float32 at head_dim 64), or null.  Non-zero on
+// (ma_attn_backward_saved; head_dim 64), or null.  Non-zero on
 // failure.
 int backward(const ma_attn_desc* d, const void* const* ptrs, float* stats, const void* fo, const float* lse,
              hipStream_t st);

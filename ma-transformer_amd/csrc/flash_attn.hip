@@ -136,15 +136,15 @@ int fwd_t(const ma_attn_desc* d, const FlArgs& a, hipStream_t st) {
   }
 }
 
-template <typename T, int ND, int NQ, int NWQ, int NWK, int KB, int OCC, bool SAVED>
+template <typename T, int ND, int NQ, int NK, int NWQ, int NWK, int KB, int NPB, int OCC, bool SAVED, bool FAST, bool PAIR>
 int run_bwd(const ma_attn_desc* d, FlArgs a, hipStream_t st) {
   Band b;
   band_of(d, &b);
-  constexpr int QT = 16 * NQ * NWQ, KT = 16 * NWK;
+  constexpr int QT = 16 * NQ * NWQ, KT = 16 * NK * NWK;
   constexpr size_t shm_q = 2 * FlStage<T, ND, KB, NWQ>::kMat;
   constexpr size_t shm_k = 2 * FlStage<T, ND, KB, NWK>::kMat + 2 * KB * sizeof(float);
-  auto kq = &flash_dq_kernel<T, ND, NQ, NWQ, KB, OCC, SAVED>;
-  auto kk = &flash_dkv_kernel<T, ND, NWK, KB, OCC>;
+  auto kq = &flash_dq_kernel<T, ND, NQ, NWQ, KB, NPB, OCC, SAVED, FAST, PAIR>;
+  auto kk = &flash_dkv_kernel<T, ND, NK, NWK, KB, NPB, OCC, FAST, PAIR>;
   if (ma_host::reserve_lds(reinterpret_cast<const void*>(kq), shm_q, st) ||
       ma_host::reserve_lds(reinterpret_cast<const void*>(kk), shm_k, st))
     return 1;
@@ -160,12 +160,46 @@ int run_bwd(const ma_attn_desc* d, FlArgs a, hipStream_t st) {
 // 4 waves and 64-row blocks (float32 above head_dim 64: 32-row): measured best
 // of 4 or 8 waves and 32- or 64-row blocks (causal 128-key window, bf16,
 // head_dim 128, 2 x 8 heads, 4096 rows: 74 us against 79-88).
+//
+// Causal rows in pairs of tiles, as in the forward: float32 above head_dim 32 on
+// at most one 128-row tile per CU (8 heads of 4096 rows: head_dim 64 628 -> 561
+// us, 128 1183 -> 981; 16-bit and narrow heads were 2-10 % slower), and 16-bit
+// from saved statistics on half to one tile per CU (4096 rows: 138 -> 128 us).
+//
+// 16-bit at head_dim 64 from saved statistics (dense; P and dS rounded to 16
+// bits, as in bwd_q_kernel / bwd_kv_kernel): blocks inside the band as
+// straight-line code; with 256-row tiles enough for every CU (twice, for causal
+// rows, whose tiles are uneven) two row groups per wave, so that each LDS read
+// feeds two MFMAs.  8 heads, bwd_q + bwd_kv -> here: causal 2048 rows 77 -> 68 us,
+// 8192 rows 339 -> 322, 16384 rows 1180 -> 975; all pairs, 8192 rows 623 -> 472.
 template <typename T, int ND>
 int bwd_nd(const ma_attn_desc* d, const FlArgs& a, hipStream_t st) {
-  constexpr int KB = sizeof(T) == 4 && ND > 2 ? 32 : 64;
-  if constexpr (sizeof(T) == 4 && ND == 2)  // saved statistics: head_dim 64
-    if (a.fo) return run_bwd<T, ND, 1, 4, 4, KB, 2, true>(d, a, st);
-  return run_bwd<T, ND, 1, 4, 4, KB, 2, false>(d, a, st);
+  constexpr bool f32 = sizeof(T) == 4;
+  constexpr int KB = f32 && ND > 2 ? 32 : 64;
+  constexpr int NP = FlElt<T>::NPB;
+  Band b;
+  band_of(d, &b);
+  const int64_t streams = d->batch * d->num_heads * b.dil;
+  const int64_t tiles128 = streams * ((b.nr + 127) / 128), tiles256 = streams * ((b.nr + 255) / 256);
+  FlArgs pair = a;
+  pair.desc = 0;
+  if constexpr (f32 && ND == 2) {  // saved statistics: head_dim 64
+    if (a.fo) {
+      if (a.desc && tiles128 <= 256) return run_bwd<T, ND, 1, 1, 8, 8, KB, NP, 2, true, false, true>(d, pair, st);
+      return run_bwd<T, ND, 1, 1, 4, 4, KB, NP, 2, true, false, false>(d, a, st);
+    }
+  }
+  if constexpr (!f32 && ND == 2) {
+    if (a.fo) {
+      if (a.desc && tiles128 > 128 && tiles128 <= 256)
+        return run_bwd<T, ND, 1, 1, 8, 8, KB, 1, 2, true, true, true>(d, pair, st);
+      if (tiles256 >= (a.desc ? 512 : 256)) return run_bwd<T, ND, 2, 2, 8, 8, KB, 1, 2, true, true, false>(d, a, st);
+      return run_bwd<T, ND, 1, 1, 4, 4, KB, 1, 3, true, true, false>(d, a, st);
+    }
+  }
+  if constexpr (f32 && ND >= 2)
+    if (a.desc && tiles128 <= 256) return run_bwd<T, ND, 1, 1, 8, 8, KB, NP, 2, false, false, true>(d, pair, st);
+  return run_bwd<T, ND, 1, 1, 4, 4, KB, NP, 2, false, false, false>(d, a, st);
 }
 
 template <typename T>

@@ -336,6 +336,32 @@ __device__ __forceinline__ FlPos fl_pos(const FlArgs& a, int elt) {
   return p;
 }
 
+// Rows of a workgroup of NW waves with W rows each: wave w has first .. first +
+// W - 1 (first = Nr: none), the workgroup lo .. hi.  PAIR: the first half of
+// the waves on tile p, the second half on tile T - 1 - p.
+struct FlRows {
+  int first, lo, hi;
+};
+template <int W, int NW, bool PAIR>
+__device__ __forceinline__ bool fl_rows(const FlPos& ps, int wv, FlRows& r) {
+  if constexpr (PAIR) {
+    constexpr int HT = W * NW / 2;
+    const int last = (ps.Nr + HT - 1) / HT - 1 - ps.tile;
+    if (ps.tile > last) return false;
+    const bool second = wv >= NW / 2;
+    r.first = (second ? last : ps.tile) * HT + W * (wv % (NW / 2));
+    if (second && last == ps.tile) r.first = ps.Nr;  // the middle tile of an odd count: one half is enough
+    r.lo = ps.tile * HT;
+    r.hi = last * HT + HT - 1;
+    return true;
+  } else {
+    r.lo = ps.tile * (W * NW);
+    r.hi = r.lo + W * NW - 1;
+    r.first = r.lo + W * wv;
+    return r.lo < ps.Nr;
+  }
+}
+
 __device__ __forceinline__ float fl_wave_sum(float x) {
 #pragma unroll
   for (int m = 32; m >= 1; m >>= 1) x += __shfl_xor(x, m, 64);
@@ -579,20 +605,15 @@ __global__ __launch_bounds__(64 * NW, 2) void flash_pair_fwd_kernel(FlArgs a) {
   using St = FlStage<T, ND, KB, NW>;
   constexpr int RS = St::RS, PL = St::kPlane, MAT = St::kMat;
   constexpr int NU = KB / 16;
-  constexpr int QT = 16 * NQ * NW;
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int c = lane & 15, g = lane >> 4;
   const FlPos ps = fl_pos(a, sizeof(T));
   const int Nr = ps.Nr, L = a.left, R = a.right, D = a.D;
-  constexpr int HT = QT / 2;
-  const int T2 = (Nr + HT - 1) / HT, lo = ps.tile, hi = T2 - 1 - ps.tile;
-  if (lo > hi) return;  // uniform per workgroup, before any barrier
-  const bool second = wv >= NW / 2;
-  int qa = (second ? hi : lo) * HT + 16 * NQ * (wv % (NW / 2));  // the wave's first query
-  if (second && lo == hi) qa = Nr;  // the middle tile of an odd count: one half is enough
-  const int qmin = lo * HT, qmax = hi * HT + HT - 1;
+  FlRows rows;
+  if (!fl_rows<16 * NQ, NW, true>(ps, wv, rows)) return;  // uniform per workgroup, before any barrier
+  const int qa = rows.first, qmin = rows.lo, qmax = rows.hi;
   const uint32_t tb = a.tok_bytes;
   const __amdgpu_buffer_rsrc_t Qr = make_rsrc(static_cast<const T*>(a.q) + ps.base, ps.nrec);
   const __amdgpu_buffer_rsrc_t Kr = make_rsrc(static_cast<const T*>(a.k) + ps.base, ps.nrec);
@@ -857,11 +878,17 @@ __device__ __forceinline__ void fl_dkv_row(const FlArgs& a, const FlPos& ps, int
     }
 }
 
+template <bool B>
+struct FlBool {
+  static constexpr bool value = B;
+};
+
 // dQ of 16 NQ NW queries.  Pass 1 over the key blocks: the online softmax's
 // maximum, sum and sum of e dp.  Pass 2, backwards over the same blocks (the
 // last one is still in LDS): p, ds, dQ^T += K^T ds^T.  SAVED: the forward's
-// statistics are read and delta = dO . O, so only the second pass runs.
-template <typename T, int ND, int NQ, int NW, int KB, int OCC, bool SAVED>
+// statistics are read and delta = dO . O, so only the second pass runs.  PAIR:
+// fl_rows; NPB: planes of a dS (and probability) operand.
+template <typename T, int ND, int NQ, int NW, int KB, int NPB, int OCC, bool SAVED, bool FAST, bool PAIR>
 __global__ __launch_bounds__(64 * NW, OCC) void flash_dq_kernel(FlArgs a) {
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
   using St = FlStage<T, ND, KB, NW>;
@@ -873,8 +900,8 @@ __global__ __launch_bounds__(64 * NW, OCC) void flash_dq_kernel(FlArgs a) {
   const int c = lane & 15, g = lane >> 4;
   const FlPos ps = fl_pos(a, sizeof(T));
   const int Nr = ps.Nr, L = a.left, R = a.right, D = a.D;
-  const int q0 = ps.tile * (16 * NQ * NW);
-  if (q0 >= Nr) return;  // uniform per workgroup, before any barrier
+  FlRows rows;
+  if (!fl_rows<16 * NQ, NW, PAIR>(ps, wv, rows)) return;  // uniform per workgroup, before any barrier
   const uint32_t tb = a.tok_bytes;
   const __amdgpu_buffer_rsrc_t Qr = make_rsrc(static_cast<const T*>(a.q) + ps.base, ps.nrec);
   const __amdgpu_buffer_rsrc_t Gr = make_rsrc(static_cast<const T*>(a.dout) + ps.base, ps.nrec);
@@ -882,9 +909,9 @@ __global__ __launch_bounds__(64 * NW, OCC) void flash_dq_kernel(FlArgs a) {
   const __amdgpu_buffer_rsrc_t Vr = make_rsrc(static_cast<const T*>(a.v) + ps.base, ps.nrec);
   const __amdgpu_buffer_rsrc_t Or = make_rsrc(static_cast<T*>(a.o) + ps.base, ps.nrec);
 
-  const int qa = q0 + 16 * NQ * wv;
-  const int k0 = max(0, q0 - L) & ~15;
-  const int kend = min(Nr, q0 + 16 * NQ * NW + R);
+  const int qa = rows.first;
+  const int k0 = max(0, rows.lo - L) & ~15;
+  const int kend = min(Nr, rows.hi + 1 + R);
   const int nb = (kend - k0 + KB - 1) / KB;
   const int steps = SAVED ? nb : 2 * nb;
   auto block_at = [&](int e) { return !SAVED && e < nb ? e : steps - 1 - e; };
@@ -943,9 +970,10 @@ __global__ __launch_bounds__(64 * NW, OCC) void flash_dq_kernel(FlArgs a) {
 
   // S and dP of sub-tile u of the block at key0, pairs outside the band
   // masked (their V row may hold anything: dP 0)
-  auto scores = [&](int u, int key0, f32x4 (&sc)[NQ], f32x4 (&dp)[NQ]) {
+  auto scores = [&](auto full, int u, int key0, f32x4 (&sc)[NQ], f32x4 (&dp)[NQ]) __attribute__((always_inline)) {
     fl_rowdot<T, ND, PL, NQ>(lds + u * 16 * RS + rl, qf, sc);
     fl_rowdot<T, ND, PL, NQ>(lds + MAT + u * 16 * RS + rl, gf, dp);
+    if constexpr (decltype(full)::value) return;
     const int key = key0 + 16 * u;
 #pragma unroll
     for (int n = 0; n < NQ; ++n) {
@@ -978,7 +1006,7 @@ __global__ __launch_bounds__(64 * NW, OCC) void flash_dq_kernel(FlArgs a) {
       for (int u = 0; u < NU; ++u) {
         if (u < u0 || u > u1) continue;  // wave-uniform
         f32x4 sc[NQ], dp[NQ];
-        scores(u, key0, sc, dp);
+        scores(FlBool<false>{}, u, key0, sc, dp);
 #pragma unroll
         for (int n = 0; n < NQ; ++n) {
           const float mn =
@@ -1012,34 +1040,45 @@ __global__ __launch_bounds__(64 * NW, OCC) void flash_dq_kernel(FlArgs a) {
         }
       }
     } else {
+      auto pass2 = [&](auto full) __attribute__((always_inline)) {
+        constexpr bool FULL = decltype(full)::value;
 #pragma unroll
-      for (int u = 0; u < NU; u += 2) {
-        if (u + 1 < u0 || u > u1) continue;  // wave-uniform
-        f32x4 sc[2][NQ], dp[2][NQ];
+        for (int u = 0; u < NU; u += 2) {
+          if (!FULL && (u + 1 < u0 || u > u1)) continue;  // wave-uniform
+          f32x4 sc[2][NQ], dp[2][NQ];
 #pragma unroll
-        for (int w = 0; w < 2; ++w) {
-          if (u + w >= u0 && u + w <= u1)
-            scores(u + w, key0, sc[w], dp[w]);
-          else
+          for (int w = 0; w < 2; ++w) {
+            if (FULL || (u + w >= u0 && u + w <= u1)) {
+              scores(full, u + w, key0, sc[w], dp[w]);
+            } else {
 #pragma unroll
-            for (int n = 0; n < NQ; ++n) {
-              sc[w][n] = f32x4{-INFINITY, -INFINITY, -INFINITY, -INFINITY};
-              dp[w][n] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+              for (int n = 0; n < NQ; ++n) {
+                sc[w][n] = f32x4{-INFINITY, -INFINITY, -INFINITY, -INFINITY};
+                dp[w][n] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+              }
             }
+          }
+          FlB<T, NPB> db[NQ];
+#pragma unroll
+          for (int n = 0; n < NQ; ++n) {
+            float ds[2][4];
+#pragma unroll
+            for (int w = 0; w < 2; ++w)
+#pragma unroll
+              for (int r = 0; r < 4; ++r) {
+                const float p = __builtin_amdgcn_exp2f(fmaf(sc[w][n][r], sl2, -m[n]));
+                ds[w][r] = (SAVED ? p : p * l[n]) * (dp[w][n][r] - dl[n]);
+              }
+            db[n].set(ds[0], ds[1]);
+          }
+          fl_trmul<T, ND, PL, NQ, NPB>(lds + u * 16 * RS + tl, lds + (u + 1) * 16 * RS + tl, db, acc);
         }
-        FlB<T> db[NQ];
-#pragma unroll
-        for (int n = 0; n < NQ; ++n) {
-          float ds[2][4];
-#pragma unroll
-          for (int w = 0; w < 2; ++w)
-#pragma unroll
-            for (int r = 0; r < 4; ++r)
-              ds[w][r] = __builtin_amdgcn_exp2f(fmaf(sc[w][n][r], sl2, -m[n])) * l[n] * (dp[w][n][r] - dl[n]);
-          db[n].set(ds[0], ds[1]);
-        }
-        fl_trmul<T, ND, PL, NQ>(lds + u * 16 * RS + tl, lds + (u + 1) * 16 * RS + tl, db, acc);
-      }
+      };
+      // FAST: blocks wholly inside the band as straight-line code
+      if (FAST && key0 >= qa + 16 * NQ - 1 - L && key0 + KB - 1 <= min(qa + R, Nr - 1) && qa < Nr)
+        pass2(FlBool<true>{});
+      else
+        pass2(FlBool<false>{});
     }
     if (more) {
       __syncthreads();
@@ -1072,10 +1111,11 @@ __global__ __launch_bounds__(64 * NW, OCC) void flash_dq_kernel(FlArgs a) {
   }
 }
 
-// dK, dV of 16 NW keys: a wave holds 16 keys' K and V rows as register
-// operands; blocks of QB query rows (Q, dO and their statistics) go through
-// LDS.  S and dP land with lane (c, g) holding queries 4 g .. 4 g + 3 of key c.
-template <typename T, int ND, int NW, int QB, int OCC>
+// dK, dV of 16 NK NW keys: a wave holds NK groups of 16 keys' K and V rows as
+// register operands; blocks of QB query rows (Q, dO and their statistics) go
+// through LDS, and every operand read from them feeds NK MFMAs.  S and dP land
+// with lane (c, g) holding queries 4 g .. 4 g + 3 of key c.
+template <typename T, int ND, int NK, int NW, int QB, int NPB, int OCC, bool FAST, bool PAIR>
 __global__ __launch_bounds__(64 * NW, OCC) void flash_dkv_kernel(FlArgs a) {
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
   using St = FlStage<T, ND, QB, NW>;
@@ -1088,8 +1128,8 @@ __global__ __launch_bounds__(64 * NW, OCC) void flash_dkv_kernel(FlArgs a) {
   const int c = lane & 15, g = lane >> 4;
   const FlPos ps = fl_pos(a, sizeof(T));
   const int Nr = ps.Nr, L = a.left, R = a.right, D = a.D;
-  const int j0 = ps.tile * (16 * NW);
-  if (j0 >= Nr) return;  // uniform per workgroup, before any barrier
+  FlRows rows;
+  if (!fl_rows<16 * NK, NW, PAIR>(ps, wv, rows)) return;  // uniform per workgroup, before any barrier
   const uint32_t tb = a.tok_bytes;
   const __amdgpu_buffer_rsrc_t Qr = make_rsrc(static_cast<const T*>(a.q) + ps.base, ps.nrec);
   const __amdgpu_buffer_rsrc_t Gr = make_rsrc(static_cast<const T*>(a.dout) + ps.base, ps.nrec);
@@ -1098,9 +1138,9 @@ __global__ __launch_bounds__(64 * NW, OCC) void flash_dkv_kernel(FlArgs a) {
   const __amdgpu_buffer_rsrc_t dKr = make_rsrc(static_cast<T*>(a.dk) + ps.base, ps.nrec);
   const __amdgpu_buffer_rsrc_t dVr = make_rsrc(static_cast<T*>(a.dv) + ps.base, ps.nrec);
 
-  const int ja = j0 + 16 * wv;  // the wave's first key
-  const int i0 = max(0, j0 - R) & ~15;
-  const int iend = min(Nr, j0 + 16 * NW + L);
+  const int ja = rows.first;  // the wave's first key
+  const int i0 = max(0, rows.lo - R) & ~15;
+  const int iend = min(Nr, rows.hi + 1 + L);
   const int nb = (iend - i0 + QB - 1) / QB;
 
   St qs, gs;
@@ -1121,14 +1161,19 @@ __global__ __launch_bounds__(64 * NW, OCC) void flash_dkv_kernel(FlArgs a) {
   qs.load(Qr, i0, tid, tb, D);
   gs.load(Gr, i0, tid, tb, D);
   load_stats(i0);
-  FlFrag<T, ND> kf[1], vf[1];
-  kf[0].load(Kr, (uint32_t)(ja + c) * tb, D, g);
-  vf[0].load(Vr, (uint32_t)(ja + c) * tb, D, g);
+  FlFrag<T, ND> kf[NK], vf[NK];
+#pragma unroll
+  for (int n = 0; n < NK; ++n) {
+    kf[n].load(Kr, (uint32_t)(ja + 16 * n + c) * tb, D, g);
+    vf[n].load(Vr, (uint32_t)(ja + 16 * n + c) * tb, D, g);
+  }
   const uint32_t rl = (uint32_t)(c * RS + 16 * g), tl = fl_tr_lane<ND>(c, g);
   const float sl2 = a.scale_log2;
-  f32x4 ak[1][2 * ND], av[1][2 * ND];
+  f32x4 ak[NK][2 * ND], av[NK][2 * ND];
 #pragma unroll
-  for (int d = 0; d < 2 * ND; ++d) ak[0][d] = av[0][d] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  for (int n = 0; n < NK; ++n)
+#pragma unroll
+    for (int d = 0; d < 2 * ND; ++d) ak[n][d] = av[n][d] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
   qs.store(lds, tid);
   gs.store(lds + MAT, tid);
   store_stats();
@@ -1143,48 +1188,66 @@ __global__ __launch_bounds__(64 * NW, OCC) void flash_dkv_kernel(FlArgs a) {
     }
     __builtin_amdgcn_sched_barrier(0);
     const int r0 = i0 + e * QB;
-    // query sub-tiles [u0, u1] see some key of the wave: i in [ja - R, ja + 15 + L]
+    // query sub-tiles [u0, u1] see some key of the wave: i in [ja - R, ja + 16 NK - 1 + L]
     const int u0 = max(0, (ja - R - r0) >> 4);
-    const int u1 = ja < Nr ? min(NU - 1, (min(ja + 15 + L, Nr - 1) - r0) >> 4) : -1;
+    const int u1 = ja < Nr ? min(NU - 1, (min(ja + 16 * NK - 1 + L, Nr - 1) - r0) >> 4) : -1;
+    auto block = [&](auto full) __attribute__((always_inline)) {
+      constexpr bool FULL = decltype(full)::value;
 #pragma unroll
-    for (int u = 0; u < NU; u += 2) {
-      if (u + 1 < u0 || u > u1) continue;  // wave-uniform
-      float p[2][4], ds[2][4];
+      for (int u = 0; u < NU; u += 2) {
+        if (!FULL && (u + 1 < u0 || u > u1)) continue;  // wave-uniform
+        float p[NK][2][4], ds[NK][2][4];
 #pragma unroll
-      for (int w = 0; w < 2; ++w) {
-        if (u + w >= u0 && u + w <= u1) {
-          f32x4 sc[1], dp[1];
-          fl_rowdot<T, ND, PL, 1>(lds + (u + w) * 16 * RS + rl, kf, sc);
-          fl_rowdot<T, ND, PL, 1>(lds + MAT + (u + w) * 16 * RS + rl, vf, dp);
-          const int qb = r0 + 16 * (u + w);
-          const int rel = ja - qb;  // key - query offsets span rel -+ 15
-          const f32x4 ls = *reinterpret_cast<const f32x4*>(lst + 16 * (u + w) + 4 * g);
-          const f32x4 dt = *reinterpret_cast<const f32x4*>(lst + QB + 16 * (u + w) + 4 * g);
-          if (rel - 15 < -L || rel + 15 > R) {
-            const int x = rel + c - 4 * g;  // key - query of element 0
+        for (int w = 0; w < 2; ++w) {
+          if (FULL || (u + w >= u0 && u + w <= u1)) {
+            f32x4 sc[NK], dp[NK];
+            fl_rowdot<T, ND, PL, NK>(lds + (u + w) * 16 * RS + rl, kf, sc);
+            fl_rowdot<T, ND, PL, NK>(lds + MAT + (u + w) * 16 * RS + rl, vf, dp);
+            const int qb = r0 + 16 * (u + w);
+            const f32x4 ls = *reinterpret_cast<const f32x4*>(lst + 16 * (u + w) + 4 * g);
+            const f32x4 dt = *reinterpret_cast<const f32x4*>(lst + QB + 16 * (u + w) + 4 * g);
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-              const bool in = x - r >= -L && x - r <= R;
-              sc[0][r] = in ? sc[0][r] : -INFINITY;
-              dp[0][r] = in ? dp[0][r] : dt[r];
+            for (int n = 0; n < NK; ++n) {
+              if constexpr (!FULL) {
+                const int rel = ja + 16 * n - qb;  // key - query offsets span rel -+ 15
+                if (rel - 15 < -L || rel + 15 > R) {
+                  const int x = rel + c - 4 * g;  // key - query of element 0
+#pragma unroll
+                  for (int r = 0; r < 4; ++r) {
+                    const bool in = x - r >= -L && x - r <= R;
+                    sc[n][r] = in ? sc[n][r] : -INFINITY;
+                    dp[n][r] = in ? dp[n][r] : dt[r];
+                  }
+                }
+              }
+#pragma unroll
+              for (int r = 0; r < 4; ++r) {
+                p[n][w][r] = __builtin_amdgcn_exp2f(fmaf(sc[n][r], sl2, -ls[r]));
+                ds[n][w][r] = p[n][w][r] * (dp[n][r] - dt[r]);
+              }
             }
-          }
+          } else {
 #pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            p[w][r] = __builtin_amdgcn_exp2f(fmaf(sc[0][r], sl2, -ls[r]));
-            ds[w][r] = p[w][r] * (dp[0][r] - dt[r]);
-          }
-        } else {
+            for (int n = 0; n < NK; ++n)
 #pragma unroll
-          for (int r = 0; r < 4; ++r) p[w][r] = ds[w][r] = 0.0f;
+              for (int r = 0; r < 4; ++r) p[n][w][r] = ds[n][w][r] = 0.0f;
+          }
         }
+        FlB<T, NPB> b[NK];
+#pragma unroll
+        for (int n = 0; n < NK; ++n) b[n].set(p[n][0], p[n][1]);
+        fl_trmul<T, ND, PL, NK, NPB>(lds + MAT + u * 16 * RS + tl, lds + MAT + (u + 1) * 16 * RS + tl, b, av);
+#pragma unroll
+        for (int n = 0; n < NK; ++n) b[n].set(ds[n][0], ds[n][1]);
+        fl_trmul<T, ND, PL, NK, NPB>(lds + u * 16 * RS + tl, lds + (u + 1) * 16 * RS + tl, b, ak);
       }
-      FlB<T> b[1];
-      b[0].set(p[0], p[1]);
-      fl_trmul<T, ND, PL, 1>(lds + MAT + u * 16 * RS + tl, lds + MAT + (u + 1) * 16 * RS + tl, b, av);
-      b[0].set(ds[0], ds[1]);
-      fl_trmul<T, ND, PL, 1>(lds + u * 16 * RS + tl, lds + (u + 1) * 16 * RS + tl, b, ak);
-    }
+    };
+    // FAST: blocks whose every pair is in the band as straight-line code (rows
+    // past the end have lse2 = infinity)
+    if (FAST && ja < Nr && r0 >= ja + 16 * NK - 1 - R && r0 + QB - 1 <= ja + L)
+      block(FlBool<true>{});
+    else
+      block(FlBool<false>{});
     if (more) {
       __syncthreads();
       qs.store(lds, tid);
@@ -1195,15 +1258,18 @@ __global__ __launch_bounds__(64 * NW, OCC) void flash_dkv_kernel(FlArgs a) {
   }
 
   if (ja >= Nr) return;  // no barrier below
-  const int j = ja + c;
-  const uint64_t bad = __builtin_amdgcn_ballot_w64(j < Nr && (fl_bad<ND>(ak[0]) || fl_bad<ND>(av[0])));
-  const bool own_bad = (bad >> c & 0x0001000100010001ull) != 0;
-  const uint32_t row = own_bad ? kOob : (uint32_t)j * tb;
-  fl_store<T, ND>(ak[0], a.scale, dKr, row, D, g);
-  fl_store<T, ND>(av[0], 1.0f, dVr, row, D, g);
-  if (__builtin_expect(bad != 0, 0)) {
-    for (int r = 0; r < 16; ++r)
-      if (bad >> r & 0x0001000100010001ull) fl_dkv_row<T, (ND + 1) / 2>(a, ps, ja + r, lane);
+#pragma unroll
+  for (int n = 0; n < NK; ++n) {
+    const int j = ja + 16 * n + c;
+    const uint64_t bad = __builtin_amdgcn_ballot_w64(j < Nr && (fl_bad<ND>(ak[n]) || fl_bad<ND>(av[n])));
+    const bool own_bad = (bad >> c & 0x0001000100010001ull) != 0;
+    const uint32_t row = own_bad ? kOob : (uint32_t)j * tb;
+    fl_store<T, ND>(ak[n], a.scale, dKr, row, D, g);
+    fl_store<T, ND>(av[n], 1.0f, dVr, row, D, g);
+    if (__builtin_expect(bad != 0, 0)) {
+      for (int r = 0; r < 16; ++r)
+        if (bad >> r & 0x0001000100010001ull) fl_dkv_row<T, (ND + 1) / 2>(a, ps, ja + 16 * n + r, lane);
+    }
   }
 }
 

@@ -2405,7 +2405,7 @@ int ma_attn_backward_saved(const ma_attn_desc* desc, const void* q, const void* 
                : desc->dtype == MA_ATTN_F16
                    ? launch_tiles_bwd<HalfPath<_Float16>>(desc, ptrs, workspace, st, o, lse)
                    : launch_tiles_bwd<F32BwdPath>(desc, ptrs, workspace, st, o, lse))
-      : flash_route(desc, ptrs, 8, true)
+      : ma_flash::applies(desc, ptrs, 8)  // dense, head_dim 64
           ? ma_flash::backward(desc, ptrs, sf, o, lse, st)
           : (desc->dtype == MA_ATTN_BF16 ? launch_backward_mfma<HalfPath<__bf16>>(desc, ptrs, sf, st, o, lse)
              : desc->dtype == MA_ATTN_F16

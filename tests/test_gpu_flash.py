@@ -80,6 +80,26 @@ def test_flash_dense_grids(ext, oracle, N, H, causal):
     assert float(np.abs(y[:, :, [0, H - 1]] - ref).max()) <= 1e-5
 
 
+@pytest.mark.parametrize("B,N,H,causal", [(1, 300, 2, True), (1, 257, 2, False), (2, 4097, 3, True),
+                                          (1, 8200, 16, True), (1, 4100, 16, False)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_flash_saved_statistics_half(ext, oracle, B, N, H, causal, dtype):
+    """16-bit dense gradients at head_dim 64 from saved statistics on each
+    grid: one row group per wave, pairs of tiles (2 x 3 heads of 4097 rows:
+    198 128-row tiles), two row groups (16 heads); the first and last head
+    against the oracle."""
+    shape = (B, N, H, 64)
+    arrs = [*qkv(shape, 8700 + N), randn(shape, 8710 + N)]
+    q, k, v, g = (torch.from_numpy(a).to(dtype).cuda() for a in arrs)
+    out, lse = ext.dense_forward(q, k, v, causal, return_lse=True)
+    got = ext.dense_backward(q, k, v, g, causal, out=out, lse=lse)
+    for b, h in ((0, 0), (B - 1, H - 1)):
+        one = [np.ascontiguousarray(t[b:b + 1, :, h:h + 1].float().cpu().numpy()) for t in (q, k, v, g)]
+        ref = oracle.backward(oracle.Spec(1, N, 1, 64, pattern="dense", causal=causal), *one)
+        for name, x, y in zip("qkv", got, ref):
+            check_grad("d" + name, x[b:b + 1, :, h:h + 1].float().cpu().numpy(), y, False)
+
+
 @pytest.mark.parametrize("N,causal", [(300, True), (257, False), (65, True)])
 def test_flash_saved_statistics(ext, oracle, N, causal):
     """float32 dense training pair at head_dim 64: the forward's statistics
