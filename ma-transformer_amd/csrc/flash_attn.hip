@@ -49,13 +49,13 @@ FlArgs args_of(const ma_attn_desc* d) {
   return a;
 }
 
-template <typename T, int ND, int NQ, int NW, int KB, bool DB, int OCC>
+template <typename T, int ND, int NQ, int NW, int KB, bool DB, int OCC, int NPB = FlElt<T>::NPB>
 int run_fwd(const ma_attn_desc* d, FlArgs a, hipStream_t st) {
   Band b;
   band_of(d, &b);
   constexpr int QT = 16 * NQ * NW;
   constexpr size_t shm = (size_t)(DB ? 2 : 1) * 2 * FlStage<T, ND, KB, NW>::kMat;
-  auto kern = &flash_fwd_kernel<T, ND, NQ, NW, KB, DB, OCC>;
+  auto kern = &flash_fwd_kernel<T, ND, NQ, NW, KB, NPB, DB, OCC>;
   if (ma_host::reserve_lds(reinterpret_cast<const void*>(kern), shm, st)) return 1;
   a.tiles = (int32_t)((b.nr + QT - 1) / QT);
   const int64_t wgs = d->batch * d->num_heads * b.dil * a.tiles;
@@ -121,6 +121,10 @@ int fwd_nd(const ma_attn_desc* d, const FlArgs& a, hipStream_t st) {
     if (b.left >= b.nr && tiles128 >= 1024) return run_fwd<T, ND, 2, 8, KB, false, 2>(d, a, st);
     if (tiles128 >= 256) return run_fwd<T, ND, 1, 8, KB, false, 2>(d, a, st);
   }
+  // head_dim 64 in 16 bits: P in 16 bits, as in the stream kernel that these
+  // windows took before; four workgroups to a CU
+  if constexpr (!f32 && ND == 2)
+    if (d->head_dim == 64) return run_fwd<T, ND, 1, 4, KB, false, 4, 1>(d, a, st);
   if constexpr (!f32 && ND == 1)
     if (b.left + b.right < 128) return run_fwd<T, ND, 1, 4, 128, false, 3>(d, a, st);
   return run_fwd<T, ND, 1, 4, KB, false, f32 ? 2 : 3>(d, a, st);

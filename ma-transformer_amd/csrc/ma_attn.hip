@@ -1644,12 +1644,30 @@ bool bwd_two_blocks(int64_t L, int64_t R) {
 // (8 heads of 32768 rows, stream / these: [i-63, i] forward 65 / 62 us,
 // backward 234 / 263; [i-100, i] 114 / 80 and 466 / 344; [i-64, i+64] 121 / 82
 // and 490 / 361; dense causal, 8 heads of 4000 rows: 211 / 136 and 924 / 594).
+//
+// 16-bit at head_dim 64: forward windows with a right side, past 48 keys, and
+// causal ones past 256, where the stream kernel's ring of 64-row slots leaves
+// one workgroup to a CU.  bf16, 8 heads of 65536 rows, stream / these:
+// [i-16, i+3] 60 / 64 us, [i-40, i+10] 69 / 65, [i-32, i+32] 72 / 65,
+// [i-64, i+64] 99 / 78, [i-200, i+50] 164 / 116; [i-100, i] 71 / 76,
+// [i-130, i] 84 / 90, [i-180, i] 92 / 92; 16384 rows: [i-300, i+300] 101 / 51,
+// [i-1000, i] 146 / 76; 4096 rows: [i-300, i] 18.1 / 14.2.  [i-32, i+31] has a
+// stream kernel of its own with the window at compile time (4 x 8 heads of
+// 8192 rows: 31.9 / 33.5).
 bool flash_route(const ma_attn_desc* d, const void* const* ptrs, int n, bool backward) {
-  if (!ma_flash::applies(d, ptrs, n)) return false;
-  if (d->head_dim != kHeadDim) return true;
-  if (d->dtype != MA_ATTN_F32) return false;
-  if (d->pattern == MA_ATTN_DENSE) return true;
-  return backward ? !bwd_two_blocks(d->left, d->right) : d->left + d->right > 64;
+  if (d->head_dim == kHeadDim) {
+    const bool sliding = d->pattern == MA_ATTN_SLIDING;
+    const int64_t keys = ma::imin64(d->left, 1 << 30) + ma::imin64(d->right, 1 << 30);
+    if (!sliding && d->pattern != MA_ATTN_DENSE) return false;
+    if (d->dtype != MA_ATTN_F32) {
+      if (backward || !sliding) return false;
+      if (d->right == 0 ? d->left <= 256 : keys <= 48 || (d->left == 32 && d->right == 31))
+        return false;
+    } else if (sliding) {
+      if (backward ? bwd_two_blocks(d->left, d->right) : keys <= 64) return false;
+    }
+  }
+  return ma_flash::applies(d, ptrs, n);
 }
 
 // The fused backward's chunks of a stream's tiles, fitted to one round of the

@@ -67,6 +67,23 @@ def test_flash_against_oracle(ext, oracle, N, D, left, right, dil, dtype):
         check_grad("d" + name, a.float().cpu().numpy(), b, dtype == torch.float32)
 
 
+@pytest.mark.parametrize("N,left,right,dil", [(64, 48, 1, 1), (129, 64, 64, 1), (700, 257, 0, 1), (321, 0, 49, 2),
+                                               (1030, 300, 300, 1), (65, 1000, 0, 1), (500, 700, 200, 3)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_flash_half_windows_at_64(ext, oracle, N, left, right, dil, dtype):
+    """16-bit forward windows at head_dim 64 past the stream kernel's: each
+    weight is rounded to 16 bits (by at most a part in 2^8 in bf16, 2^11 in f16,
+    so that times sum p |v| bounds the row's error) and the row once more."""
+    q, k, v = (torch.from_numpy(a).to(dtype).cuda() for a in qkv((2, N, 3, 64), 8800 + N))
+    up = [t.float().cpu().numpy() for t in (q, k, v)]
+    spec = _spec(oracle, (2, N, 3, 64), left, right, dil)
+    y = ext.sliding_forward(q, k, v, left, right, dil).float().cpu().numpy()
+    ref, mass = oracle.forward(spec, *up), oracle.forward(spec, *up[:2], np.abs(up[2]))
+    u = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}[dtype]
+    err = np.abs(y - ref)
+    assert (err <= 1e-4 + u * np.abs(ref) + u * mass).all(), float(err.max())
+
+
 @pytest.mark.parametrize("N,H,causal", [(4200, 8, True), (9000, 16, True), (3000, 16, False)])
 def test_flash_dense_grids(ext, oracle, N, H, causal):
     """float32 dense rows at head_dim 64 where the tiles pass one per CU (no
