@@ -866,7 +866,10 @@ __global__ __launch_bounds__(256, LG ? 2 : P::kMinBlocks) void stream_kernel(Str
       if (a.lse && g == 0 && m < Nr) a.lse[row] = lse2;
       if (dm && g == 0 && m < Nr) a.delta[row] = dlt;
     }
-    if (LG) {  // global query rows against keys 64t + 16wv .. +15 (in the ring at tile t)
+    // Global query rows against keys 64t + 16wv .. +15 (in the ring at tile t).
+    // A wave past the last key skips: its slot may never have been stored (fp32,
+    // half a tile), and a weight of 0 times what LDS then holds may be NaN.
+    if (LG && t * 64 + 16 * wv < Nr) {  // wave-uniform
       const int key0 = t * 64 + 16 * wv;
       constexpr int kSubs = RS / 16;
       f32x4 z = P::qk(ring + ring_slot_bytes<P, NSLOT>(key0 / 16) + P::k_sub((key0 / 16) % kSubs) + kl, qg);
@@ -938,14 +941,13 @@ __global__ __launch_bounds__(256, LG ? 2 : P::kMinBlocks) void stream_kernel(Str
     }
     float lt = 0.0f, dtt = 0.0f;
     f32x4 at = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    if (mt != -INFINITY) {
+    const float mr = mt == -INFINITY ? 0.0f : mt;  // a NaN among the sums is kept, also where no score was a number
 #pragma unroll
-      for (int w = 0; w < 4; ++w) {
-        const float cw = __builtin_amdgcn_exp2f(mw[w] - mt);  // 0 for a wave that saw no key
-        lt = fmaf(sp[w * 16 * kRowF + kHeadDim + 1], cw, lt);
-        dtt = fmaf(sp[w * 16 * kRowF + kHeadDim + 2], cw, dtt);
-        at += *reinterpret_cast<const f32x4*>(sp + w * 16 * kRowF + d0) * cw;
-      }
+    for (int w = 0; w < 4; ++w) {
+      const float cw = __builtin_amdgcn_exp2f(mw[w] - mr);  // 0 for a wave that saw no key
+      lt = fmaf(sp[w * 16 * kRowF + kHeadDim + 1], cw, lt);
+      dtt = fmaf(sp[w * 16 * kRowF + kHeadDim + 2], cw, dtt);
+      at += *reinterpret_cast<const f32x4*>(sp + w * 16 * kRowF + d0) * cw;
     }
     float* dst = a.partials + ((((int64_t)b * a.H + h) * a.chunks + chunk_id) * 16 + qq) * kPartial;
     *reinterpret_cast<f32x4*>(dst + d0) = at;  // rows of 68 floats: 16 B aligned
@@ -996,20 +998,19 @@ __global__ __launch_bounds__(256) void longformer_combine(const float* __restric
     float mb = m;
 #pragma unroll
     for (int k = 0; k < 8; ++k) mb = fmaxf(mb, mk[k]);
-    if (mb != -INFINITY) {
-      const float c = __builtin_amdgcn_exp2f(m - mb);  // 0 while m is -inf
-      l *= c;
-      acc *= c;
-      dsum *= c;
+    const float mr = mb == -INFINITY ? 0.0f : mb;
+    const float c = __builtin_amdgcn_exp2f(m - mr);  // 0 while m is -inf
+    l *= c;
+    acc *= c;
+    dsum *= c;
 #pragma unroll
-      for (int k = 0; k < 8; ++k) {
-        const float w = __builtin_amdgcn_exp2f(mk[k] - mb);  // 0 for a partial that saw no key
-        l = fmaf(lk[k], w, l);
-        acc = fmaf(ak[k], w, acc);
-        dsum = fmaf(dk[k], w, dsum);
-      }
-      m = mb;
+    for (int k = 0; k < 8; ++k) {
+      const float w = __builtin_amdgcn_exp2f(mk[k] - mr);  // 0 for a partial that saw no key
+      l = fmaf(lk[k], w, l);
+      acc = fmaf(ak[k], w, acc);
+      dsum = fmaf(dk[k], w, dsum);
     }
+    m = mb;
   }
   sh[wv][d] = acc;
   if (d == 0) {
@@ -1023,20 +1024,19 @@ __global__ __launch_bounds__(256) void longformer_combine(const float* __restric
 #pragma unroll
     for (int w = 0; w < 4; ++w) mt = fmaxf(mt, sh[w][kHeadDim]);
     float lt = 0.0f, at = 0.0f, dt = 0.0f;
-    if (mt != -INFINITY) {
+    const float mr = mt == -INFINITY ? 0.0f : mt;
 #pragma unroll
-      for (int w = 0; w < 4; ++w) {
-        const float c = __builtin_amdgcn_exp2f(sh[w][kHeadDim] - mt);
-        lt = fmaf(sh[w][kHeadDim + 1], c, lt);
-        at = fmaf(sh[w][d], c, at);
-        dt = fmaf(sh[w][kHeadDim + 2], c, dt);
-      }
+    for (int w = 0; w < 4; ++w) {
+      const float c = __builtin_amdgcn_exp2f(sh[w][kHeadDim] - mr);
+      lt = fmaf(sh[w][kHeadDim + 1], c, lt);
+      at = fmaf(sh[w][d], c, at);
+      dt = fmaf(sh[w][kHeadDim + 2], c, dt);
     }
     const int64_t row = ((int64_t)b * N + gq) * H + h;
     if (dm) {  // delta mode: the row's sum_j P_ij dP_ij; O not written
       if (d == 0) delta[row] = lt > 0.0f ? dt / lt : 0.0f;
     } else {
-      o[row * kHeadDim + d] = static_cast<Elt>(lt > 0.0f ? at / lt : 0.0f);
+      o[row * kHeadDim + d] = static_cast<Elt>(lt != 0.0f ? at / lt : 0.0f);
     }
     // the global row's statistic (mt is in log2 units of the scaled scores)
     if (lse && d == 0) lse[row] = lt > 0.0f ? mt + __log2f(lt) : 0.0f;

@@ -84,6 +84,20 @@ def test_flash_half_windows_at_64(ext, oracle, N, left, right, dil, dtype):
     assert (err <= 1e-4 + u * np.abs(ref) + u * mass).all(), float(err.max())
 
 
+@pytest.mark.parametrize("N", [12, 32, 70, 96])
+def test_longformer_float32_last_half_tile(ext, oracle, N):
+    """float32 Longformer on the stream kernel with at least half of the last
+    tile past the end, after a call that leaves NaN in LDS."""
+    nan = torch.full((1, 256, 8, 64), float("nan"), device="cuda")
+    arrs = qkv((1, N, 2, 64), 8960 + N)
+    q, k, v = (torch.from_numpy(a).cuda() for a in arrs)
+    ref = oracle.forward(oracle.Spec(1, N, 2, 64, pattern="longformer", left=0, right=0, num_global=5), *arrs)
+    for _ in range(3):
+        ext.longformer_forward(nan, nan, nan, 7, 0, 5)
+        y = ext.longformer_forward(q, k, v, 0, 0, 5)
+        assert float(np.abs(y.cpu().numpy() - ref).max()) <= 1e-5
+
+
 @pytest.mark.parametrize("N,H,causal", [(4200, 8, True), (9000, 16, True), (3000, 16, False)])
 def test_flash_dense_grids(ext, oracle, N, H, causal):
     """float32 dense rows at head_dim 64 where the tiles pass one per CU (no
