@@ -49,13 +49,13 @@ FlArgs args_of(const ma_attn_desc* d) {
   return a;
 }
 
-template <typename T, int ND, int NQ, int NW, int KB, bool DB, int OCC, int NPB = FlElt<T>::NPB>
+template <typename T, int ND, int NQ, int NW, int KB, bool DB, int OCC, int NPB = FlElt<T>::NPB, bool GL = false>
 int run_fwd(const ma_attn_desc* d, FlArgs a, hipStream_t st) {
   Band b;
   band_of(d, &b);
   constexpr int QT = 16 * NQ * NW;
   constexpr size_t shm = (size_t)(DB ? 2 : 1) * 2 * FlStage<T, ND, KB, NW>::kMat;
-  auto kern = &flash_fwd_kernel<T, ND, NQ, NW, KB, NPB, DB, OCC>;
+  auto kern = &flash_fwd_kernel<T, ND, NQ, NW, KB, NPB, DB, OCC, GL>;
   if (ma_host::reserve_lds(reinterpret_cast<const void*>(kern), shm, st)) return 1;
   a.tiles = (int32_t)((b.nr + QT - 1) / QT);
   const int64_t wgs = d->batch * d->num_heads * b.dil * a.tiles;
@@ -242,6 +242,20 @@ int forward(const ma_attn_desc* d, const void* q, const void* k, const void* v, 
     case MA_ATTN_BF16: return fwd_t<__bf16>(d, a, st);
     default: return fwd_t<_Float16>(d, a, st);
   }
+}
+
+int forward_globals(const ma_attn_desc* d, int64_t num_global, const void* q, const void* k, const void* v, void* o,
+                    hipStream_t st) {
+  FlArgs a = args_of(d);
+  a.q = q;
+  a.k = k;
+  a.v = v;
+  a.o = o;
+  a.globals = (int32_t)num_global;
+  a.desc = 0;
+  if (d->batch * d->num_heads * ((d->seq_len + 127) / 128) >= 256)
+    return run_fwd<float, 2, 1, 8, 64, false, 2, FlElt<float>::NPB, true>(d, a, st);
+  return run_fwd<float, 2, 1, 4, 64, false, 2, FlElt<float>::NPB, true>(d, a, st);
 }
 
 int backward(const ma_attn_desc* d, const void* const* ptrs, float* stats, const void* fo, const float* lse,

@@ -49,6 +49,7 @@ struct FlArgs {
   int32_t H, D, left, right, dil;
   int32_t tiles;      // tiles of the longest residue class
   int32_t desc;       // 1: the last tile first (causal rows: longest first)
+  int32_t globals;    // forward, GL kernels: keys 0..globals-1 (at most 16) join every row's window
   uint32_t tok_bytes; // bytes between consecutive rows of a residue class
   float scale, scale_log2;
 };
@@ -401,7 +402,9 @@ __device__ __forceinline__ void fl_fwd_row(const FlArgs& a, const FlPos& ps, int
   }
   float m = -INFINITY, l = 0.0f;
   const int j0 = max(0, i - a.left), j1 = min(ps.Nr - 1, i + a.right);
-  for (int j = j0; j <= j1; ++j) {
+  const int ng = min(j0, a.globals);
+  for (int e = j0 - ng; e <= j1; ++e) {
+    const int j = e < j0 ? e - (j0 - ng) : e;
     float s = 0.0f;
 #pragma unroll
     for (int c = 0; c < NC; ++c) s = fmaf(qd[c], fl_at(k, j, rs, lane + 64 * c, a.D), s);
@@ -422,7 +425,11 @@ __device__ __forceinline__ void fl_fwd_row(const FlArgs& a, const FlPos& ps, int
 
 constexpr float kSlack = 8.0f;
 
-template <typename T, int ND, int NQ, int NW, int KB, int NPB, bool DB, int OCC>
+// GL (Longformer windows; one residue class, one buffer): after the window's
+// blocks one more holds the global keys, of which a row takes those before its
+// window.  Rows below `globals` are not written: they attend every key and
+// another kernel splits them.
+template <typename T, int ND, int NQ, int NW, int KB, int NPB, bool DB, int OCC, bool GL>
 __global__ __launch_bounds__(64 * NW, OCC) void flash_fwd_kernel(FlArgs a) {
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
   using St = FlStage<T, ND, KB, NW>;
@@ -445,7 +452,8 @@ __global__ __launch_bounds__(64 * NW, OCC) void flash_fwd_kernel(FlArgs a) {
   const int qa = q0 + 16 * NQ * wv;  // the wave's first query
   const int k0 = max(0, q0 - L) & ~15;
   const int kend = min(Nr, q0 + 16 * NQ * NW + R);
-  const int nb = (kend - k0 + KB - 1) / KB;
+  const int nwin = (kend - k0 + KB - 1) / KB;
+  const int nb = nwin + (GL && q0 + 16 * NQ * NW - 1 > L ? 1 : 0);
 
   St ks, vs;
   ks.load(Kr, k0, tid, tb, D);
@@ -471,15 +479,19 @@ __global__ __launch_bounds__(64 * NW, OCC) void flash_fwd_kernel(FlArgs a) {
 
   for (int e = 0; e < nb; ++e) {
     if (e + 1 < nb) {
-      ks.load(Kr, k0 + (e + 1) * KB, tid, tb, D);
-      vs.load(Vr, k0 + (e + 1) * KB, tid, tb, D);
+      const int next = GL && e + 1 == nwin ? 0 : k0 + (e + 1) * KB;
+      ks.load(Kr, next, tid, tb, D);
+      vs.load(Vr, next, tid, tb, D);
     }
     __builtin_amdgcn_sched_barrier(0);
     const uint8_t* buf = lds + (DB && (e & 1) ? BUF : 0);
-    const int key0 = k0 + e * KB;
+    const bool glob = GL && e == nwin;
+    const int key0 = glob ? 0 : k0 + e * KB;
     // sub-tiles [u0, u1] of the block meet some window of the wave
-    const int u0 = max(0, (qa - L - key0) >> 4);
-    const int u1 = qa < Nr ? min(NU - 1, (min(qa + 16 * NQ - 1 + R, Nr - 1) - key0) >> 4) : -1;
+    const int u0 = glob ? 0 : max(0, (qa - L - key0) >> 4);
+    const int u1 = qa >= Nr ? -1
+                   : glob   ? (qa + 16 * NQ - 1 > L ? 0 : -1)
+                            : min(NU - 1, (min(qa + 16 * NQ - 1 + R, Nr - 1) - key0) >> 4);
     if (u0 <= u1) {  // wave-uniform
       f32x4 sc[NU][NQ];
       float mx[NQ], mu[NQ];
@@ -493,7 +505,12 @@ __global__ __launch_bounds__(64 * NW, OCC) void flash_fwd_kernel(FlArgs a) {
 #pragma unroll
           for (int n = 0; n < NQ; ++n) {
             const int rel = key - (qa + 16 * n);  // key - query offsets span rel -+ 15
-            if (rel - 15 < -L || rel + 15 > R || key + 15 >= Nr) {
+            if (GL && glob) {
+              const int x = rel + 4 * g - c;
+#pragma unroll
+              for (int r = 0; r < 4; ++r)
+                sc[u][n][r] = x + r < -L && 4 * g + r < a.globals ? sc[u][n][r] : -INFINITY;
+            } else if (rel - 15 < -L || rel + 15 > R || key + 15 >= Nr) {
               const int x = rel + 4 * g - c, hi = min(R, Nr - 1 - (qa + 16 * n) - c);
 #pragma unroll
               for (int r = 0; r < 4; ++r) sc[u][n][r] = x + r >= -L && x + r <= hi ? sc[u][n][r] : -INFINITY;
@@ -573,8 +590,8 @@ __global__ __launch_bounds__(64 * NW, OCC) void flash_fwd_kernel(FlArgs a) {
     const float inv = l_tot != 0.0f ? 1.0f / l_tot : 0.0f;
     const int i = qa + 16 * n + c;
     // bit r of each lane group: row r is left to fl_fwd_row
-    const uint64_t bad = __builtin_amdgcn_ballot_w64(i < Nr && (fl_bad<ND>(acc[n]) || !(l_tot < INFINITY)));
-    const bool own_bad = (bad >> c & 0x0001000100010001ull) != 0;
+    const uint64_t bad = __builtin_amdgcn_ballot_w64(i < Nr && !(GL && i < a.globals) && (fl_bad<ND>(acc[n]) || !(l_tot < INFINITY)));
+    const bool own_bad = (bad >> c & 0x0001000100010001ull) != 0 || (GL && i < a.globals);
     fl_store<T, ND>(acc[n], inv, Or, own_bad ? kOob : (uint32_t)i * tb, D, g);
     if (a.lse && g == 0 && i < Nr)
       a.lse[((int64_t)ps.b * a.N + ps.rho + (int64_t)a.dil * i) * a.H + ps.h] =

@@ -1670,6 +1670,41 @@ bool flash_route(const ma_attn_desc* d, const void* const* ptrs, int n, bool bac
   return ma_flash::applies(d, ptrs, n);
 }
 
+// float32 Longformer rows whose window passes the stream kernel's ring (left >
+// 128): the rows past the globals on the banded kernels with the global keys as
+// one more block; the global rows, which attend every key, from a pass of the
+// stream kernel with a one-key window (whose other rows the banded kernel then
+// writes over) and its merge.  The gather kernel read every key once per row:
+// LF_FIGURES
+struct LfWide {
+  ma_attn_desc rows, globals;  // the banded rows as a window; the global rows' stream pass
+  size_t ws_bytes;
+};
+bool lf_wide(const ma_attn_desc* d, const void* q, const void* k, const void* v, const void* o, LfWide* w) {
+  if (d->pattern != MA_ATTN_LONGFORMER || d->dtype != MA_ATTN_F32 || d->head_dim != kHeadDim || d->num_global < 1 || d->num_global > kMaxGlobal ||
+      d->left < 0 || d->right < 0)
+    return false;
+  w->rows = w->globals = *d;
+  w->rows.pattern = MA_ATTN_SLIDING;
+  w->rows.dilation = 1;
+  w->globals.left = w->globals.right = 0;
+  const void* const qkvo[4] = {q, k, v, o};
+  if (stream_applies(d, q, k, v, o) || !stream_applies(&w->globals, q, k, v, o) ||
+      !ma_flash::applies(&w->rows, qkvo, 4))
+    return false;
+  w->ws_bytes = (size_t)stream_plan(&w->globals).partial_bytes;
+  return true;
+}
+
+int launch_lf_wide(const LfWide& w, const void* q, const void* k, const void* v, void* o, void* ws, size_t ws_bytes,
+                   hipStream_t st) {
+  hipEvent_t stop = g_ev_stop;  // the banded kernel is the last
+  g_ev_stop = nullptr;
+  const int rc = launch_stream(&w.globals, q, k, v, o, nullptr, ws, ws_bytes, st);
+  g_ev_stop = stop;
+  return rc ? rc : ma_flash::forward_globals(&w.rows, ma::imin64(w.rows.num_global, w.rows.seq_len), q, k, v, o, st);
+}
+
 // The fused backward's chunks of a stream's tiles, fitted to one round of the
 // resident workgroups (two per CU).
 void fused_chunks(BwdArgs& a, int64_t streams) {
@@ -2126,6 +2161,8 @@ size_t ma_attn_workspace_size(const ma_attn_desc* desc) {
   const void* const ptrs[4] = {dummy, dummy, dummy, dummy};
   if (tiles_apply(desc, ptrs, 4)) return (size_t)tiles_fwd_part_bytes(desc);
   if (desc->pattern != MA_ATTN_LONGFORMER) return 0;
+  LfWide wide;
+  if (lf_wide(desc, dummy, dummy, dummy, dummy, &wide)) return wide.ws_bytes;
   if (!stream_applies(desc, dummy, dummy, dummy, dummy)) return 0;
   return (size_t)stream_plan(desc).partial_bytes;
 }
@@ -2215,6 +2252,9 @@ int forward_launch(const ma_attn_desc* desc, const void* q, const void* k, const
         rc = launch_tiles_fwd<HalfPath<_Float16>>(desc, q, k, v, o, lse, workspace, workspace_bytes, st);
         break;
     }
+  } else if (LfWide wide; !want_rows && !want_band && lf_wide(desc, q, k, v, o, &wide) && workspace &&
+                          workspace_bytes >= wide.ws_bytes) {
+    rc = launch_lf_wide(wide, q, k, v, o, workspace, workspace_bytes, st);
   } else if (!want_rows && gather_applies(desc, q, k, v, o)) {
     switch (desc->dtype) {
       case MA_ATTN_F32:

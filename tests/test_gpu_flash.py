@@ -84,6 +84,35 @@ def test_flash_half_windows_at_64(ext, oracle, N, left, right, dil, dtype):
     assert (err <= 1e-4 + u * np.abs(ref) + u * mass).all(), float(err.max())
 
 
+@pytest.mark.parametrize("N,H,left,right,G", [(300, 3, 129, 0, 16), (1100, 2, 200, 5, 3), (90, 2, 300, 0, 16),
+                                              (12, 2, 200, 0, 16), (4300, 8, 131, 64, 1)])
+def test_flash_wide_longformer(ext, oracle, N, H, left, right, G):
+    """float32 Longformer windows past the stream kernel's ring: global rows
+    from its partials, the others on the banded kernels (grids of 4 and 8
+    waves), the window covering the globals, parted from them, and longer than
+    the sequence; without a workspace the gather kernel.  The gradients run over
+    split lists of the global tile and block."""
+    import ma_attn as ma
+    shape = (1, N, H, 64)
+    arrs = [*qkv(shape, 8900 + N), randn(shape, 8910 + N)]
+    q, k, v, g = (torch.from_numpy(a).cuda() for a in arrs)
+    heads = sorted({0, H - 1})
+    up = [np.ascontiguousarray(a[:, :, heads]) for a in arrs]
+    spec = oracle.Spec(1, N, len(heads), 64, pattern="longformer", left=left, right=right, num_global=G)
+    ref = oracle.forward(spec, *up[:3])
+    gather = torch.empty_like(q)
+    desc = ma.make_desc(*shape, ma.F32, ma.LONGFORMER, left=left, right=right, num_global=G)
+    assert ma.workspace_size(desc) > 0
+    ma.forward_raw(desc, q.data_ptr(), k.data_ptr(), v.data_ptr(), gather.data_ptr(), 0, 0,
+                   torch.cuda.current_stream().cuda_stream)
+    for y in (ext.longformer_forward(q, k, v, left, right, G), gather):
+        assert float(np.abs(y.cpu().numpy()[:, :, heads] - ref).max()) <= 1e-5
+    if N < 2000:
+        grads = ext.longformer_backward(q, k, v, g, left, right, G)
+        for name, x, y in zip("qkv", grads, oracle.backward(spec, *up)):
+            check_grad("d" + name, x.cpu().numpy()[:, :, heads], y, True)
+
+
 @pytest.mark.parametrize("N", [12, 32, 70, 96])
 def test_longformer_float32_last_half_tile(ext, oracle, N):
     """float32 Longformer on the stream kernel with at least half of the last
@@ -96,6 +125,23 @@ def test_longformer_float32_last_half_tile(ext, oracle, N):
         ext.longformer_forward(nan, nan, nan, 7, 0, 5)
         y = ext.longformer_forward(q, k, v, 0, 0, 5)
         assert float(np.abs(y.cpu().numpy() - ref).max()) <= 1e-5
+
+
+def test_flash_wide_longformer_bad_values(ext):
+    """A NaN key and value reach the rows that attend them and no others."""
+    N, left, G, bad = 700, 150, 4, 300
+    q, k, v = (torch.from_numpy(a).cuda() for a in qkv((1, N, 2, 64), 8950))
+    want = ext.longformer_forward(q, k, v, left, 0, G)
+    k[0, bad, 0] = v[0, bad, 0] = float("nan")
+    got = ext.longformer_forward(q, k, v, left, 0, G)
+    i = torch.arange(N, device="cuda")
+    hit = (i < G) | ((i >= bad) & (i <= bad + left))
+    assert bool(got[0, hit, 0].isnan().all())
+    assert float((got[0, ~hit, 0] - want[0, ~hit, 0]).abs().max()) <= 1e-5
+    assert torch.equal(got[0, :, 1], want[0, :, 1])
+    q[0, 1, 1] = float("nan")  # a global row with no score that is a number
+    got = ext.longformer_forward(q, k, v, left, 0, G)
+    assert bool(got[0, 1, 1].isnan().all()) and torch.equal(got[0, 2:, 1], want[0, 2:, 1])
 
 
 @pytest.mark.parametrize("N,H,causal", [(4200, 8, True), (9000, 16, True), (3000, 16, False)])
