@@ -374,13 +374,13 @@ class IndexSet:
 _pattern_sets: dict = {}
 
 
-def _enumerated_set(code: int, seq_len: int, device, host_table=None, **kw) -> "IndexSet":
+def _enumerated_set(code: int, seq_len: int, device, host_table=None, tile_seg=0, **kw) -> "IndexSet":
     tptr = host_table.data_ptr() if host_table is not None else 0  # host pointer: enumeration only
     if host_table is not None:
         kw["blocks_per_row"] = int(host_table.shape[1])
     desc = _ma.make_desc(1, seq_len, 1, 64, _ma.F32, code, block_table_ptr=tptr, **kw)
     offsets, keys = _ma.pattern_csr(desc, host_table)
-    return IndexSet(offsets, keys, seq_len, device)
+    return IndexSet(offsets, keys, seq_len, device, tile_seg=tile_seg)
 
 
 def pattern_index_set(pattern: str, seq_len: int, device, **kw) -> IndexSet:
@@ -419,7 +419,16 @@ def pattern_index_set(pattern: str, seq_len: int, device, **kw) -> IndexSet:
     if hit is None:
         if len(_pattern_sets) > 16:
             _pattern_sets.clear()
-        hit = _pattern_sets[key] = _enumerated_set(_ma.LONGFORMER, seq_len, device, **kw)
+        # The global rows' tile and the global keys' block list every block of the
+        # sequence, and a work item walks its list serially: 8 blocks an item (the
+        # plan's default is 32), or a window tile's own list where that is longer,
+        # so that only the global ones are split.  float32 training, default ->
+        # here: 2 streams of 3422 rows 339 -> 118 us, 12 of 5976 442 -> 225, 12 of
+        # 12000 595 -> 435; bf16, 8 of 19119 rows 175 -> 170.  4 an item splits the
+        # window tiles too: 94, 199 and 423, but 289 on the bf16 one.
+        window = (int(kw["left"]) + int(kw["right"]) + 63) // 64 + 3
+        hit = _pattern_sets[key] = _enumerated_set(_ma.LONGFORMER, seq_len, device,
+                                                   tile_seg=min(32, max(8, window)), **kw)
     return hit
 
 
