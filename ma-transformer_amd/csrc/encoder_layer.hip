@@ -653,7 +653,7 @@ extern "C" int ma_encoder_model_forward(const ma_encoder_model* M, const float* 
   if (!M) return fail("ma_encoder_model_forward: null model");
   const int64_t D = M->d_model, max_seq = ma_encoder_model_max_seq(D);
   if (max_seq == 0) return fail("ma_encoder_model_forward: d_model %lld unsupported (16, 32, 64 or 128)", (long long)D);
-  if (M->batch < 0 || M->batch > (int64_t)INT32_MAX) return fail("ma_encoder_model_forward: bad batch");
+  if (M->batch < 0 || M->batch > (1LL << 30)) return fail("ma_encoder_model_forward: bad batch");
   if (M->seq_len < 1 || M->seq_len > max_seq)
     return fail("ma_encoder_model_forward: seq_len must be in [1, %lld]", (long long)max_seq);
   if (M->input_dim < 1 || M->input_dim > (1 << 16)) return fail("ma_encoder_model_forward: bad input_dim");

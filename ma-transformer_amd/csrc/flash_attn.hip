@@ -63,15 +63,6 @@ int run_fwd(const ma_attn_desc* d, FlArgs a, hipStream_t st) {
   return 0;
 }
 
-// One query group per wave, 4 waves, 64-key blocks in one buffer: measured
-// best of 1 or 2 groups, 4 or 8 waves, 32- or 64-key blocks and one or two
-// buffers at head_dim 32 and 128 (causal 128-key window, bf16, head_dim 128,
-// 8 heads, 32768 rows: 83 us against 87-104; two-sided 64-key window, head_dim
-// 32, 4 x 8 heads, 8191 rows: f16 26 us against 28-31, f32 43 us against
-// 43-70).  16-bit windows of at most 128 keys at head_dim 32 take 128-key
-// blocks: a 64-query tile of a 64-key window is then one block (22 us against
-// 24 on the f16 window above).  float32 above head_dim 64 takes 32-key blocks (three planes of 64
-// rows would leave one workgroup per CU, or spill).
 // Causal rows, the longest and the shortest tile of a stream in one workgroup.
 template <typename T, int ND, int NW, int KB>
 int run_pair(const ma_attn_desc* d, FlArgs a, hipStream_t st) {
@@ -95,8 +86,8 @@ int run_pair(const ma_attn_desc* d, FlArgs a, hipStream_t st) {
 // 32, 4 x 8 heads, 8191 rows: f16 26 us against 28-31, f32 43 us against
 // 43-70).  16-bit windows of at most 128 keys at head_dim 32 take 128-key
 // blocks: a 64-query tile of a 64-key window is then one block (22 us against
-// 24 on the f16 window above).  float32 above head_dim 64 takes 32-key blocks (three planes of 64
-// rows would leave one workgroup per CU, or spill).
+// 24 on the f16 window above).  float32 above head_dim 64 takes 32-key blocks
+// (three planes of 64 rows would leave one workgroup per CU, or spill).
 //
 // Causal rows whose 128-row tiles are at most one per CU run in pairs, longest
 // with shortest (float32, head_dim 64, 8 heads of 4000 rows: 136 us against
