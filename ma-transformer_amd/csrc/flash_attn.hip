@@ -215,9 +215,13 @@ bool applies(const ma_attn_desc* d, const void* const* ptrs, int n) {
   for (int i = 0; i < n; ++i)
     if (!aligned16(ptrs[i])) return false;
   const int64_t tb = b.dil * d->num_heads * d->head_dim * elt_of(d);
-  // every byte offset a workgroup forms, and the 16-row tiles' ids
-  return (b.nr + 512) * tb < (1LL << 31) && b.nr < (1LL << 29) &&
-         d->batch * d->num_heads * b.dil * ((b.nr + 15) / 16) <= (int64_t)INT32_MAX;
+  // every byte offset a workgroup forms, the 16-row tiles' ids, and a launch's
+  // 2^32 threads (64-row tiles of 256 and 128-row tiles of 512: many short
+  // sequences reach it first)
+  const int64_t streams = d->batch * d->num_heads * b.dil;
+  return (b.nr + 512) * tb < (1LL << 31) && b.nr < (1LL << 29) && streams < (1LL << 31) &&
+         streams * ((b.nr + 15) / 16) <= (int64_t)INT32_MAX && streams * ((b.nr + 63) / 64) < (1LL << 24) &&
+         streams * ((b.nr + 127) / 128) < (1LL << 23);
 }
 
 int forward(const ma_attn_desc* d, const void* q, const void* k, const void* v, void* o, float* lse,

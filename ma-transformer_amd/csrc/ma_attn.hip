@@ -15,6 +15,9 @@
 //                    row, lanes over keys for the scores, lanes over head_dim
 //                    for P.V (above 512, in passes of 512 output columns).
 //                    Used where no other kernel applies.
+//   flash_fwd_kernel and its backward (flash_kernel.h, through flash_attn.h)
+//                    windows and dense rows at head_dims 8 to 128; the lines
+//                    against the other kernels are flash_route's.
 //
 // Semantics follow ma_core::compute_sparse_attention
 // (/root/reference src/csrc/ma_core.cpp:160-246): softmax over the row's key
@@ -1633,10 +1636,10 @@ bool bwd_two_blocks(int64_t L, int64_t R) {
 //
 // Head_dims other than 64 (8 to 128, a multiple of 8): in both directions.  In
 // bf16 at head_dim 128 the row kernels took 2740 us for a causal 128-key window
-// over 8 heads of 32768 rows, these take 83 us (backward over 2 x 8 heads of
+// over 8 heads of 32768 rows, these take 71 us (backward over 2 x 8 heads of
 // 4096 rows: 3017 -> 74 us); at head_dim 32 the narrow kernel took 174 us for a
-// two-sided 64-key window over 4 x 8 heads of 8191 rows (f16), these 26 us, and
-// 10.4 against 9.0 us on 4 heads of 1024 rows of 16.
+// two-sided 64-key window over 4 x 8 heads of 8191 rows (f16), these 21 us, and
+// 8.9 against 7.6 us on 4 heads of 1024 rows of 16.
 //
 // float32 at head_dim 64: dense rows, windows of more than 65 keys forward, and
 // windows past two 64-row blocks backward; shorter ones stay on the stream

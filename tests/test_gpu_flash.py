@@ -229,3 +229,17 @@ def test_flash_float32_extremes(ext):
     V = v.repeat(1, 70, 1, 1)
     o = ext.sliding_forward(q, q, V, 0, 0)
     torch.testing.assert_close(o, V, rtol=2e-7, atol=0)
+
+
+def test_flash_launch_limit(ext):
+    """2^24 one-row sequences: a workgroup each would pass a launch's 2^32
+    threads, so the row kernels (4 rows a workgroup) keep this call.  One key
+    has weight 1: O = V, dV = dO, dQ = dK = 0."""
+    shape = (1 << 22, 1, 4, 40)
+    q = torch.ones(shape, dtype=torch.bfloat16, device="cuda")
+    v = torch.arange(1 << 24, device="cuda").remainder(251).to(torch.bfloat16).view(1 << 22, 1, 4, 1).expand(shape)
+    v = v.contiguous()
+    assert torch.equal(ext.sliding_forward(q, q, v, 3, 0), v)
+    dq, dk, dv = ext.sliding_backward(q, q, q, v, 3, 0)
+    assert torch.equal(dv, v)
+    assert not dq.any() and not dk.any()
