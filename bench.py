@@ -73,6 +73,7 @@ METRIC_BWD = "sparse-attn backward queries/sec (dQ, dK, dV per query row), 1 GPU
 HBM_PEAK_GBPS = 8000.0
 MFMA_BF16_PEAK_TFLOPS = 2500.0
 MFMA_F32_PEAK_TFLOPS = 157.3
+MFMA_F32_SPLIT_PEAK_TFLOPS = MFMA_BF16_PEAK_TFLOPS / 6  # fp32 as six products of bf16 planes (dense rows)
 
 # name: (B, H, N, D, dtype, pattern kwargs, description)
 WORKLOADS = {
@@ -700,7 +701,8 @@ def measure(workload: str, which: str = "forward", saved: bool = False, steps: i
     traffic = load_traffic(tkey)
 
     # the bound is whichever peak the algorithmic work reaches first
-    mfma_peak = MFMA_BF16_PEAK_TFLOPS if dt_name == "bf16" else MFMA_F32_PEAK_TFLOPS
+    mfma_peak = (MFMA_BF16_PEAK_TFLOPS if dt_name == "bf16" else
+                 MFMA_F32_SPLIT_PEAK_TFLOPS if pk["pattern"] == "dense" else MFMA_F32_PEAK_TFLOPS)
     tflops = flops / (mean_launch_ms * 1e-3) / 1e12
     # traffic is not measured in this run: it is the committed rocprofv3 counter summary
     tsrc = f"profiles/traffic_{tkey}.txt (rocprofv3 FETCH_SIZE + WRITE_SIZE, committed)" \
