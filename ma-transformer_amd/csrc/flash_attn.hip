@@ -154,7 +154,9 @@ int run_bwd(const ma_attn_desc* d, FlArgs a, hipStream_t st) {
 
 // 4 waves and 64-row blocks (float32 above head_dim 64: 32-row): measured best
 // of 4 or 8 waves and 32- or 64-row blocks (causal 128-key window, bf16,
-// head_dim 128, 2 x 8 heads, 4096 rows: 74 us against 79-88).
+// head_dim 128, 2 x 8 heads, 4096 rows: 74 us against 79-88).  Two workgroups a
+// CU: registers for three cost more than they bring (same case, dQ 38 -> 41 us,
+// dK/dV 35 -> 63).
 //
 // Causal rows in pairs of tiles, as in the forward: float32 above head_dim 32 on
 // at most one 128-row tile per CU (8 heads of 4096 rows: head_dim 64 628 -> 561
