@@ -381,7 +381,10 @@ __device__ __forceinline__ float fl_at(const T* p, int64_t row, int64_t rs, int 
 // feeds NQ MFMAs.  Key blocks of KB rows go through LDS (DB: two buffers, the
 // next block's loads in flight while this one computes; otherwise one buffer,
 // refilled between two barriers), softmax online in registers, rescaled only
-// when a row's maximum rose.  16-key sub-tiles outside every window of the
+// when a row's maximum rose.  The running maximum is kept times scale log2(e),
+// rounded: a row whose maximum stayed is rescaled by 2^0 exactly (a difference
+// formed from the raw maximum inside one fma would leave that product's
+// rounding error, once per key block).  16-key sub-tiles outside every window of the
 // wave are skipped.
 //
 // A row whose sums come out infinite or NaN is computed again key by key
@@ -534,16 +537,16 @@ __global__ __launch_bounds__(64 * NW, OCC) void flash_fwd_kernel(FlArgs a) {
         // largest of them exact (relative error of bf16 rows against float64
         // with the slack 2.27e-3, without 2.13e-3)
         constexpr float slack = NPB == 1 ? 0.0f : kSlack;
-        mx[n] = col_max(mx[n]);
-        const bool up = !(mx[n] * sl2 <= fmaf(m_run[n], sl2, slack));
+        mx[n] = col_max(mx[n]) * sl2;
+        const bool up = !(mx[n] <= m_run[n] + slack);
         mx[n] = up ? fmaxf(m_run[n], mx[n]) : m_run[n];
-        mu[n] = mx[n] == -INFINITY ? 0.0f : mx[n] * sl2;
+        mu[n] = mx[n] == -INFINITY ? 0.0f : mx[n];
         rose = rose || up;
       }
       if (__builtin_amdgcn_ballot_w64(rose) != 0) {
 #pragma unroll
         for (int n = 0; n < NQ; ++n) {
-          const float corr = __builtin_amdgcn_exp2f(m_run[n] * sl2 - mu[n]);  // 0 on a row's first block
+          const float corr = __builtin_amdgcn_exp2f(m_run[n] - mu[n]);  // 0 on a row's first block, 1 without a rise
           l_run[n] *= corr;
 #pragma unroll
           for (int d = 0; d < 2 * ND; ++d) acc[n][d] *= corr;
@@ -595,7 +598,7 @@ __global__ __launch_bounds__(64 * NW, OCC) void flash_fwd_kernel(FlArgs a) {
     fl_store<T, ND>(acc[n], inv, Or, own_bad ? kOob : (uint32_t)i * tb, D, g);
     if (a.lse && g == 0 && i < Nr)
       a.lse[((int64_t)ps.b * a.N + ps.rho + (int64_t)a.dil * i) * a.H + ps.h] =
-          l_tot > 0.0f ? m_run[n] * sl2 + __log2f(l_tot) : 0.0f;
+          l_tot > 0.0f ? m_run[n] + __log2f(l_tot) : 0.0f;
     if (__builtin_expect(bad != 0, 0)) {
       for (int r = 0; r < 16; ++r)
         if (bad >> r & 0x0001000100010001ull) fl_fwd_row<T, (ND + 1) / 2>(a, ps, qa + 16 * n + r, lane);
@@ -700,16 +703,16 @@ __global__ __launch_bounds__(64 * NW, 2) void flash_pair_fwd_kernel(FlArgs a) {
       for (int u = 1; u < NU; ++u)
 #pragma unroll
         for (int r = 0; r < 4; ++r) mx = fl_max(mx, sc[u][n][r]);
-      mx = col_max(mx);
-      const bool up = !(mx * sl2 <= fmaf(m_run[n], sl2, kSlack));
+      mx = col_max(mx) * sl2;
+      const bool up = !(mx <= m_run[n] + kSlack);
       mn[n] = up ? fmaxf(m_run[n], mx) : m_run[n];
-      mu[n] = mn[n] == -INFINITY ? 0.0f : mn[n] * sl2;
+      mu[n] = mn[n] == -INFINITY ? 0.0f : mn[n];
       rose = rose || up;
     }
     if (__builtin_amdgcn_ballot_w64(rose) != 0) {
 #pragma unroll
       for (int n = 0; n < NQ; ++n) {
-        const float corr = __builtin_amdgcn_exp2f(m_run[n] * sl2 - mu[n]);  // 0 on a row's first block
+        const float corr = __builtin_amdgcn_exp2f(m_run[n] - mu[n]);  // 0 on a row's first block, 1 without a rise
         l_run[n] *= corr;
 #pragma unroll
         for (int d = 0; d < 2 * ND; ++d) acc[n][d] *= corr;
@@ -802,7 +805,7 @@ __global__ __launch_bounds__(64 * NW, 2) void flash_pair_fwd_kernel(FlArgs a) {
     fl_store<T, ND>(acc[n], inv, Or, own_bad ? kOob : (uint32_t)i * tb, D, g);
     if (a.lse && g == 0 && i < Nr)
       a.lse[((int64_t)ps.b * a.N + ps.rho + (int64_t)a.dil * i) * a.H + ps.h] =
-          l_tot > 0.0f ? m_run[n] * sl2 + __log2f(l_tot) : 0.0f;
+          l_tot > 0.0f ? m_run[n] + __log2f(l_tot) : 0.0f;
     if (__builtin_expect(bad != 0, 0)) {
       for (int r = 0; r < 16; ++r)
         if (bad >> r & 0x0001000100010001ull) fl_fwd_row<T, (ND + 1) / 2>(a, ps, qa + 16 * n + r, lane);
@@ -1031,9 +1034,9 @@ __global__ __launch_bounds__(64 * NW, OCC) void flash_dq_kernel(FlArgs a) {
 #pragma unroll
         for (int n = 0; n < NQ; ++n) {
           const float mn =
-              fmaxf(m[n], col_max(fmaxf(fmaxf(sc[n][0], sc[n][1]), fmaxf(sc[n][2], sc[n][3]))));
-          const float mu = mn == -INFINITY ? 0.0f : mn * sl2;
-          const float corr = __builtin_amdgcn_exp2f(m[n] * sl2 - mu);
+              fmaxf(m[n], col_max(fmaxf(fmaxf(sc[n][0], sc[n][1]), fmaxf(sc[n][2], sc[n][3]))) * sl2);
+          const float mu = mn == -INFINITY ? 0.0f : mn;
+          const float corr = __builtin_amdgcn_exp2f(m[n] - mu);  // 1 without a rise
           l[n] *= corr;
           dl[n] *= corr;
           m[n] = mn;
@@ -1049,7 +1052,7 @@ __global__ __launch_bounds__(64 * NW, OCC) void flash_dq_kernel(FlArgs a) {
 #pragma unroll
         for (int n = 0; n < NQ; ++n) {
           const float lt = col_sum(l[n]), dt = col_sum(dl[n]);
-          const float mu = m[n] == -INFINITY ? 0.0f : m[n] * sl2;
+          const float mu = m[n] == -INFINITY ? 0.0f : m[n];
           l[n] = lt != 0.0f ? 1.0f / lt : 0.0f;
           dl[n] = dt * l[n];
           const int i = qa + 16 * n + c;

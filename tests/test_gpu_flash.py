@@ -243,3 +243,31 @@ def test_flash_launch_limit(ext):
     dq, dk, dv = ext.sliding_backward(q, q, q, v, 3, 0)
     assert torch.equal(dv, v)
     assert not dq.any() and not dk.any()
+
+
+def _double(q, k, v, g, left, right):
+    """Output and gradients of [1, N, 1, D] tensors in float64 (left None: every key)."""
+    q, k, v, g = (t[0, :, 0].double().cpu() for t in (q, k, v, g))
+    scale = q.shape[1] ** -0.5
+    s = (q @ k.T) * scale
+    if left is not None:
+        d = torch.arange(len(q))[None, :] - torch.arange(len(q))[:, None]
+        s = s.masked_fill((d < -left) | (d > right), float("-inf"))
+    p = torch.softmax(s, -1)
+    dp = g @ v.T
+    ds = p * (dp - (p * dp).sum(-1, keepdim=True)) * scale
+    return p @ v, ds @ k, ds.T @ q, p.T @ g
+
+
+@pytest.mark.parametrize("N,D", [(2048, 128), (2048, 32), (4096, 64)])
+def test_flash_float32_long_rows(ext, N, D):
+    """float32 rows of thousands of keys: a weight is off by its exponent's
+    rounding, below 2^-20 for exponents down to -16, and a row's sums of N terms
+    by about sqrt(N) 2^-25, so 2^-19 of each result's norm in all; an error per
+    key block that adds up over a row (5e-6 and 1e-5 here) does not fit."""
+    q, k, v, g = (torch.from_numpy(a).cuda() for a in [*qkv((1, N, 1, D), 8990 + D), randn((1, N, 1, D), 8991 + D)])
+    got = [ext.dense_forward(q, k, v, False), *ext.dense_backward(q, k, v, g, False)]
+    for name, x, ref in zip(("o", "dq", "dk", "dv"), got, _double(q, k, v, g, None, 0)):
+        err = float((x[0, :, 0].cpu().double() - ref).norm() / ref.norm())
+        print(f"  {name}: relative error {err:.2e}", flush=True)
+        assert err <= 2.0 ** -19, name
