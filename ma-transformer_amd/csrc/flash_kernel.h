@@ -5,17 +5,21 @@
 // float32 is computed on the bf16 matrix cores.  x = x0 + x1 + x2 with x0, x1,
 // x2 the successive bf16 roundings of what is left (24 bits in all, float32's
 // exponent range), and a product takes the six partial products whose bf16
-// planes p, p' have p + p' <= 2, smallest first; the three left out are below
-// 2^-26 of it.  Six 16x16x32 MFMAs take 6/16 of the time of the sixteen
+// planes p, p' have p + p' <= 2, smallest first; the three left out come to
+// 2^-24 of it at most (x1 reaches 2^-8 of x, x2 2^-16), 2^-27 on average.  Six 16x16x32 MFMAs take 6/16 of the time of the sixteen
 // 16x16x4 fp32 MFMAs they replace, and 64-term dot products came out closer to
 // 64-bit ones (relative error 4.6e-8 against 1.44e-7 on normal data; 7.7e-8
 // against 1.24e-7 on data spread over e^(+-9)): each MFMA rounds once per 32
 // terms instead of once per term.
 //
 // 16-bit inputs multiply exactly (one plane).  Probabilities and dS are float32
-// and enter their products as a 16-bit value plus its 16-bit remainder (two
-// MFMAs, 16 or more significant bits), so nothing but the stored results is
-// rounded to 16 bits.
+// and enter their products in planes too, so that nothing but the stored
+// results is rounded to 16 bits: bf16 as the three planes above (all 24 bits),
+// f16 as a value and its remainder (22 bits) times a power of two that puts the
+// largest just below f16's maximum, as f16 has no bits below 2^-24 (FlScale).
+// A sum then keeps the bits of weights down to 2^-26 of its largest, below a
+// float32 sum's own rounding.  head_dim 64 is the exception: P and dS are one
+// 16-bit plane there, as on the kernels that share its calls.
 //
 // Operand layouts (lane = 16 g + c).  Row operand: lane (c, g) holds row c at
 // head_dim 32 j + 8 g .. +7 for each j (one 16-byte LDS read, or registers).
@@ -59,13 +63,26 @@ template <typename T>
 struct FlElt {
   using E = T;
   static constexpr int NP = 1;
-  static constexpr int NPB = 2;  // planes of a probability or dS operand
+  // planes of a probability or dS operand
+  static constexpr int NPB = __is_same(T, __bf16) ? 3 : 2;
 };
 template <>
 struct FlElt<float> {
   using E = __bf16;
   static constexpr int NP = 3;
   static constexpr int NPB = 3;
+};
+
+// Powers of two on f16's two-plane operands; other operands take none.
+template <typename T, int NPB>
+struct FlScale {
+  static constexpr bool kOn = __is_same(T, _Float16) && NPB == 2;
+  static constexpr float kFwd = kOn ? 7.0f : 0.0f;   // forward weights: up to 2^kSlack, so up to 2^15
+  static constexpr float kProb = kOn ? 15.0f : 0.0f; // normalised probabilities: up to 1
+  // the exponent that takes values up to x to [2^(top - 1), 2^top)
+  static __device__ __forceinline__ int exponent(float x, int top) {
+    return min(top - __builtin_amdgcn_frexp_expf(x), 100);
+  }
 };
 
 template <typename E>
@@ -436,6 +453,7 @@ template <typename T, int ND, int NQ, int NW, int KB, int NPB, bool DB, int OCC,
 __global__ __launch_bounds__(64 * NW, OCC) void flash_fwd_kernel(FlArgs a) {
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
   using St = FlStage<T, ND, KB, NW>;
+  using Sc = FlScale<T, NPB>;
   constexpr int RS = St::RS, PL = St::kPlane, MAT = St::kMat, BUF = 2 * MAT;
   constexpr int NU = KB / 16;
   const int tid = threadIdx.x;
@@ -562,8 +580,8 @@ __global__ __launch_bounds__(64 * NW, OCC) void flash_fwd_kernel(FlArgs a) {
           float p0[4], p1[4];
 #pragma unroll
           for (int r = 0; r < 4; ++r) {
-            p0[r] = __builtin_amdgcn_exp2f(fmaf(sc[u][n][r], sl2, -mu[n]));
-            p1[r] = __builtin_amdgcn_exp2f(fmaf(sc[u + 1][n][r], sl2, -mu[n]));
+            p0[r] = __builtin_amdgcn_exp2f(fmaf(sc[u][n][r], sl2, Sc::kFwd - mu[n]));
+            p1[r] = __builtin_amdgcn_exp2f(fmaf(sc[u + 1][n][r], sl2, Sc::kFwd - mu[n]));
             l_run[n] += p0[r] + p1[r];
           }
           pb[n].set(p0, p1);
@@ -598,7 +616,7 @@ __global__ __launch_bounds__(64 * NW, OCC) void flash_fwd_kernel(FlArgs a) {
     fl_store<T, ND>(acc[n], inv, Or, own_bad ? kOob : (uint32_t)i * tb, D, g);
     if (a.lse && g == 0 && i < Nr)
       a.lse[((int64_t)ps.b * a.N + ps.rho + (int64_t)a.dil * i) * a.H + ps.h] =
-          l_tot > 0.0f ? m_run[n] + __log2f(l_tot) : 0.0f;
+          l_tot > 0.0f ? m_run[n] + (__log2f(l_tot) - Sc::kFwd) : 0.0f;
     if (__builtin_expect(bad != 0, 0)) {
       for (int r = 0; r < 16; ++r)
         if (bad >> r & 0x0001000100010001ull) fl_fwd_row<T, (ND + 1) / 2>(a, ps, qa + 16 * n + r, lane);
@@ -627,6 +645,7 @@ template <typename T, int ND, int NQ, int NW, int KB, int NPB>
 __global__ __launch_bounds__(64 * NW, 2) void flash_pair_fwd_kernel(FlArgs a) {
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
   using St = FlStage<T, ND, KB, NW>;
+  using Sc = FlScale<T, NPB>;
   constexpr int RS = St::RS, PL = St::kPlane, MAT = St::kMat;
   constexpr int NU = KB / 16;
   const int tid = threadIdx.x;
@@ -729,8 +748,8 @@ __global__ __launch_bounds__(64 * NW, 2) void flash_pair_fwd_kernel(FlArgs a) {
         float p0[4], p1[4];
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          p0[r] = __builtin_amdgcn_exp2f(fmaf(sc[u][n][r], sl2, -mu[n]));
-          p1[r] = __builtin_amdgcn_exp2f(fmaf(sc[u + 1][n][r], sl2, -mu[n]));
+          p0[r] = __builtin_amdgcn_exp2f(fmaf(sc[u][n][r], sl2, Sc::kFwd - mu[n]));
+          p1[r] = __builtin_amdgcn_exp2f(fmaf(sc[u + 1][n][r], sl2, Sc::kFwd - mu[n]));
           l_run[n] += p0[r] + p1[r];
         }
         pb[u / 2][n].set(p0, p1);
@@ -805,7 +824,7 @@ __global__ __launch_bounds__(64 * NW, 2) void flash_pair_fwd_kernel(FlArgs a) {
     fl_store<T, ND>(acc[n], inv, Or, own_bad ? kOob : (uint32_t)i * tb, D, g);
     if (a.lse && g == 0 && i < Nr)
       a.lse[((int64_t)ps.b * a.N + ps.rho + (int64_t)a.dil * i) * a.H + ps.h] =
-          l_tot > 0.0f ? m_run[n] + __log2f(l_tot) : 0.0f;
+          l_tot > 0.0f ? m_run[n] + (__log2f(l_tot) - Sc::kFwd) : 0.0f;
     if (__builtin_expect(bad != 0, 0)) {
       for (int r = 0; r < 16; ++r)
         if (bad >> r & 0x0001000100010001ull) fl_fwd_row<T, (ND + 1) / 2>(a, ps, qa + 16 * n + r, lane);
@@ -916,6 +935,7 @@ template <typename T, int ND, int NQ, int NW, int KB, int NPB, int OCC, bool SAV
 __global__ __launch_bounds__(64 * NW, OCC) void flash_dq_kernel(FlArgs a) {
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
   using St = FlStage<T, ND, KB, NW>;
+  using Sc = FlScale<T, NPB>;
   constexpr int RS = St::RS, PL = St::kPlane, MAT = St::kMat;
   constexpr int NU = KB / 16;
   const int tid = threadIdx.x;
@@ -945,6 +965,7 @@ __global__ __launch_bounds__(64 * NW, OCC) void flash_dq_kernel(FlArgs a) {
   vs.load(Vr, k0 + block_at(0) * KB, tid, tb, D);
   FlFrag<T, ND> qf[NQ], gf[NQ];
   float m[NQ], l[NQ], dl[NQ];  // pass 1: maximum, sum, sum of e dp; then mu, 1/sum, delta
+  float top[NQ];  // f16: pass 1: largest |dp|; then the power of two on the row's dS, which is below 2 top
   const float sl2 = a.scale_log2;
 #pragma unroll
   for (int n = 0; n < NQ; ++n) {
@@ -952,7 +973,7 @@ __global__ __launch_bounds__(64 * NW, OCC) void flash_dq_kernel(FlArgs a) {
     qf[n].load(Qr, row, D, g);
     gf[n].load(Gr, row, D, g);
     m[n] = -INFINITY;
-    l[n] = dl[n] = 0.0f;
+    l[n] = dl[n] = top[n] = 0.0f;
     if constexpr (SAVED) {
       const __amdgpu_buffer_rsrc_t Fr = make_rsrc(static_cast<const T*>(a.fo) + ps.base, ps.nrec);
       FlFrag<T, ND> of;
@@ -1045,6 +1066,7 @@ __global__ __launch_bounds__(64 * NW, OCC) void flash_dq_kernel(FlArgs a) {
             const float p = __builtin_amdgcn_exp2f(fmaf(sc[n][r], sl2, -mu));
             l[n] += p;
             dl[n] = fmaf(p, dp[n][r], dl[n]);
+            if constexpr (Sc::kOn) top[n] = fmaxf(top[n], fabsf(dp[n][r]));
           }
         }
       }
@@ -1061,6 +1083,10 @@ __global__ __launch_bounds__(64 * NW, OCC) void flash_dq_kernel(FlArgs a) {
             *reinterpret_cast<f32x2*>(a.stats + 2 * row) = f32x2{lt != 0.0f ? mu + __log2f(lt) : 0.0f, dl[n]};
           }
           m[n] = mu;
+          if constexpr (Sc::kOn) {
+            top[n] = __builtin_amdgcn_ldexpf(1.0f, Sc::exponent(col_max(top[n]), 14));
+            l[n] *= top[n];
+          }
         }
       }
     } else {
@@ -1124,7 +1150,12 @@ __global__ __launch_bounds__(64 * NW, OCC) void flash_dq_kernel(FlArgs a) {
     }
     const uint64_t bad = __builtin_amdgcn_ballot_w64(i < Nr && fl_bad<ND>(acc[n]));
     const bool own_bad = (bad >> c & 0x0001000100010001ull) != 0;
-    fl_store<T, ND>(acc[n], a.scale, Or, own_bad ? kOob : (uint32_t)i * tb, D, g);
+    float f = a.scale;
+    if constexpr (Sc::kOn) {
+      f /= top[n];
+      l[n] /= top[n];
+    }
+    fl_store<T, ND>(acc[n], f, Or, own_bad ? kOob : (uint32_t)i * tb, D, g);
     if (__builtin_expect(bad != 0, 0)) {
       for (int r = 0; r < 16; ++r)
         if (bad >> r & 0x0001000100010001ull) {
@@ -1143,6 +1174,7 @@ template <typename T, int ND, int NK, int NW, int QB, int NPB, int OCC, bool FAS
 __global__ __launch_bounds__(64 * NW, OCC) void flash_dkv_kernel(FlArgs a) {
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
   using St = FlStage<T, ND, QB, NW>;
+  using Sc = FlScale<T, NPB>;
   constexpr int RS = St::RS, PL = St::kPlane, MAT = St::kMat;
   constexpr int NU = QB / 16;
   float* lst = reinterpret_cast<float*>(lds + 2 * MAT);  // QB lse2, then QB delta
@@ -1194,6 +1226,9 @@ __global__ __launch_bounds__(64 * NW, OCC) void flash_dkv_kernel(FlArgs a) {
   const uint32_t rl = (uint32_t)(c * RS + 16 * g), tl = fl_tr_lane<ND>(c, g);
   const float sl2 = a.scale_log2;
   f32x4 ak[NK][2 * ND], av[NK][2 * ND];
+  float sk[NK];  // f16: the power of two on the key's dS, lowered (and ak with it) when one would pass 2^15
+#pragma unroll
+  for (int n = 0; n < NK; ++n) sk[n] = 0x1p100f;
 #pragma unroll
   for (int n = 0; n < NK; ++n)
 #pragma unroll
@@ -1246,7 +1281,7 @@ __global__ __launch_bounds__(64 * NW, OCC) void flash_dkv_kernel(FlArgs a) {
               }
 #pragma unroll
               for (int r = 0; r < 4; ++r) {
-                p[n][w][r] = __builtin_amdgcn_exp2f(fmaf(sc[n][r], sl2, -ls[r]));
+                p[n][w][r] = __builtin_amdgcn_exp2f(fmaf(sc[n][r], sl2, Sc::kProb - ls[r]));
                 ds[n][w][r] = p[n][w][r] * (dp[n][r] - dt[r]);
               }
             }
@@ -1261,6 +1296,34 @@ __global__ __launch_bounds__(64 * NW, OCC) void flash_dkv_kernel(FlArgs a) {
 #pragma unroll
         for (int n = 0; n < NK; ++n) b[n].set(p[n][0], p[n][1]);
         fl_trmul<T, ND, PL, NK, NPB>(lds + MAT + u * 16 * RS + tl, lds + MAT + (u + 1) * 16 * RS + tl, b, av);
+        if constexpr (Sc::kOn) {
+          float mx[NK];
+          bool over = false;
+#pragma unroll
+          for (int n = 0; n < NK; ++n) {
+            mx[n] = 0.0f;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) mx[n] = fmaxf(mx[n], fmaxf(fabsf(ds[n][0][r]), fabsf(ds[n][1][r])));
+            over = over || mx[n] * sk[n] > 0x1p15f;
+          }
+          if (__builtin_amdgcn_ballot_w64(over) != 0) {
+#pragma unroll
+            for (int n = 0; n < NK; ++n) {
+              mx[n] = col_max(mx[n]);
+              const float s = mx[n] * sk[n] > 0x1p15f ? __builtin_amdgcn_ldexpf(1.0f, Sc::exponent(mx[n], 12)) : sk[n];
+              const float f = s / sk[n];
+#pragma unroll
+              for (int d = 0; d < 2 * ND; ++d) ak[n][d] *= f;
+              sk[n] = s;
+            }
+          }
+#pragma unroll
+          for (int n = 0; n < NK; ++n)
+#pragma unroll
+            for (int w = 0; w < 2; ++w)
+#pragma unroll
+              for (int r = 0; r < 4; ++r) ds[n][w][r] *= sk[n];
+        }
 #pragma unroll
         for (int n = 0; n < NK; ++n) b[n].set(ds[n][0], ds[n][1]);
         fl_trmul<T, ND, PL, NK, NPB>(lds + u * 16 * RS + tl, lds + (u + 1) * 16 * RS + tl, b, ak);
@@ -1288,8 +1351,9 @@ __global__ __launch_bounds__(64 * NW, OCC) void flash_dkv_kernel(FlArgs a) {
     const uint64_t bad = __builtin_amdgcn_ballot_w64(j < Nr && (fl_bad<ND>(ak[n]) || fl_bad<ND>(av[n])));
     const bool own_bad = (bad >> c & 0x0001000100010001ull) != 0;
     const uint32_t row = own_bad ? kOob : (uint32_t)j * tb;
-    fl_store<T, ND>(ak[n], a.scale, dKr, row, D, g);
-    fl_store<T, ND>(av[n], 1.0f, dVr, row, D, g);
+    constexpr float kUp = Sc::kOn ? 0x1p-15f : 1.0f;  // 2^-kProb
+    fl_store<T, ND>(ak[n], Sc::kOn ? a.scale * kUp / sk[n] : a.scale, dKr, row, D, g);
+    fl_store<T, ND>(av[n], kUp, dVr, row, D, g);
     if (__builtin_expect(bad != 0, 0)) {
       for (int r = 0; r < 16; ++r)
         if (bad >> r & 0x0001000100010001ull) fl_dkv_row<T, (ND + 1) / 2>(a, ps, ja + 16 * n + r, lane);

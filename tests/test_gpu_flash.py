@@ -271,3 +271,39 @@ def test_flash_float32_long_rows(ext, N, D):
         err = float((x[0, :, 0].cpu().double() - ref).norm() / ref.norm())
         print(f"  {name}: relative error {err:.2e}", flush=True)
         assert err <= 2.0 ** -19, name
+
+
+# N, head_dim, left, right (left None: every key), dO's size, rows of dO 2^10 times as large
+SMALL_GRADS = [(2048, 128, None, 0, 1e-3, None), (2048, 32, None, 0, 1e-3, None), (1500, 128, 600, 0, 1e-4, None),
+               (700, 40, 100, 100, 1e-3, slice(400, 410)), (1000, 8, None, 0, 1.0, None)]
+
+
+@pytest.mark.parametrize("N,D,left,right,size,loud", SMALL_GRADS)
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_flash_half_keeps_small_weights(ext, N, D, left, right, size, loud, dtype):
+    """16-bit calls at head_dims other than 64: the results of exact sums,
+    rounded once, also where dS and P lie under f16's smallest steps (output
+    gradients as an unscaled mean loss gives them, long rows).  A result is off
+    by the rounding to the type, e, and by its float32 sums' f: the norms add
+    in quadrature, and f up to 2^-18 of the result's norm moves the sum of
+    bf16's e (2^-9.6) or f16's (2^-12.6) by less than one part in 2000.  A sum
+    off by f of the elements' size lands on the other side of a rounding in
+    about f 2^7 1.15 ln(1/f) of bf16's elements (spacing 2^-7 of the power of
+    two below them, smaller elements more often): 1e-3 for the 5e-7 of sums of
+    this length, 2.5e-3 and more where weights keep 16 bits."""
+    q, k, v, g = (torch.from_numpy(a) for a in [*qkv((1, N, 1, D), 8970 + N), randn((1, N, 1, D), 8980 + N)])
+    g *= size
+    if loud is not None:
+        g[:, loud] *= 1024
+    q, k, v, g = (t.to(dtype).cuda() for t in (q, k, v, g))
+    if left is None:
+        got = [ext.dense_forward(q, k, v, False), *ext.dense_backward(q, k, v, g, False)]
+    else:
+        got = [ext.sliding_forward(q, k, v, left, right), *ext.sliding_backward(q, k, v, g, left, right)]
+    for name, x, ref in zip(("o", "dq", "dk", "dv"), got, _double(q, k, v, g, left, right)):
+        x = x[0, :, 0].cpu()
+        err, store = float((x.double() - ref).norm()), float((ref.to(dtype).double() - ref).norm())
+        flips = float((x != ref.to(dtype)).double().mean())
+        print(f"  {name}: error {err:.4e}, of storing alone {store:.4e}, rounded otherwise {flips:.2e}", flush=True)
+        assert err <= 1.0005 * store, name
+        assert dtype == torch.float16 or flips <= 1.5e-3, name
