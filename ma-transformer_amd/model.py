@@ -25,6 +25,7 @@ subclasses, tracing, autocast, tensor subclasses) keeps the layer calls.
 """
 from __future__ import annotations
 
+import functools
 import math
 
 import torch
@@ -151,14 +152,44 @@ def _plain(module: nn.Module, cls) -> bool:
             and not (module._forward_hooks or module._forward_pre_hooks))
 
 
-def _linear_params(lin: nn.Linear):
-    return lin._parameters.get("weight"), lin._parameters.get("bias")
+@functools.lru_cache(maxsize=16)
+def _model_shapes(D: int, inputs: int, layers: int) -> list:
+    block = [(D,), (D,), (4 * D, D), (4 * D,), (D, 4 * D), (D,), (D,), (D,)]
+    return [(D, inputs), (D,), (1, D), (1,)] + block * layers
+
+
+def _model_params(model: "TransformerModel"):
+    """The parameters encoder_model_forward reads (encoder, decoder, then each
+    layer's norm1, linear1, linear2, norm2; weight before bias) and the layers'
+    (window, eps), or None when the model holds anything but plain modules of
+    the shapes its constructor gives them: a replaced head, for instance."""
+    mods = model._modules
+    enc, pos, dec, layers = mods["encoder"], mods["pos_encoder"], mods["decoder"], mods["encoder_layers"]
+    D = model.model_dim
+    if D not in _FUSED_WIDTHS or not (_plain(enc, nn.Linear) and _plain(dec, nn.Linear)
+                                      and _plain(pos, PositionalEncoding)):
+        return None
+    pairs, windows = [enc._parameters, dec._parameters], []
+    for layer in layers._modules.values():
+        if not (_plain(layer, CustomTransformerEncoderLayer) and layer.fused):
+            return None
+        sub = layer._modules
+        attn, n1, n2 = sub["self_attn"], sub["norm1"], sub["norm2"]
+        if not (type(attn) is SparseAttention and attn.use_ma_core) or n1.eps != n2.eps:
+            return None
+        if layer.training and any(sub[n].p > 0 for n in ("dropout", "dropout1", "dropout2")):
+            return None
+        pairs += (n1._parameters, sub["linear1"]._parameters, sub["linear2"]._parameters, n2._parameters)
+        windows.append((int(attn.window_size), float(n1.eps)))
+    params = [p.get(n) for p in pairs for n in ("weight", "bias")]
+    shapes = [None if p is None else p.shape for p in params]
+    return (params, windows) if shapes == _model_shapes(D, enc.in_features, len(windows)) else None
 
 
 def _model_launch(model: "TransformerModel", src: torch.Tensor):
     """model(src) as one launch, or None when the call needs its modules:
-    gradients, training-mode dropout, other types, hooks, a width, depth or
-    length the kernel does not take."""
+    gradients, training-mode dropout, other types, hooks, a width, depth,
+    length or parameter shape the kernel does not take."""
     import torch.nn.modules.module as _m
     if type(src) is not torch.Tensor or not src.is_cuda or src.dtype != torch.float32 or src.dim() != 3:
         return None
@@ -166,52 +197,31 @@ def _model_launch(model: "TransformerModel", src: torch.Tensor):
             torch.jit.is_tracing() or torch.compiler.is_compiling() or torch._C._len_torch_dispatch_stack() or \
             torch._C._len_torch_function_stack() or torch._C._functorch.peek_interpreter_stack() is not None:
         return None
-    mods = model._modules
-    enc, pos, dec, layers = mods["encoder"], mods["pos_encoder"], mods["decoder"], mods["encoder_layers"]
-    D = model.model_dim
     B, S, I = src.shape
-    if D not in _FUSED_WIDTHS or B == 0 or S == 0 or not (_plain(enc, nn.Linear) and _plain(dec, nn.Linear)
-                                                         and _plain(pos, PositionalEncoding)):
+    found = _model_params(model) if B > 0 and S > 0 else None
+    if found is None:
         return None
-    blocks = list(layers._modules.values())
+    params, windows = found
+    D, pe = model.model_dim, model._modules["pos_encoder"]._buffers["pe"]
+    if pe.dtype != torch.float32 or pe.device != src.device or pe.shape[0] < B or pe.shape[1:] != (1, D) or \
+            not pe.is_contiguous() or pe.data_ptr() % 16:
+        return None
     grad = torch.is_grad_enabled()
-    params = [*_linear_params(enc), *_linear_params(dec)]
-    windows = []
-    for layer in blocks:
-        if not (_plain(layer, CustomTransformerEncoderLayer) and layer.fused):
-            return None
-        sub = layer._modules
-        attn = sub["self_attn"]
-        if not (type(attn) is SparseAttention and attn.use_ma_core):
-            return None
-        if layer.training and any(sub[n].p > 0 for n in ("dropout", "dropout1", "dropout2")):
-            return None
-        l1, l2, n1, n2 = sub["linear1"], sub["linear2"], sub["norm1"], sub["norm2"]
-        if (l1.in_features, l1.out_features) != (D, 4 * D) or n1.eps != n2.eps:
-            return None
-        for m in (n1, l1, l2, n2):
-            params += _linear_params(m)
-        windows.append((int(attn.window_size), float(n1.eps)))
-    pe = pos._buffers["pe"]
-    if pe.dtype != torch.float32 or pe.device != src.device or pe.shape[0] < B or not pe.is_contiguous() or \
-            pe.data_ptr() % 16:
-        return None
     ptrs = []
     for p in params:
-        if p is None or p.device != src.device or p.dtype != torch.float32 or not p.is_contiguous() or \
-                (grad and p.requires_grad):
+        if p.device != src.device or p.dtype != torch.float32 or not p.is_contiguous() or (grad and p.requires_grad):
             return None
         ptrs.append(p.data_ptr())
-    if (grad and src.requires_grad) or enc.in_features != I or any(p % 16 for p in ptrs[1:3] + ptrs[4:]):
+    if (grad and src.requires_grad) or params[0].shape[1] != I or any(p % 16 for p in ptrs[1:3] + ptrs[4:]):
         return None
     import ma_attn as _ma
-    if len(blocks) < 1 or len(blocks) > _ma.ENCODER_MAX_LAYERS or S > _ma.LIB.ma_encoder_model_max_seq(D):
+    if len(windows) < 1 or len(windows) > _ma.ENCODER_MAX_LAYERS or S > _ma.LIB.ma_encoder_model_max_seq(D):
         return None
     from sparse_attention_cuda import _on_device
-    descs = (_ma.EncoderLayer * len(blocks))()
+    descs = (_ma.EncoderLayer * len(windows))()
     for i, (w, eps) in enumerate(windows):
         descs[i] = _ma.EncoderLayer(B, S, D, 4 * D, w, eps, 0, *ptrs[4 + 8 * i:12 + 8 * i])
-    M = _ma.EncoderModel(B, S, I, D, len(blocks), descs, ptrs[0], ptrs[1], pe.data_ptr(), ptrs[2], ptrs[3])
+    M = _ma.EncoderModel(B, S, I, D, len(windows), descs, ptrs[0], ptrs[1], pe.data_ptr(), ptrs[2], ptrs[3])
     src = src.contiguous()
     out = torch.empty((B, 1), dtype=torch.float32, device=src.device)
     _on_device(src.get_device(),

@@ -248,3 +248,16 @@ def test_model_launch_leaves_observed_modules_alone(model_mod):
         assert take(m, src) is None
         m.eval()
     assert take(m, src) is None  # parameters record gradients
+
+
+def test_model_launch_leaves_replaced_heads_alone(model_mod):
+    """A decoder of three outputs gives all of them."""
+    m = model_mod.TransformerModel(5, 64, 2, 2, fused_layers=True).cuda().eval()
+    src = torch.randn(4, 10, 5, device="cuda")
+    with torch.no_grad():
+        m.decoder = torch.nn.Linear(64, 3).cuda()
+        assert model_mod._model_launch(m, src) is None
+        x = m.pos_encoder(m.encoder(src) * 8.0)
+        for layer in m.encoder_layers:
+            x = layer(x)
+        assert torch.equal(m(src), m.decoder(x[:, -1, :]))

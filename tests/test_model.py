@@ -48,3 +48,36 @@ def test_cpu_forward_matches_restatement(model_dim, num_layers):
         ref = _manual_forward(m, src)
     assert out.shape == (64, 1)
     torch.testing.assert_close(out, ref, rtol=1e-5, atol=1e-5)
+
+
+def _grown(lin):
+    lin.weight = torch.nn.Parameter(torch.zeros(lin.weight.shape[0], lin.weight.shape[1] + 1))
+
+
+@pytest.mark.parametrize("change", [
+    lambda m: setattr(m, "decoder", torch.nn.Linear(32, 3)),
+    lambda m: setattr(m, "decoder", torch.nn.Linear(16, 1)),
+    lambda m: setattr(m, "decoder", torch.nn.Linear(32, 1, bias=False)),
+    lambda m: setattr(m, "encoder", torch.nn.Linear(5, 16)),
+    lambda m: setattr(m.encoder_layers[1], "linear2", torch.nn.Linear(64, 32)),
+    lambda m: setattr(m.encoder_layers[1], "linear1", torch.nn.Linear(32, 64)),
+    lambda m: setattr(m.encoder_layers[0], "norm2", torch.nn.LayerNorm(16)),
+    lambda m: setattr(m.encoder_layers[0], "norm1", torch.nn.LayerNorm((1, 32))),
+    lambda m: _grown(m.encoder),
+    lambda m: _grown(m.encoder_layers[0].linear2),
+], ids=["head3", "head16", "no_bias", "encoder16", "linear2", "linear1", "norm2", "norm1_2d", "encoder_in", "ff_in"])
+def test_one_launch_needs_the_constructors_shapes(change):
+    """The one-launch model takes pointers only, so a model whose modules were
+    replaced by ones of other shapes keeps its modules' own forward."""
+    from model import TransformerModel, _model_params
+    m = TransformerModel(input_dim=5, model_dim=32, num_heads=2, num_layers=2, fused_layers=True).eval()
+    params, windows = _model_params(m)
+    assert len(params) == 4 + 8 * 2 and windows == [(3, 1e-5)] * 2
+    src = torch.randn(3, 10, 5)
+    with torch.no_grad():
+        assert m(src).shape == (3, 1)
+        change(m)
+        if m.decoder.out_features == 3:
+            assert m(src).shape == (3, 3)
+    found = _model_params(m)  # the encoder's input width is compared with the call's
+    assert found is None or found[0][0].shape[1] != src.shape[2]
