@@ -31,6 +31,7 @@ import math
 import torch
 import torch.nn as nn
 import torch.nn.functional as F
+import torch.nn.modules.module as _module
 
 from layers.sparse_attention import SparseAttention
 
@@ -186,16 +187,25 @@ def _model_params(model: "TransformerModel"):
     return (params, windows) if shapes == _model_shapes(D, enc.in_features, len(windows)) else None
 
 
+def _observed() -> bool:
+    """Whether something would see the operations inside a call: global hooks,
+    autocast, tracing, torch modes or function transforms.  A torch that lacks
+    one of the (partly private) names asked here counts as observing."""
+    try:
+        return bool(_module._global_forward_hooks or _module._global_forward_pre_hooks
+                    or torch.is_autocast_enabled("cuda") or torch.jit.is_tracing() or torch.compiler.is_compiling()
+                    or torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack()
+                    or torch._C._functorch.peek_interpreter_stack() is not None)
+    except (AttributeError, TypeError):
+        return True
+
+
 def _model_launch(model: "TransformerModel", src: torch.Tensor):
     """model(src) as one launch, or None when the call needs its modules:
     gradients, training-mode dropout, other types, hooks, a width, depth,
     length or parameter shape the kernel does not take."""
-    import torch.nn.modules.module as _m
-    if type(src) is not torch.Tensor or not src.is_cuda or src.dtype != torch.float32 or src.dim() != 3:
-        return None
-    if _m._global_forward_hooks or _m._global_forward_pre_hooks or torch.is_autocast_enabled("cuda") or \
-            torch.jit.is_tracing() or torch.compiler.is_compiling() or torch._C._len_torch_dispatch_stack() or \
-            torch._C._len_torch_function_stack() or torch._C._functorch.peek_interpreter_stack() is not None:
+    if type(src) is not torch.Tensor or not src.is_cuda or src.dtype != torch.float32 or src.dim() != 3 or \
+            _observed():
         return None
     B, S, I = src.shape
     found = _model_params(model) if B > 0 and S > 0 else None

@@ -81,3 +81,15 @@ def test_one_launch_needs_the_constructors_shapes(change):
             assert m(src).shape == (3, 3)
     found = _model_params(m)  # the encoder's input width is compared with the call's
     assert found is None or found[0][0].shape[1] != src.shape[2]
+
+
+@pytest.mark.parametrize("where,name", [(torch._C, "_len_torch_dispatch_stack"), (torch._C, "_len_torch_function_stack"),
+                                        (torch._C._functorch, "peek_interpreter_stack"),
+                                        (torch.nn.modules.module, "_global_forward_pre_hooks")])
+def test_one_launch_stays_off_without_a_private_name(monkeypatch, where, name):
+    """The one-launch model asks torch, partly by private names, whether
+    anything observes the call; a torch without one of them keeps the modules."""
+    from model import _observed
+    assert _observed() is False
+    monkeypatch.delattr(where, name)
+    assert _observed() is True
