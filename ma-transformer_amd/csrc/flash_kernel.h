@@ -79,6 +79,9 @@ struct FlScale {
   static constexpr bool kOn = __is_same(T, _Float16) && NPB == 2;
   static constexpr float kFwd = kOn ? 7.0f : 0.0f;   // forward weights: up to 2^kSlack, so up to 2^15
   static constexpr float kProb = kOn ? 15.0f : 0.0f; // normalised probabilities: up to 1
+  // exponents' offsets of a weight (mu: the row's maximum) and of a probability
+  static __device__ __forceinline__ float fwd(float mu) { return kOn ? kFwd - mu : -mu; }
+  static __device__ __forceinline__ float prob(float lse2) { return kOn ? kProb - lse2 : -lse2; }
   // the exponent that takes values up to x to [2^(top - 1), 2^top)
   static __device__ __forceinline__ int exponent(float x, int top) {
     return min(top - __builtin_amdgcn_frexp_expf(x), 100);
@@ -580,8 +583,8 @@ __global__ __launch_bounds__(64 * NW, OCC) void flash_fwd_kernel(FlArgs a) {
           float p0[4], p1[4];
 #pragma unroll
           for (int r = 0; r < 4; ++r) {
-            p0[r] = __builtin_amdgcn_exp2f(fmaf(sc[u][n][r], sl2, Sc::kFwd - mu[n]));
-            p1[r] = __builtin_amdgcn_exp2f(fmaf(sc[u + 1][n][r], sl2, Sc::kFwd - mu[n]));
+            p0[r] = __builtin_amdgcn_exp2f(fmaf(sc[u][n][r], sl2, Sc::fwd(mu[n])));
+            p1[r] = __builtin_amdgcn_exp2f(fmaf(sc[u + 1][n][r], sl2, Sc::fwd(mu[n])));
             l_run[n] += p0[r] + p1[r];
           }
           pb[n].set(p0, p1);
@@ -748,8 +751,8 @@ __global__ __launch_bounds__(64 * NW, 2) void flash_pair_fwd_kernel(FlArgs a) {
         float p0[4], p1[4];
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          p0[r] = __builtin_amdgcn_exp2f(fmaf(sc[u][n][r], sl2, Sc::kFwd - mu[n]));
-          p1[r] = __builtin_amdgcn_exp2f(fmaf(sc[u + 1][n][r], sl2, Sc::kFwd - mu[n]));
+          p0[r] = __builtin_amdgcn_exp2f(fmaf(sc[u][n][r], sl2, Sc::fwd(mu[n])));
+          p1[r] = __builtin_amdgcn_exp2f(fmaf(sc[u + 1][n][r], sl2, Sc::fwd(mu[n])));
           l_run[n] += p0[r] + p1[r];
         }
         pb[u / 2][n].set(p0, p1);
@@ -1281,7 +1284,7 @@ __global__ __launch_bounds__(64 * NW, OCC) void flash_dkv_kernel(FlArgs a) {
               }
 #pragma unroll
               for (int r = 0; r < 4; ++r) {
-                p[n][w][r] = __builtin_amdgcn_exp2f(fmaf(sc[n][r], sl2, Sc::kProb - ls[r]));
+                p[n][w][r] = __builtin_amdgcn_exp2f(fmaf(sc[n][r], sl2, Sc::prob(ls[r])));
                 ds[n][w][r] = p[n][w][r] * (dp[n][r] - dt[r]);
               }
             }
