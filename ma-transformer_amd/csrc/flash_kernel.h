@@ -383,16 +383,74 @@ __device__ __forceinline__ bool fl_rows(const FlPos& ps, int wv, FlRows& r) {
   }
 }
 
-__device__ __forceinline__ float fl_wave_sum(float x) {
+// ---------------------------------------------------------------- rows redone
+//
+// The weight of a masked pair is 0, but 0 times an infinity or NaN in its row
+// of V (K, Q, dO) is NaN and reaches sums that do not hold that pair; likewise
+// an infinity times an operand's negative remainder plane.  A group of 16 rows
+// with such sums is computed again in float32 over each row's own set: lane
+// (c, g) holds row c at head_dim 32 h + 8 g .. +7 for each h, as the sums do,
+// and walks the group's keys (queries).  Rows that are NaN throughout in either
+// computation keep their sums: those whose statistics are NaN, and keys of such
+// queries (fl_dkv_nan).
+//
+// Bound by the VALU's products (two of head_dim 64 for a pair of the forward, four
+// for the backward's dK and dV), after the clean call's own time.  Causal, 8 heads
+// of 8192 rows, clean call / every row redone (an infinite first V row; infinite
+// output gradients): float32 at head_dim 64 0.51 / 5.9 and 1.5 / 5.9 ms, f16 at
+// head_dim 128 0.27 / 6.0 and 1.1 / 7.5 ms.  One row and key at a time took 14 to
+// 46 ms for 2048 rows; 16 rows at once take 0.6 to 1.8.
+template <typename T, int ND>
+struct FlRow {
+  float x[8 * ND];
+  __device__ __forceinline__ void load(__amdgpu_buffer_rsrc_t rs, uint32_t row, int D, int g) {
 #pragma unroll
-  for (int m = 32; m >= 1; m >>= 1) x += __shfl_xor(x, m, 64);
-  return x;
-}
-
-template <typename T>
-__device__ __forceinline__ float fl_at(const T* p, int64_t row, int64_t rs, int d, int D) {
-  return d < D ? static_cast<float>(p[row * rs + d]) : 0.0f;
-}
+    for (int h = 0; h < ND; ++h) {
+      const int d = 32 * h + 8 * g;
+      const uint32_t off = d < D ? row + (uint32_t)(d * sizeof(T)) : kOob;
+      const uint4 a = bload16(rs, off);
+      const uint32_t w[4] = {a.x, a.y, a.z, a.w};
+      if constexpr (sizeof(T) == 4) {
+        const uint4 b = bload16(rs, off + 16);
+        const uint32_t y[4] = {b.x, b.y, b.z, b.w};
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          x[8 * h + i] = __uint_as_float(w[i]);
+          x[8 * h + 4 + i] = __uint_as_float(y[i]);
+        }
+      } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          x[8 * h + 2 * i] = fl_lo<T>(w[i]);
+          x[8 * h + 2 * i + 1] = fl_hi<T>(w[i]);
+        }
+      }
+    }
+  }
+  __device__ __forceinline__ float dot(const FlRow& o) const {
+    float s = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 8 * ND; ++i) s = fmaf(x[i], o.x[i], s);
+    return col_sum(s);
+  }
+  __device__ __forceinline__ void add(float f, const FlRow& o) {
+#pragma unroll
+    for (int i = 0; i < 8 * ND; ++i) x[i] = fmaf(f, o.x[i], x[i]);
+  }
+  __device__ __forceinline__ void zero() {
+#pragma unroll
+    for (int i = 0; i < 8 * ND; ++i) x[i] = 0.0f;
+  }
+  __device__ __forceinline__ void scale(float f) {
+#pragma unroll
+    for (int i = 0; i < 8 * ND; ++i) x[i] *= f;
+  }
+  // as a product's accumulator, for fl_store
+  __device__ __forceinline__ void sums(f32x4 (&acc)[2 * ND]) const {
+#pragma unroll
+    for (int i = 0; i < 2 * ND; ++i) acc[i] = f32x4{x[4 * i], x[4 * i + 1], x[4 * i + 2], x[4 * i + 3]};
+  }
+};
 
 // ---------------------------------------------------------------- forward
 //
@@ -407,43 +465,50 @@ __device__ __forceinline__ float fl_at(const T* p, int64_t row, int64_t rs, int 
 // rounding error, once per key block).  16-key sub-tiles outside every window of the
 // wave are skipped.
 //
-// A row whose sums come out infinite or NaN is computed again key by key
-// (fl_fwd_row): a masked key's probability is 0, but 0 times an infinity or
-// NaN in its V row would reach queries that do not attend it.
-template <typename T, int NC>
-__device__ __forceinline__ void fl_fwd_row(const FlArgs& a, const FlPos& ps, int i, int lane) {
-  const int64_t rs = (int64_t)a.dil * a.H * a.D;
-  const T* q = static_cast<const T*>(a.q) + ps.base;
-  const T* k = static_cast<const T*>(a.k) + ps.base;
-  const T* v = static_cast<const T*>(a.v) + ps.base;
-  T* o = static_cast<T*>(a.o) + ps.base;
-  float qd[NC], acc[NC];
+// Rows of the group r0 .. r0 + 15 (lane's own: r0 + c) over their own keys:
+// unnormalised sums and the weights' total.
+template <typename T, int ND, bool GL>
+__device__ __forceinline__ void fl_fwd_rows(const FlArgs& a, const FlPos& ps, __amdgpu_buffer_rsrc_t Qr,
+                                            __amdgpu_buffer_rsrc_t Kr, __amdgpu_buffer_rsrc_t Vr, int r0, int c, int g,
+                                            f32x4 (&sums)[2 * ND], float& l) {
+  constexpr int U = ND == 1 ? 4 : ND == 2 ? 2 : 1;
+  const uint32_t tb = a.tok_bytes;
+  const int i = r0 + c, lo = max(0, r0 - a.left), hi = min(ps.Nr, r0 + 16 + a.right);
+  const int ng = GL ? min(a.globals, lo) : 0;
+  FlRow<T, ND> q, acc;
+  q.load(Qr, (uint32_t)i * tb, a.D, g);
+  acc.zero();
+  float m = -INFINITY;
+  l = 0.0f;
+  for (int e = 0; e < ng + hi - lo; e += U) {
+    FlRow<T, ND> k[U], v[U];
+    float s[U], mn = m;
+    bool in[U];
 #pragma unroll
-  for (int c = 0; c < NC; ++c) {
-    qd[c] = fl_at(q, i, rs, lane + 64 * c, a.D);
-    acc[c] = 0.0f;
-  }
-  float m = -INFINITY, l = 0.0f;
-  const int j0 = max(0, i - a.left), j1 = min(ps.Nr - 1, i + a.right);
-  const int ng = min(j0, a.globals);
-  for (int e = j0 - ng; e <= j1; ++e) {
-    const int j = e < j0 ? e - (j0 - ng) : e;
-    float s = 0.0f;
+    for (int u = 0; u < U; ++u) {
+      const int j = e + u < ng ? e + u : lo + e + u - ng;  // past hi: in range of the buffer or zeros, and masked
+      k[u].load(Kr, (uint32_t)j * tb, a.D, g);
+      v[u].load(Vr, (uint32_t)j * tb, a.D, g);
+      in[u] = j < hi && j <= i + a.right && (j >= i - a.left || (GL && j < a.globals));
+    }
 #pragma unroll
-    for (int c = 0; c < NC; ++c) s = fmaf(qd[c], fl_at(k, j, rs, lane + 64 * c, a.D), s);
-    s = fl_wave_sum(s) * a.scale;
-    const float mn = fmaxf(m, s);
-    const float mu = mn == -INFINITY ? 0.0f : mn;
-    const float corr = expf(m - mu), p = expf(s - mu);
-    l = fmaf(l, corr, p);
+    for (int u = 0; u < U; ++u) {
+      s[u] = q.dot(k[u]) * a.scale_log2;
+      s[u] = in[u] ? s[u] : -INFINITY;
+      mn = fmaxf(mn, s[u]);
+    }
+    const float mu = mn == -INFINITY ? 0.0f : mn, corr = __builtin_amdgcn_exp2f(m - mu);
+    l *= corr;
+    acc.scale(corr);
 #pragma unroll
-    for (int c = 0; c < NC; ++c) acc[c] = fmaf(p, fl_at(v, j, rs, lane + 64 * c, a.D), acc[c] * corr);
+    for (int u = 0; u < U; ++u) {
+      const float p = __builtin_amdgcn_exp2f(s[u] - mu);
+      l += p;
+      if (in[u]) acc.add(p, v[u]);
+    }
     m = mn;
   }
-  const float inv = l != 0.0f ? 1.0f / l : 0.0f;
-#pragma unroll
-  for (int c = 0; c < NC; ++c)
-    if (lane + 64 * c < a.D) o[i * rs + lane + 64 * c] = static_cast<T>(acc[c] * inv);
+  acc.sums(sums);
 }
 
 constexpr float kSlack = 8.0f;
@@ -613,16 +678,17 @@ __global__ __launch_bounds__(64 * NW, OCC) void flash_fwd_kernel(FlArgs a) {
     const float l_tot = col_sum(l_run[n]);
     const float inv = l_tot != 0.0f ? 1.0f / l_tot : 0.0f;
     const int i = qa + 16 * n + c;
-    // bit r of each lane group: row r is left to fl_fwd_row
-    const uint64_t bad = __builtin_amdgcn_ballot_w64(i < Nr && !(GL && i < a.globals) && (fl_bad<ND>(acc[n]) || !(l_tot < INFINITY)));
-    const bool own_bad = (bad >> c & 0x0001000100010001ull) != 0 || (GL && i < a.globals);
-    fl_store<T, ND>(acc[n], inv, Or, own_bad ? kOob : (uint32_t)i * tb, D, g);
+    const bool mine = !(GL && i < a.globals);
+    const uint64_t bad = __builtin_amdgcn_ballot_w64(i < Nr && mine && fl_bad<ND>(acc[n]) && l_tot < INFINITY);
+    const bool own_bad = (bad >> c & 0x0001000100010001ull) != 0;  // in some lane of the row
+    fl_store<T, ND>(acc[n], inv, Or, own_bad || !mine ? kOob : (uint32_t)i * tb, D, g);
     if (a.lse && g == 0 && i < Nr)
       a.lse[((int64_t)ps.b * a.N + ps.rho + (int64_t)a.dil * i) * a.H + ps.h] =
           l_tot > 0.0f ? m_run[n] + (__log2f(l_tot) - Sc::kFwd) : 0.0f;
     if (__builtin_expect(bad != 0, 0)) {
-      for (int r = 0; r < 16; ++r)
-        if (bad >> r & 0x0001000100010001ull) fl_fwd_row<T, (ND + 1) / 2>(a, ps, qa + 16 * n + r, lane);
+      float l;
+      fl_fwd_rows<T, ND, GL>(a, ps, Qr, Kr, Vr, qa + 16 * n, c, g, acc[n], l);
+      fl_store<T, ND>(acc[n], l != 0.0f ? 1.0f / l : 0.0f, Or, own_bad ? (uint32_t)i * tb : kOob, D, g);
     }
   }
 }
@@ -822,15 +888,16 @@ __global__ __launch_bounds__(64 * NW, 2) void flash_pair_fwd_kernel(FlArgs a) {
     const float l_tot = col_sum(l_run[n]);
     const float inv = l_tot != 0.0f ? 1.0f / l_tot : 0.0f;
     const int i = qa + 16 * n + c;
-    const uint64_t bad = __builtin_amdgcn_ballot_w64(i < Nr && (fl_bad<ND>(acc[n]) || !(l_tot < INFINITY)));
+    const uint64_t bad = __builtin_amdgcn_ballot_w64(i < Nr && fl_bad<ND>(acc[n]) && l_tot < INFINITY);
     const bool own_bad = (bad >> c & 0x0001000100010001ull) != 0;
     fl_store<T, ND>(acc[n], inv, Or, own_bad ? kOob : (uint32_t)i * tb, D, g);
     if (a.lse && g == 0 && i < Nr)
       a.lse[((int64_t)ps.b * a.N + ps.rho + (int64_t)a.dil * i) * a.H + ps.h] =
           l_tot > 0.0f ? m_run[n] + (__log2f(l_tot) - Sc::kFwd) : 0.0f;
     if (__builtin_expect(bad != 0, 0)) {
-      for (int r = 0; r < 16; ++r)
-        if (bad >> r & 0x0001000100010001ull) fl_fwd_row<T, (ND + 1) / 2>(a, ps, qa + 16 * n + r, lane);
+      float l;
+      fl_fwd_rows<T, ND, false>(a, ps, Qr, Kr, Vr, qa + 16 * n, c, g, acc[n], l);
+      fl_store<T, ND>(acc[n], l != 0.0f ? 1.0f / l : 0.0f, Or, own_bad ? (uint32_t)i * tb : kOob, D, g);
     }
   }
 }
@@ -843,85 +910,100 @@ __global__ __launch_bounds__(64 * NW, 2) void flash_pair_fwd_kernel(FlArgs a) {
 // dQ_i = scale sum_j ds_ij K_j, dK_j = scale sum_i ds_ij Q_i,
 // dV_j = sum_i p_ij dO_i.  Each output row has one writer.
 //
-// As in the forward, a row whose sums come out infinite or NaN is computed
-// again over its own set alone.
-template <typename T, int NC>
-__device__ __forceinline__ void fl_dq_row(const FlArgs& a, const FlPos& ps, int i, float lse2, float dlt, int lane) {
-  const int64_t rs = (int64_t)a.dil * a.H * a.D;
-  const T* q = static_cast<const T*>(a.q) + ps.base;
-  const T* k = static_cast<const T*>(a.k) + ps.base;
-  const T* v = static_cast<const T*>(a.v) + ps.base;
-  const T* go = static_cast<const T*>(a.dout) + ps.base;
-  T* dq = static_cast<T*>(a.o) + ps.base;
-  float qd[NC], gd[NC], acc[NC];
+// Sums of dQ's rows r0 .. r0 + 15 over their own keys: p = 2^(s - mu) inv,
+// with the row's delta dlt.
+template <typename T, int ND>
+__device__ __forceinline__ void fl_dq_rows(const FlArgs& a, const FlPos& ps, __amdgpu_buffer_rsrc_t Qr,
+                                           __amdgpu_buffer_rsrc_t Gr, __amdgpu_buffer_rsrc_t Kr,
+                                           __amdgpu_buffer_rsrc_t Vr, int r0, int c, int g, float mu, float inv,
+                                           float dlt, f32x4 (&sums)[2 * ND]) {
+  constexpr int U = ND == 1 ? 2 : 1;
+  const uint32_t tb = a.tok_bytes;
+  const int i = r0 + c, lo = max(0, r0 - a.left), hi = min(ps.Nr, r0 + 16 + a.right);
+  FlRow<T, ND> q, go, acc;
+  q.load(Qr, (uint32_t)i * tb, a.D, g);
+  go.load(Gr, (uint32_t)i * tb, a.D, g);
+  acc.zero();
+  for (int e = lo; e < hi; e += U) {
+    FlRow<T, ND> k[U], v[U];
 #pragma unroll
-  for (int c = 0; c < NC; ++c) {
-    qd[c] = fl_at(q, i, rs, lane + 64 * c, a.D);
-    gd[c] = fl_at(go, i, rs, lane + 64 * c, a.D);
-    acc[c] = 0.0f;
-  }
-  const int j0 = max(0, i - a.left), j1 = min(ps.Nr - 1, i + a.right);
-  for (int j = j0; j <= j1; ++j) {
-    float s = 0.0f, dp = 0.0f;
-#pragma unroll
-    for (int c = 0; c < NC; ++c) {
-      s = fmaf(qd[c], fl_at(k, j, rs, lane + 64 * c, a.D), s);
-      dp = fmaf(gd[c], fl_at(v, j, rs, lane + 64 * c, a.D), dp);
+    for (int u = 0; u < U; ++u) {
+      k[u].load(Kr, (uint32_t)(e + u) * tb, a.D, g);
+      v[u].load(Vr, (uint32_t)(e + u) * tb, a.D, g);
     }
-    s = fl_wave_sum(s);
-    dp = fl_wave_sum(dp);
-    const float ds = __builtin_amdgcn_exp2f(fmaf(s, a.scale_log2, -lse2)) * (dp - dlt);
 #pragma unroll
-    for (int c = 0; c < NC; ++c) acc[c] = fmaf(ds, fl_at(k, j, rs, lane + 64 * c, a.D), acc[c]);
+    for (int u = 0; u < U; ++u) {
+      const float s = q.dot(k[u]), dp = go.dot(v[u]);
+      const float ds = __builtin_amdgcn_exp2f(fmaf(s, a.scale_log2, -mu)) * inv * (dp - dlt);
+      if (e + u < hi && e + u >= i - a.left && e + u <= i + a.right) acc.add(ds, k[u]);
+    }
   }
-#pragma unroll
-  for (int c = 0; c < NC; ++c)
-    if (lane + 64 * c < a.D) dq[i * rs + lane + 64 * c] = static_cast<T>(acc[c] * a.scale);
+  acc.sums(sums);
 }
 
-template <typename T, int NC>
-__device__ __forceinline__ void fl_dkv_row(const FlArgs& a, const FlPos& ps, int j, int lane) {
-  const int64_t rs = (int64_t)a.dil * a.H * a.D;
-  const T* q = static_cast<const T*>(a.q) + ps.base;
-  const T* k = static_cast<const T*>(a.k) + ps.base;
-  const T* v = static_cast<const T*>(a.v) + ps.base;
-  const T* go = static_cast<const T*>(a.dout) + ps.base;
-  float kd[NC], vd[NC], dk[NC], dv[NC];
+// Sums of dK's and dV's rows r0 .. r0 + 15 over their own queries.
+template <typename T, int ND>
+__device__ __forceinline__ void fl_dkv_rows(const FlArgs& a, const FlPos& ps, __amdgpu_buffer_rsrc_t Qr,
+                                            __amdgpu_buffer_rsrc_t Gr, __amdgpu_buffer_rsrc_t Kr,
+                                            __amdgpu_buffer_rsrc_t Vr, int r0, int c, int g, f32x4 (&sk)[2 * ND],
+                                            f32x4 (&sv)[2 * ND]) {
+  constexpr int U = ND == 1 ? 2 : 1;
+  const uint32_t tb = a.tok_bytes;
+  const int j = r0 + c, lo = max(0, r0 - a.right), hi = min(ps.Nr, r0 + 16 + a.left);
+  FlRow<T, ND> k, v, dk, dv;
+  k.load(Kr, (uint32_t)j * tb, a.D, g);
+  v.load(Vr, (uint32_t)j * tb, a.D, g);
+  dk.zero();
+  dv.zero();
+  for (int e = lo; e < hi; e += U) {
+    FlRow<T, ND> q[U], go[U];
+    f32x2 st[U];
 #pragma unroll
-  for (int c = 0; c < NC; ++c) {
-    kd[c] = fl_at(k, j, rs, lane + 64 * c, a.D);
-    vd[c] = fl_at(v, j, rs, lane + 64 * c, a.D);
-    dk[c] = dv[c] = 0.0f;
+    for (int u = 0; u < U; ++u) {
+      q[u].load(Qr, (uint32_t)(e + u) * tb, a.D, g);
+      go[u].load(Gr, (uint32_t)(e + u) * tb, a.D, g);
+      const int64_t row = ((int64_t)ps.b * a.N + ps.rho + (int64_t)a.dil * min(e + u, hi - 1)) * a.H + ps.h;
+      st[u] = *reinterpret_cast<const f32x2*>(a.stats + 2 * row);
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const float s = k.dot(q[u]), dp = v.dot(go[u]);
+      const float p = __builtin_amdgcn_exp2f(fmaf(s, a.scale_log2, -st[u][0]));
+      if (e + u < hi && e + u >= j - a.right && e + u <= j + a.left) {
+        dv.add(p, go[u]);
+        dk.add(p * (dp - st[u][1]), q[u]);
+      }
+    }
   }
-  const int i0 = max(0, j - a.right), i1 = min(ps.Nr - 1, j + a.left);
-  for (int i = i0; i <= i1; ++i) {
+  dk.sums(sk);
+  dv.sums(sv);
+}
+
+// Whether the sums of dK and dV stand for the keys r0 .. r0 + 15: each has, in
+// its query set, a query whose statistics are NaN, or whose delta and whole dO
+// row are (dK and dV all NaN in either computation), or whose delta is NaN where
+// dV's sums are finite (v_ok; dK all NaN).
+template <typename T, int ND>
+__device__ __forceinline__ bool fl_dkv_nan(const FlArgs& a, const FlPos& ps, __amdgpu_buffer_rsrc_t Gr, int r0, int lane,
+                                           bool v_ok) {
+  bool nan_l = false;
+  int w = -1;
+  for (int i = max(0, r0 + 15 - a.right) + lane; i <= min(ps.Nr - 1, r0 + a.left); i += 64) {
     const int64_t row = ((int64_t)ps.b * a.N + ps.rho + (int64_t)a.dil * i) * a.H + ps.h;
-    float s = 0.0f, dp = 0.0f, qd[NC], gd[NC];
-#pragma unroll
-    for (int c = 0; c < NC; ++c) {
-      qd[c] = fl_at(q, i, rs, lane + 64 * c, a.D);
-      gd[c] = fl_at(go, i, rs, lane + 64 * c, a.D);
-      s = fmaf(qd[c], kd[c], s);
-      dp = fmaf(gd[c], vd[c], dp);
-    }
-    s = fl_wave_sum(s);
-    dp = fl_wave_sum(dp);
-    const float p = __builtin_amdgcn_exp2f(fmaf(s, a.scale_log2, -a.stats[2 * row]));
-    const float ds = p * (dp - a.stats[2 * row + 1]);
-#pragma unroll
-    for (int c = 0; c < NC; ++c) {
-      dv[c] = fmaf(p, gd[c], dv[c]);
-      dk[c] = fmaf(ds, qd[c], dk[c]);
-    }
+    const f32x2 st = *reinterpret_cast<const f32x2*>(a.stats + 2 * row);
+    nan_l = nan_l || st[0] != st[0];
+    w = st[1] != st[1] ? i : w;
   }
-  T* ok = static_cast<T*>(a.dk) + ps.base;
-  T* ov = static_cast<T*>(a.dv) + ps.base;
+  if (__builtin_amdgcn_ballot_w64(nan_l) != 0) return true;
+  const uint64_t found = __builtin_amdgcn_ballot_w64(w >= 0);
+  if (found == 0 || v_ok) return found != 0;
+  FlRow<T, ND> go;
+  go.load(Gr, (uint32_t)__shfl(w, __builtin_ctzll(found), 64) * a.tok_bytes, a.D, lane >> 4);
+  bool all = true;
 #pragma unroll
-  for (int c = 0; c < NC; ++c)
-    if (lane + 64 * c < a.D) {
-      ok[j * rs + lane + 64 * c] = static_cast<T>(dk[c] * a.scale);
-      ov[j * rs + lane + 64 * c] = static_cast<T>(dv[c]);
-    }
+  for (int i = 0; i < 8 * ND; ++i)
+    all = all && (go.x[i] != go.x[i] || 32 * (i >> 3) + 8 * (lane >> 4) >= a.D);
+  return __builtin_amdgcn_ballot_w64(!all) == 0;
 }
 
 template <bool B>
@@ -1151,20 +1233,17 @@ __global__ __launch_bounds__(64 * NW, OCC) void flash_dq_kernel(FlArgs a) {
         *reinterpret_cast<f32x2*>(a.stats + 2 * row) = f32x2{m[n], dl[n]};
       }
     }
-    const uint64_t bad = __builtin_amdgcn_ballot_w64(i < Nr && fl_bad<ND>(acc[n]));
-    const bool own_bad = (bad >> c & 0x0001000100010001ull) != 0;
     float f = a.scale;
     if constexpr (Sc::kOn) {
       f /= top[n];
       l[n] /= top[n];
     }
+    const uint64_t bad = __builtin_amdgcn_ballot_w64(i < Nr && fl_bad<ND>(acc[n]) && l[n] == l[n] && dl[n] == dl[n]);
+    const bool own_bad = (bad >> c & 0x0001000100010001ull) != 0;  // in some lane of the row
     fl_store<T, ND>(acc[n], f, Or, own_bad ? kOob : (uint32_t)i * tb, D, g);
     if (__builtin_expect(bad != 0, 0)) {
-      for (int r = 0; r < 16; ++r)
-        if (bad >> r & 0x0001000100010001ull) {
-          const float mu = __shfl(m[n], r, 64), inv = __shfl(l[n], r, 64), dd = __shfl(dl[n], r, 64);
-          fl_dq_row<T, (ND + 1) / 2>(a, ps, qa + 16 * n + r, mu - __log2f(inv), dd, lane);
-        }
+      fl_dq_rows<T, ND>(a, ps, Qr, Gr, Kr, Vr, qa + 16 * n, c, g, m[n], l[n], dl[n], acc[n]);
+      fl_store<T, ND>(acc[n], a.scale, Or, own_bad ? (uint32_t)i * tb : kOob, D, g);
     }
   }
 }
@@ -1348,18 +1427,23 @@ __global__ __launch_bounds__(64 * NW, OCC) void flash_dkv_kernel(FlArgs a) {
   }
 
   if (ja >= Nr) return;  // no barrier below
+  // the lane's numbers again: held over the loop they would spill at head_dims above 64
+  const int el = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)), ec = el & 15, eg = el >> 4;
 #pragma unroll
   for (int n = 0; n < NK; ++n) {
-    const int j = ja + 16 * n + c;
-    const uint64_t bad = __builtin_amdgcn_ballot_w64(j < Nr && (fl_bad<ND>(ak[n]) || fl_bad<ND>(av[n])));
-    const bool own_bad = (bad >> c & 0x0001000100010001ull) != 0;
-    const uint32_t row = own_bad ? kOob : (uint32_t)j * tb;
+    const int j = ja + 16 * n + ec;
+    const uint64_t bad_v = __builtin_amdgcn_ballot_w64(j < Nr && fl_bad<ND>(av[n]));
+    uint64_t bad = bad_v | __builtin_amdgcn_ballot_w64(j < Nr && fl_bad<ND>(ak[n]));
+    if (__builtin_expect(bad != 0, 0) && fl_dkv_nan<T, ND>(a, ps, Gr, ja + 16 * n, el, bad_v == 0)) bad = 0;
+    const bool own_bad = (bad >> ec & 0x0001000100010001ull) != 0;  // in some lane of the row
+    const uint32_t row = (uint32_t)j * tb;
     constexpr float kUp = Sc::kOn ? 0x1p-15f : 1.0f;  // 2^-kProb
-    fl_store<T, ND>(ak[n], Sc::kOn ? a.scale * kUp / sk[n] : a.scale, dKr, row, D, g);
-    fl_store<T, ND>(av[n], kUp, dVr, row, D, g);
+    fl_store<T, ND>(ak[n], Sc::kOn ? a.scale * kUp / sk[n] : a.scale, dKr, own_bad ? kOob : row, D, eg);
+    fl_store<T, ND>(av[n], kUp, dVr, own_bad ? kOob : row, D, eg);
     if (__builtin_expect(bad != 0, 0)) {
-      for (int r = 0; r < 16; ++r)
-        if (bad >> r & 0x0001000100010001ull) fl_dkv_row<T, (ND + 1) / 2>(a, ps, ja + 16 * n + r, lane);
+      fl_dkv_rows<T, ND>(a, ps, Qr, Gr, Kr, Vr, ja + 16 * n, ec, eg, ak[n], av[n]);
+      fl_store<T, ND>(ak[n], a.scale, dKr, own_bad ? row : kOob, D, eg);
+      fl_store<T, ND>(av[n], 1.0f, dVr, own_bad ? row : kOob, D, eg);
     }
   }
 }

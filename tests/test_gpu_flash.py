@@ -307,3 +307,63 @@ def test_flash_half_keeps_small_weights(ext, N, D, left, right, size, loud, dtyp
         print(f"  {name}: error {err:.4e}, of storing alone {store:.4e}, rounded otherwise {flips:.2e}", flush=True)
         assert err <= 1.0005 * store, name
         assert dtype == torch.float16 or flips <= 1.5e-3, name
+
+
+@pytest.mark.parametrize("D", [24, 64, 128])
+@pytest.mark.parametrize("dtype", DTYPES)
+def test_flash_causal_rows_with_infinities(ext, dtype, D):
+    """An infinity in the first key's V row makes that column of every causal
+    row infinite and leaves the other columns alone; one in a query's dO makes
+    that column of dV infinite, and dK infinite or NaN, for the keys it attends
+    only."""
+    N, r = 150, 70
+    q, k, v, g = (torch.from_numpy(a).to(dtype).cuda()
+                  for a in [*qkv((1, N, 2, D), 8400 + D), randn((1, N, 2, D), 8410)])
+    tol = 1e-5 if dtype == torch.float32 else 1e-2
+    y = ext.dense_forward(q, k, v, True)
+    v2 = v.clone()
+    v2[0, 0, 1, 3] = float("inf")
+    y2 = ext.dense_forward(q, k, v2, True)
+    if D != 64 or dtype == torch.float32:  # 16-bit rows at head_dim 64 are another kernel's
+        assert bool((y2[0, :, 1, 3] == float("inf")).all())
+        y2[0, :, 1, 3] = y[0, :, 1, 3]
+        torch.testing.assert_close(y2, y, rtol=tol, atol=tol)
+    g2 = g.clone()
+    g2[0, r, 1, 3] = float("inf")
+    out, lse = ext.dense_forward(q, k, v, True, return_lse=True) if D == 64 else (None, None)
+    d1, d2 = ([t.clone() for t in ext.dense_backward(q, k, v, x, True, out=out, lse=lse)] for x in (g, g2))
+    assert not torch.isfinite(d2[0][0, r, 1]).any() and not torch.isfinite(d2[1][0, :r + 1, 1]).any()
+    assert bool((d2[2][0, :r + 1, 1, 3] == float("inf")).all())
+    d2[0][0, r, 1], d2[1][0, :r + 1, 1] = d1[0][0, r, 1], d1[1][0, :r + 1, 1]
+    d2[2][0, :r + 1, 1, 3] = d1[2][0, :r + 1, 1, 3]
+    for a, b in zip(d2, d1):
+        torch.testing.assert_close(a, b, rtol=tol, atol=tol)
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+def test_flash_bad_values_cost(ext, dtype, D):
+    """Calls in which every row is redone, as after an overflowed loss scale:
+    at most 30 times the clean call's time (one wave per row, a key at a time,
+    took 100 to 400 times).  NaN gradients leave the sums as they are."""
+    N = 2048
+    q, k, v, g = (torch.randn(1, N, 8, D, device="cuda").to(dtype) for _ in range(4))
+    v2 = v.clone()
+    v2[0, 0] = float("inf")
+
+    def time(f):
+        f()
+        a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+        a.record()
+        for _ in range(3):
+            f()
+        b.record()
+        b.synchronize()
+        return a.elapsed_time(b)
+
+    fwd, fwd2 = (time(lambda: ext.dense_forward(q, k, x, True)) for x in (v, v2))
+    out, lse = ext.dense_forward(q, k, v, True, return_lse=True) if D == 64 else (None, None)
+    bwd, bwd2, bwd3 = (time(lambda: ext.dense_backward(q, k, v, x, True, out=out, lse=lse))
+                       for x in (g, torch.full_like(g, float("inf")), torch.full_like(g, float("nan"))))
+    print(f"  forward {fwd2 / fwd:.1f}x, backward {bwd2 / bwd:.1f}x, NaN {bwd3 / bwd:.1f}x", flush=True)
+    assert fwd2 <= 30 * fwd and bwd2 <= 30 * bwd and bwd3 <= 3 * bwd
