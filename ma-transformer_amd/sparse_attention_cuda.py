@@ -383,6 +383,20 @@ def _enumerated_set(code: int, seq_len: int, device, host_table=None, tile_seg=0
     return IndexSet(offsets, keys, seq_len, device, tile_seg=tile_seg)
 
 
+def _longformer_item_blocks(seq_len: int, left: int, right: int) -> int:
+    """Blocks of a Longformer set's list that one work item walks.  The global
+    rows' tile and the global keys' block list every block of the sequence, and
+    an item walks its blocks serially: 8 (the plan's default is 32), or a window
+    tile's own list where that is longer, so that only the global ones are
+    split.  float32 gradients at 8 / 16 / 32: 12 heads of 12000 rows 354 / 436 /
+    582 us, 4 of 24576 268 / 302 / 447.  Past 24576 rows 16, whose partials cost
+    no more than they save on any head count (bf16, 12 heads of 32768 rows, forward
+    92 / 90 / 89 us, gradients 327 / 316 / 322; of 65536 198 / 178 / 172, 658 / 613
+    / 607; one head 47 / 37 / 43, 137 / 125 / 146)."""
+    window = (int(left) + int(right) + 63) // 64 + 3
+    return min(32, max(8 if seq_len <= 24576 else 16, window))
+
+
 def pattern_index_set(pattern: str, seq_len: int, device, **kw) -> IndexSet:
     """The key sets of a closed-form pattern ("block_sparse" with block_table=
     and block_size=, "longformer" with left=, right=, num_global=) as an
@@ -419,16 +433,8 @@ def pattern_index_set(pattern: str, seq_len: int, device, **kw) -> IndexSet:
     if hit is None:
         if len(_pattern_sets) > 16:
             _pattern_sets.clear()
-        # The global rows' tile and the global keys' block list every block of the
-        # sequence, and a work item walks its list serially: 8 blocks an item (the
-        # plan's default is 32), or a window tile's own list where that is longer,
-        # so that only the global ones are split.  float32 training, default ->
-        # here: 2 streams of 3422 rows 339 -> 118 us, 12 of 5976 442 -> 225, 12 of
-        # 12000 595 -> 435; bf16, 8 of 19119 rows 175 -> 170.  4 an item splits the
-        # window tiles too: 94, 199 and 423, but 289 on the bf16 one.
-        window = (int(kw["left"]) + int(kw["right"]) + 63) // 64 + 3
-        hit = _pattern_sets[key] = _enumerated_set(_ma.LONGFORMER, seq_len, device,
-                                                   tile_seg=min(32, max(8, window)), **kw)
+        hit = _pattern_sets[key] = _enumerated_set(
+            _ma.LONGFORMER, seq_len, device, tile_seg=_longformer_item_blocks(seq_len, kw["left"], kw["right"]), **kw)
     return hit
 
 

@@ -122,3 +122,12 @@ def test_index_set_builds_plan_when_keys_cluster():
     assert s2.tile_plan is None
     s3 = ext.IndexSet(torch.from_numpy(off2), torch.from_numpy(keys2), N, device="cpu", tiles=False)
     assert s3.tile_plan is None
+
+
+def test_longformer_item_blocks():
+    """Work items of Longformer sets: 8 blocks, 16 past 24576 rows, a window
+    tile's own list where that is longer, 32 at most."""
+    from sparse_attention_cuda import _longformer_item_blocks as blocks
+    assert [blocks(n, 127, 0) for n in (100, 24576, 24577, 65536)] == [8, 8, 16, 16]
+    assert blocks(4096, 600, 0) == 13 and blocks(65536, 600, 0) == 16
+    assert blocks(4096, 5000, 5000) == blocks(65536, 5000, 5000) == 32
