@@ -26,8 +26,9 @@ bool band_of(const ma_attn_desc* d, Band* b) {
     return true;
   }
   if (d->pattern != MA_ATTN_SLIDING || d->left < 0 || d->right < 0) return false;
-  const int64_t nr = (d->seq_len + d->dilation - 1) / d->dilation;
-  *b = Band{std::min(d->left, nr), std::min(d->right, nr), d->dilation, nr};
+  const int64_t dil = std::min(d->dilation, std::max<int64_t>(d->seq_len, 1));  // classes past the rows are empty
+  const int64_t nr = (d->seq_len + dil - 1) / dil;
+  *b = Band{std::min(d->left, nr), std::min(d->right, nr), dil, nr};
   return true;
 }
 
@@ -92,14 +93,17 @@ int run_pair(const ma_attn_desc* d, FlArgs a, hipStream_t st) {
 // Causal rows whose 128-row tiles are at most one per CU run in pairs, longest
 // with shortest (float32, head_dim 64, 8 heads of 4000 rows: 136 us against
 // 173 unpaired; above one tile per CU the scheduler evens the tiles out: 8000
-// rows 415 us unpaired, 442 paired).
+// rows 415 us unpaired, 442 paired), past two 64-row tiles (float32, head_dim 64,
+// 100 rows: 8.4 us, paired 10.1); not the 16-bit windows at head_dim 64 ([i-300,
+// i] on 200 rows: 6.4 us, paired 9.3).
 //
 // float32 at head_dim 33 to 64 splits every staged row into three planes, so 8
 // waves share a block once there are workgroups enough for every CU (two-sided
 // 129-key window, 8 heads of 32768 rows: 82 us against 102 with 4 waves; 2
 // heads of 600 rows: 14.7 against 11.8), and two query groups per wave pay on
 // very long rows (causal, 8 heads of 16384 rows: 1275 us against 1387; 8000
-// rows: 558 against 415).
+// rows: 558 against 415).  Sequences of one 64-row tile would leave half of the 8
+// waves idle.
 template <typename T, int ND>
 int fwd_nd(const ma_attn_desc* d, const FlArgs& a, hipStream_t st) {
   constexpr bool f32 = sizeof(T) == 4;
@@ -107,10 +111,10 @@ int fwd_nd(const ma_attn_desc* d, const FlArgs& a, hipStream_t st) {
   Band b;
   band_of(d, &b);
   const int64_t tiles128 = d->batch * d->num_heads * b.dil * ((b.nr + 127) / 128);
-  if (a.desc && tiles128 <= 256) return run_pair<T, ND, 8, KB>(d, a, st);
+  if (a.desc && b.nr > 128 && tiles128 <= 256 && (f32 || d->head_dim != 64)) return run_pair<T, ND, 8, KB>(d, a, st);
   if constexpr (f32 && ND == 2) {
     if (b.left >= b.nr && tiles128 >= 1024) return run_fwd<T, ND, 2, 8, KB, false, 2>(d, a, st);
-    if (tiles128 >= 256) return run_fwd<T, ND, 1, 8, KB, false, 2>(d, a, st);
+    if (b.nr > 64 && tiles128 >= 256) return run_fwd<T, ND, 1, 8, KB, false, 2>(d, a, st);
   }
   // head_dim 64 in 16 bits: P in 16 bits, as in the stream kernel that these
   // windows took before; four workgroups to a CU
@@ -168,7 +172,11 @@ int run_bwd(const ma_attn_desc* d, FlArgs a, hipStream_t st) {
 // straight-line code; with 256-row tiles enough for every CU (twice, for causal
 // rows, whose tiles are uneven) two row groups per wave, so that each LDS read
 // feeds two MFMAs.  8 heads, bwd_q + bwd_kv -> here: causal 2048 rows 77 -> 68 us,
-// 8192 rows 339 -> 322, 16384 rows 1180 -> 975; all pairs, 8192 rows 623 -> 472.
+// 8192 rows 339 -> 324, 16384 rows 1196 -> 980; all pairs, 8192 rows 629 -> 477.
+// The longer tiles pay on long rows only (one group / two, bf16): causal 32 heads
+// of 4096 rows 356 / 413 us, 16 of 8192 638 / 527; all pairs 400 heads of 600 rows
+// 210 / 218, 64 of 1024 94 / 77; a 256-row tile of 64 rows is mostly idle (1024
+// heads: 22 / 40).
 template <typename T, int ND>
 int bwd_nd(const ma_attn_desc* d, const FlArgs& a, hipStream_t st) {
   constexpr bool f32 = sizeof(T) == 4;
@@ -182,7 +190,8 @@ int bwd_nd(const ma_attn_desc* d, const FlArgs& a, hipStream_t st) {
   pair.desc = 0;
   if constexpr (f32 && ND == 2) {  // saved statistics: head_dim 64
     if (a.fo) {
-      if (a.desc && tiles128 <= 256) return run_bwd<T, ND, 1, 1, 8, 8, KB, NP, 2, true, false, true>(d, pair, st);
+      if (a.desc && b.nr > 128 && tiles128 <= 256)
+        return run_bwd<T, ND, 1, 1, 8, 8, KB, NP, 2, true, false, true>(d, pair, st);
       return run_bwd<T, ND, 1, 1, 4, 4, KB, NP, 2, true, false, false>(d, a, st);
     }
   }
@@ -190,12 +199,14 @@ int bwd_nd(const ma_attn_desc* d, const FlArgs& a, hipStream_t st) {
     if (a.fo) {
       if (a.desc && tiles128 > 128 && tiles128 <= 256)
         return run_bwd<T, ND, 1, 1, 8, 8, KB, 1, 2, true, true, true>(d, pair, st);
-      if (tiles256 >= (a.desc ? 512 : 256)) return run_bwd<T, ND, 2, 2, 8, 8, KB, 1, 2, true, true, false>(d, a, st);
+      if (b.nr >= (a.desc ? 8192 : 1024) && tiles256 >= (a.desc ? 512 : 256))
+        return run_bwd<T, ND, 2, 2, 8, 8, KB, 1, 2, true, true, false>(d, a, st);
       return run_bwd<T, ND, 1, 1, 4, 4, KB, 1, 3, true, true, false>(d, a, st);
     }
   }
   if constexpr (f32 && ND >= 2)
-    if (a.desc && tiles128 <= 256) return run_bwd<T, ND, 1, 1, 8, 8, KB, NP, 2, false, false, true>(d, pair, st);
+    if (a.desc && b.nr > 128 && tiles128 <= 256)
+      return run_bwd<T, ND, 1, 1, 8, 8, KB, NP, 2, false, false, true>(d, pair, st);
   return run_bwd<T, ND, 1, 1, 4, 4, KB, NP, 2, false, false, false>(d, a, st);
 }
 

@@ -103,11 +103,14 @@ namespace {
 // them again):
 //   MA_ATTN_KERNEL=rows     every launch on the generic row kernels
 //   MA_ATTN_KERNEL=band     16-bit windows on the band kernel, not the stream kernel
+//   MA_ATTN_KERNEL=flash    the kernels of flash_kernel.h wherever they can take the
+//                           call, not only where they are the faster ones
+//   MA_ATTN_KERNEL=noflash  every call on the other kernels
 //   MA_ATTN_NO_FIXED=1      forward windows on the generic stream tiles
 //   MA_ATTN_BWD_NO_FIXED=1  backward windows on the generic stream tiles
 //   MA_ATTN_BWD_UNFUSED=1   the fixed-window 16-bit backward as two launches (dQ, then dK/dV)
 struct Options {
-  bool force_rows, force_band, no_fixed, bwd_no_fixed, bwd_unfused;
+  bool force_rows, force_band, force_flash, no_flash, no_fixed, bwd_no_fixed, bwd_unfused;
 };
 
 Options read_options() {
@@ -115,6 +118,8 @@ Options read_options() {
   Options o;
   o.force_rows = k && strcmp(k, "rows") == 0;
   o.force_band = k && strcmp(k, "band") == 0;
+  o.force_flash = k && strcmp(k, "flash") == 0;
+  o.no_flash = k && strcmp(k, "noflash") == 0;
   o.no_fixed = getenv("MA_ATTN_NO_FIXED") != nullptr;
   o.bwd_no_fixed = getenv("MA_ATTN_BWD_NO_FIXED") != nullptr;
   o.bwd_unfused = getenv("MA_ATTN_BWD_UNFUSED") != nullptr;
@@ -1657,20 +1662,74 @@ bool bwd_two_blocks(int64_t L, int64_t R) {
 // [i-1000, i] 146 / 76; 4096 rows: [i-300, i] 18.1 / 14.2.  [i-32, i+31] has a
 // stream kernel of its own with the window at compile time (4 x 8 heads of
 // 8192 rows: 31.9 / 33.5).
+//
+// Short residue classes and small grids, where a 64-row tile is mostly padding or
+// the launch is over before its many stages have filled (older kernel / these, us):
+//   float32 windows at head_dim 64, against the stream kernel: on less than two
+//   tiles a CU ([i-40, i+30], 8 heads: 2048 rows 9.9 / 11.7, 4096 rows 14 / 13) and
+//   up to one tile a class ([i-64, i+64], 4096 heads: 64 rows 100 / 118, 80 rows
+//   200 / 154); against the gather kernel, up to 24 rows ([i-300, i+300], 256 heads,
+//   dilation 64: 256 rows 46 / 289; 4096 heads: 16 rows 56 / 76, 32 rows 181 / 92).
+//   16-bit ones against the stream kernel: on less than two tiles a CU, past two
+//   tiles a class ([i-100, i+100], 1000 rows 7.7 / 8.4; 128 rows 5.9 / 5.5).
+//   float32 dense rows at head_dim 64: up to 64 rows on more than two tiles a CU
+//   (2048 heads of 64 rows 40 / 61); past 128 rows on up to a tile a CU, all
+//   pairs (2048 rows of one head 85 / 92) and causal up to 256 rows (13.8 / 14.4).
+//   float32 gradients at head_dim 64: dense up to 32 rows (12.1 / 13.1 at 24 rows,
+//   16384 heads of 16 rows 355 / 392), windows on up to two tiles a CU (4096 heads
+//   of 24 rows 136 / 116).
+//   Other head_dims, against the row kernels: up to 2 rows a class in 16 bits (4096
+//   heads, head_dim 128: 12 / 16), 4 in float32 (30 / 45; gradients 120 / 137), 3 for
+//   gradients at head_dims 17 to 32 and 12 forward at 33 to 64, whose float32 blocks
+//   are the widest (62 / 73); undilated windows at head_dims up to 32 stay here (narrow
+//   kernel, 4 rows: 34 / 16).  float32 windows of up to 24 keys on few rows, which
+//   are over in one short pass there (head_dim 128, [i-3, i+3], 1000 rows: 7.6 /
+//   12.0, gradients 26 / 39; 16 keys, 2000 rows: 12 / 12), at head_dims up to 32
+//   two-sided ones (gradients, [i-3, i+3], 1000 rows: 14 / 17).
+bool flash_pays(const ma_attn_desc* d, const void* const* ptrs, bool backward) {
+  const bool f32 = d->dtype == MA_ATTN_F32, dense = d->pattern == MA_ATTN_DENSE;
+  const int64_t dil = dense ? 1 : d->dilation, D = d->head_dim, rows = d->batch * d->num_heads * d->seq_len;
+  const int64_t nr = (d->seq_len + dil - 1) / dil, tiles = d->batch * d->num_heads * dil * ((nr + 63) / 64);
+  if (D == kHeadDim) {
+    if (backward) return !(f32 && nr <= 32 && (dense || tiles <= 512));
+    if (dense) return nr <= 64 ? tiles <= 512 : nr <= 128 || tiles > 256 || (d->causal && nr > 256);
+    if (stream_applies(d, ptrs[0], ptrs[1], ptrs[2], ptrs[3]))
+      return f32 ? nr > 64 && tiles >= 512 : nr <= 128 || tiles >= 512;
+    return !f32 || nr > 24;
+  }
+  if (nr <= (!f32 ? 2 : backward && D > 16 && D <= 32 ? 3 : !backward && D > 32 && D <= 64 ? 12 : 4))
+    return !backward && !dense && dil == 1 && D <= 32;
+  if (!f32) return true;
+  const int64_t left = dense ? nr - 1 : ma::imin64(d->left, nr - 1);
+  const int64_t right = dense ? (d->causal ? 0 : nr - 1) : ma::imin64(d->right, nr - 1), keys = left + right + 1;
+  if (D <= 32)
+    return !(left > 0 && right > 0 && keys <= 8 && (backward || dil > 1) && rows * keys <= 14000);
+  if (keys > 24) return true;
+  if (backward) return rows > (keys > 1 ? 4000 : 2000) || rows * keys > 21000;
+  return rows > 4000 || rows * keys > (keys > 16 ? 11000 : 32000);
+}
+
 bool flash_route(const ma_attn_desc* d, const void* const* ptrs, int n, bool backward) {
+  if (g_opt.no_flash) return false;
   if (d->head_dim == kHeadDim) {
     const bool sliding = d->pattern == MA_ATTN_SLIDING;
     const int64_t keys = ma::imin64(d->left, 1 << 30) + ma::imin64(d->right, 1 << 30);
     if (!sliding && d->pattern != MA_ATTN_DENSE) return false;
-    if (d->dtype != MA_ATTN_F32) {
-      if (backward || !sliding) return false;
-      if (d->right == 0 ? d->left <= 256 : keys <= 48 || (d->left == 32 && d->right == 31))
-        return false;
-    } else if (sliding) {
-      if (backward ? bwd_two_blocks(d->left, d->right) : keys <= 64) return false;
-    }
+    if (d->dtype != MA_ATTN_F32 && (backward || !sliding)) return false;
+    const bool narrow = d->dtype != MA_ATTN_F32 ? (d->right == 0 ? d->left <= 256
+                                                                 : keys <= 48 || (d->left == 32 && d->right == 31))
+                        : backward ? bwd_two_blocks(d->left, d->right)
+                                   : keys <= 64;
+    if (sliding && narrow && !g_opt.force_flash) return false;
   }
-  return ma_flash::applies(d, ptrs, n);
+  return ma_flash::applies(d, ptrs, n) && (g_opt.force_flash || flash_pays(d, ptrs, backward));
+}
+
+// Dense gradients from saved statistics (head_dim 64): float32 up to 32 rows stays
+// on the per-tile kernels (1024 heads of 16 rows 27 / 32 us, of 48 rows 52 / 48).
+bool flash_saved_route(const ma_attn_desc* d, const void* const* ptrs, int n) {
+  return !g_opt.no_flash && ma_flash::applies(d, ptrs, n) &&
+         (g_opt.force_flash || !(d->dtype == MA_ATTN_F32 && d->seq_len <= 32));
 }
 
 // float32 Longformer rows whose window passes the stream kernel's ring (left >
@@ -1679,13 +1738,14 @@ bool flash_route(const ma_attn_desc* d, const void* const* ptrs, int n, bool bac
 // stream kernel with a one-key window (whose other rows the banded kernel then
 // writes over) and its merge.  The gather kernel read every key once per row,
 // a global row's keys in one wave: 12 heads of 22136 rows, window [i-252, i], 7
-// globals, 7104 us there, 223 here.
+// globals, 7104 us there, 223 here; up to 64 rows it is the faster one (13 / 16)
+// and keeps the call.
 struct LfWide {
   ma_attn_desc rows, globals;  // the banded rows as a window; the global rows' stream pass
   size_t ws_bytes;
 };
 bool lf_wide(const ma_attn_desc* d, const void* q, const void* k, const void* v, const void* o, LfWide* w) {
-  if (d->pattern != MA_ATTN_LONGFORMER || d->dtype != MA_ATTN_F32 || d->head_dim != kHeadDim || d->num_global < 1 ||
+  if (g_opt.no_flash || d->pattern != MA_ATTN_LONGFORMER || d->dtype != MA_ATTN_F32 || d->head_dim != kHeadDim || d->num_global < 1 ||
       d->num_global > kMaxGlobal || d->left < 0 || d->right < 0)
     return false;
   w->rows = w->globals = *d;
@@ -2256,8 +2316,8 @@ int forward_launch(const ma_attn_desc* desc, const void* q, const void* k, const
         rc = launch_tiles_fwd<HalfPath<_Float16>>(desc, q, k, v, o, lse, workspace, workspace_bytes, st);
         break;
     }
-  } else if (LfWide wide; !want_rows && !want_band && lf_wide(desc, q, k, v, o, &wide) && workspace &&
-                          workspace_bytes >= wide.ws_bytes) {
+  } else if (LfWide wide; !want_rows && !want_band && (desc->seq_len > 64 || g_opt.force_flash) &&
+                          lf_wide(desc, q, k, v, o, &wide) && workspace && workspace_bytes >= wide.ws_bytes) {
     rc = launch_lf_wide(wide, q, k, v, o, workspace, workspace_bytes, st);
   } else if (!want_rows && gather_applies(desc, q, k, v, o)) {
     switch (desc->dtype) {
@@ -2467,7 +2527,7 @@ int ma_attn_backward_saved(const ma_attn_desc* desc, const void* q, const void* 
                : desc->dtype == MA_ATTN_F16
                    ? launch_tiles_bwd<HalfPath<_Float16>>(desc, ptrs, workspace, st, o, lse)
                    : launch_tiles_bwd<F32BwdPath>(desc, ptrs, workspace, st, o, lse))
-      : ma_flash::applies(desc, ptrs, 8)  // dense, head_dim 64
+      : flash_saved_route(desc, ptrs, 8)
           ? ma_flash::backward(desc, ptrs, sf, o, lse, st)
           : (desc->dtype == MA_ATTN_BF16 ? launch_backward_mfma<HalfPath<__bf16>>(desc, ptrs, sf, st, o, lse)
              : desc->dtype == MA_ATTN_F16

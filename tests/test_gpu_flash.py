@@ -367,3 +367,135 @@ def test_flash_bad_values_cost(ext, dtype, D):
                        for x in (g, torch.full_like(g, float("inf")), torch.full_like(g, float("nan"))))
     print(f"  forward {fwd2 / fwd:.1f}x, backward {bwd2 / bwd:.1f}x, NaN {bwd3 / bwd:.1f}x", flush=True)
     assert fwd2 <= 30 * fwd and bwd2 <= 30 * bwd and bwd3 <= 3 * bwd
+
+
+# B, N, H, head_dim, left, right (left None: dense, causal when right == 0), dilation: both sides of every line of
+# the dispatch between these kernels and the others, and classes that are shorter than the dilation
+ROUTES = [
+    *[(2, n, 3, D, 3, 3, 4) for n in (3, 8, 12, 17, 48, 52) for D in (16, 24, 48, 96)],
+    *[(3, n, 2, D, 15, 0, 1) for n in (2, 4, 5, 12, 13) for D in (8, 48, 128)],
+    *[(3, n, 2, D, None, 0, 1) for n in (2, 5, 13) for D in (16, 40, 128)],
+    (1, 1000, 1, 96, 11, 12, 1), (1, 1000, 1, 96, 12, 12, 1), (1, 500, 1, 80, 10, 11, 1), (1, 4001, 1, 72, 1, 1, 1),
+    (1, 2001, 1, 128, 0, 0, 1), (1, 2000, 1, 16, 3, 3, 1), (1, 2001, 1, 32, 3, 3, 2), (2, 30, 2, 48, 40, 40, 100),
+    *[(2, n, 2, 64, 300, 300, 4) for n in (5, 96, 100, 130)], (2, 64, 2, 64, 64, 64, 1), (2, 65, 2, 64, 64, 64, 1),
+    (1, 4032, 8, 64, 64, 64, 1), (1, 4096, 8, 64, 40, 30, 1), (5, 40, 2, 64, 100, 0, 64), (1, 129, 2, 64, 100, 100, 1),
+    *[(2, n, 2, 64, None, 0, 1) for n in (32, 33, 64, 128, 129, 256, 257)],
+    *[(2, n, 2, 64, None, 1, 1) for n in (32, 65, 129)], (257, 64, 2, 64, None, 0, 1), (129, 129, 1, 64, None, 1, 1),
+]
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_flash_routes_agree(ext, kernel_env, dtype):
+    """The call as dispatched, on these kernels wherever they can take it, and
+    on none of them: float32 within the parity suites' tolerance, bf16 within two
+    roundings (2^-7) and, at head_dim 64, weights of 16 bits."""
+    tol = dict(rtol=1e-5, atol=2e-5) if dtype == torch.float32 else dict(rtol=2.0 ** -7, atol=2e-2)
+    for i, (B, N, H, D, left, right, dil) in enumerate(ROUTES):
+        gen = torch.Generator(device="cuda").manual_seed(i)
+        q, k, v, g = (torch.randn(B, N, H, D, generator=gen, device="cuda").to(dtype) for _ in range(4))
+        got = {}
+        for route in ("default", "flash", "noflash"):
+            kernel_env("MA_ATTN_KERNEL", route)
+            if left is None:
+                got[route] = [ext.dense_forward(q, k, v, right == 0), *ext.dense_backward(q, k, v, g, right == 0)]
+                if D == 64:
+                    out, lse = ext.dense_forward(q, k, v, right == 0, return_lse=True)
+                    got[route] += ext.dense_backward(q, k, v, g, right == 0, out=out, lse=lse)
+            else:
+                got[route] = [ext.sliding_forward(q, k, v, left, right, dil),
+                              *ext.sliding_backward(q, k, v, g, left, right, dil)]
+        for route in ("flash", "noflash"):
+            for x, y in zip(got["default"], got[route]):
+                torch.testing.assert_close(x, y, **tol, msg=lambda m: f"{ROUTES[i]} {route}: {m}")
+
+
+@pytest.mark.parametrize("N,D,left,right,dil", [(129, 64, 64, 64, 1), (700, 64, 100, 0, 2), (257, 64, None, 1, 1),
+                                               (100, 96, 3, 3, 1), (65, 48, 2, 9, 8), (12, 128, None, 0, 1),
+                                               (190, 64, None, 0, 1), (30, 64, 20, 70, 3)])
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("route", ["flash", "noflash"])
+def test_flash_forced_routes(ext, oracle, kernel_env, route, N, D, left, right, dil, dtype):
+    """Small calls on these kernels though others are faster for them, and on the
+    others (per-tile and row kernels that the dispatch reaches only for rows
+    past 2^31 bytes or 2^24 tiles), against the oracle."""
+    kernel_env("MA_ATTN_KERNEL", route)
+    shape = (2, N, 3, D)
+    arrs = [*qkv(shape, 8200 + N), randn(shape, 8210 + N)]
+    q, k, v, g = (torch.from_numpy(a).to(dtype).cuda() for a in arrs)
+    up = [t.float().cpu().numpy() for t in (q, k, v, g)]
+    spec, extra = _spec(oracle, shape, left, right, dil), []
+    if left is None:
+        y, grads = ext.dense_forward(q, k, v, right == 0), ext.dense_backward(q, k, v, g, right == 0)
+        if D == 64:
+            out, lse = ext.dense_forward(q, k, v, right == 0, return_lse=True)
+            extra = ext.dense_backward(q, k, v, g, right == 0, out=out, lse=lse)
+    else:
+        y, grads = ext.sliding_forward(q, k, v, left, right, dil), ext.sliding_backward(q, k, v, g, left, right, dil)
+    ref, want = oracle.forward(spec, *up[:3]), oracle.backward(spec, *up)
+    u = {torch.float32: 0.0, torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}[dtype]
+    mass = oracle.forward(spec, *up[:2], np.abs(up[2])) if D == 64 else 0.0  # weights of 16 bits there
+    err = np.abs(y.float().cpu().numpy() - ref)
+    assert (err <= (1e-5 if dtype == torch.float32 else 1e-4) + u * np.abs(ref) + u * mass).all(), float(err.max())
+    for name, a, b in zip(("dq", "dk", "dv") * 2, [*grads, *extra], [*want, *want]):
+        check_grad(name, a.float().cpu().numpy(), b, dtype == torch.float32)
+
+
+@pytest.mark.parametrize("N,left,right,dil", [(64, 32, 31, 1), (130, 100, 0, 1), (300, 70, 70, 2), (65, 300, 9, 3)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_band_kernel(ext, oracle, kernel_env, N, left, right, dil, dtype):
+    """16-bit windows at head_dim 64 on the band kernel (rows past the others'
+    2^31 bytes): weights and rows rounded to 16 bits."""
+    kernel_env("MA_ATTN_KERNEL", "band")
+    q, k, v = (torch.from_numpy(a).to(dtype).cuda() for a in qkv((2, N, 3, 64), 8250 + N))
+    up = [t.float().cpu().numpy() for t in (q, k, v)]
+    spec = _spec(oracle, (2, N, 3, 64), left, right, dil)
+    y = ext.sliding_forward(q, k, v, left, right, dil).float().cpu().numpy()
+    ref, mass = oracle.forward(spec, *up), oracle.forward(spec, *up[:2], np.abs(up[2]))
+    u = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}[dtype]
+    err = np.abs(y - ref)
+    assert (err <= 1e-4 + u * np.abs(ref) + u * mass).all(), float(err.max())
+
+
+# calls that 64-row tiles served 2 to 6 times slower than the kernels before them
+SHORT = [(64, 256, 4, 64, 300, 300, 64, False), (64, 10, 4, 48, 3, 3, 7, False), (64, 10, 4, 128, 3, 3, 7, True),
+         (1024, 2, 4, 128, None, 0, 1, False), (512, 64, 4, 64, None, 1, 1, False), (1, 300, 1, 128, 3, 3, 1, False)]
+
+
+@pytest.mark.parametrize("B,N,H,D,left,right,dil,backward", SHORT)
+def test_flash_dispatch_short_calls(ext, kernel_env, B, N, H, D, left, right, dil, backward):
+    """Short classes and small grids in float32 take no more than 1.3 times the
+    time of the other kernels (20 calls in a graph)."""
+    q, k, v, g = (torch.randn(B, N, H, D, device="cuda") for _ in range(4))
+
+    def call():
+        if left is None:
+            return ext.dense_backward(q, k, v, g, right == 0) if backward else ext.dense_forward(q, k, v, right == 0)
+        return ext.sliding_backward(q, k, v, g, left, right, dil) if backward else \
+            ext.sliding_forward(q, k, v, left, right, dil)
+
+    def time():
+        side = torch.cuda.Stream()
+        side.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(side):
+            call()
+        torch.cuda.current_stream().wait_stream(side)
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            for _ in range(20):
+                call()
+        graph.replay()
+        times = []
+        for _ in range(3):
+            a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            a.record()
+            graph.replay()
+            b.record()
+            b.synchronize()
+            times.append(a.elapsed_time(b))
+        return min(times)
+
+    t = time()
+    kernel_env("MA_ATTN_KERNEL", "noflash")
+    other = time()
+    print(f"  {50 * t:.1f} us, other kernels {50 * other:.1f}", flush=True)
+    assert t <= 1.3 * other
