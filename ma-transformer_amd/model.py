@@ -212,17 +212,20 @@ def _model_launch(model: "TransformerModel", src: torch.Tensor):
     if found is None:
         return None
     params, windows = found
-    D, pe = model.model_dim, model._modules["pos_encoder"]._buffers["pe"]
-    if pe.dtype != torch.float32 or pe.device != src.device or pe.shape[0] < B or pe.shape[1:] != (1, D) or \
+    D, pe, dev = model.model_dim, model._modules["pos_encoder"]._buffers["pe"], src.device
+    if pe.dtype != torch.float32 or pe.device != dev or pe.shape[0] < B or pe.shape[1:] != (1, D) or \
             not pe.is_contiguous() or pe.data_ptr() % 16:
         return None
     grad = torch.is_grad_enabled()
-    ptrs = []
+    ptrs, low = [], 0
     for p in params:
-        if p.device != src.device or p.dtype != torch.float32 or not p.is_contiguous() or (grad and p.requires_grad):
+        if p.device != dev or p.dtype != torch.float32 or not p.is_contiguous() or (grad and p.requires_grad):
             return None
         ptrs.append(p.data_ptr())
-    if (grad and src.requires_grad) or params[0].shape[1] != I or any(p % 16 for p in ptrs[1:3] + ptrs[4:]):
+        low |= ptrs[-1]
+    if (grad and src.requires_grad) or params[0].shape[1] != I:
+        return None
+    if low % 16 and any(p % 16 for p in ptrs[1:3] + ptrs[4:]):  # encoder.weight and decoder.bias may lie anywhere
         return None
     import ma_attn as _ma
     if len(windows) < 1 or len(windows) > _ma.ENCODER_MAX_LAYERS or S > _ma.LIB.ma_encoder_model_max_seq(D):
