@@ -50,13 +50,13 @@ FlArgs args_of(const ma_attn_desc* d) {
   return a;
 }
 
-template <typename T, int ND, int NQ, int NW, int KB, bool DB, int OCC, int NPB = FlElt<T>::NPB, bool GL = false>
+template <typename T, int ND, int NQ, int NW, int KB, int OCC, int NPB = FlElt<T>::NPB, bool GL = false>
 int run_fwd(const ma_attn_desc* d, FlArgs a, hipStream_t st) {
   Band b;
   band_of(d, &b);
   constexpr int QT = 16 * NQ * NW;
-  constexpr size_t shm = (size_t)(DB ? 2 : 1) * 2 * FlStage<T, ND, KB, NW>::kMat;
-  auto kern = &flash_fwd_kernel<T, ND, NQ, NW, KB, NPB, DB, OCC, GL>;
+  constexpr size_t shm = 2 * FlStage<T, ND, KB, NW>::kMat;
+  auto kern = &flash_fwd_kernel<T, ND, NQ, NW, KB, NPB, OCC, GL>;
   if (ma_host::reserve_lds(reinterpret_cast<const void*>(kern), shm, st)) return 1;
   a.tiles = (int32_t)((b.nr + QT - 1) / QT);
   const int64_t wgs = d->batch * d->num_heads * b.dil * a.tiles;
@@ -113,16 +113,16 @@ int fwd_nd(const ma_attn_desc* d, const FlArgs& a, hipStream_t st) {
   const int64_t tiles128 = d->batch * d->num_heads * b.dil * ((b.nr + 127) / 128);
   if (a.desc && b.nr > 128 && tiles128 <= 256 && (f32 || d->head_dim != 64)) return run_pair<T, ND, 8, KB>(d, a, st);
   if constexpr (f32 && ND == 2) {
-    if (b.left >= b.nr && tiles128 >= 1024) return run_fwd<T, ND, 2, 8, KB, false, 2>(d, a, st);
-    if (b.nr > 64 && tiles128 >= 256) return run_fwd<T, ND, 1, 8, KB, false, 2>(d, a, st);
+    if (b.left >= b.nr && tiles128 >= 1024) return run_fwd<T, ND, 2, 8, KB, 2>(d, a, st);
+    if (b.nr > 64 && tiles128 >= 256) return run_fwd<T, ND, 1, 8, KB, 2>(d, a, st);
   }
   // head_dim 64 in 16 bits: P in 16 bits, as in the stream kernel that these
   // windows took before; four workgroups to a CU
   if constexpr (!f32 && ND == 2)
-    if (d->head_dim == 64) return run_fwd<T, ND, 1, 4, KB, false, 4, 1>(d, a, st);
+    if (d->head_dim == 64) return run_fwd<T, ND, 1, 4, KB, 4, 1>(d, a, st);
   if constexpr (!f32 && ND == 1)
-    if (b.left + b.right < 128) return run_fwd<T, ND, 1, 4, 128, false, 3>(d, a, st);
-  return run_fwd<T, ND, 1, 4, KB, false, f32 ? 2 : 3>(d, a, st);
+    if (b.left + b.right < 128) return run_fwd<T, ND, 1, 4, 128, 3>(d, a, st);
+  return run_fwd<T, ND, 1, 4, KB, f32 ? 2 : 3>(d, a, st);
 }
 
 template <typename T>
@@ -262,8 +262,8 @@ int forward_globals(const ma_attn_desc* d, int64_t num_global, const void* q, co
   a.globals = (int32_t)num_global;
   a.desc = 0;
   if (d->batch * d->num_heads * ((d->seq_len + 127) / 128) >= 256)
-    return run_fwd<float, 2, 1, 8, 64, false, 2, FlElt<float>::NPB, true>(d, a, st);
-  return run_fwd<float, 2, 1, 4, 64, false, 2, FlElt<float>::NPB, true>(d, a, st);
+    return run_fwd<float, 2, 1, 8, 64, 2, FlElt<float>::NPB, true>(d, a, st);
+  return run_fwd<float, 2, 1, 4, 64, 2, FlElt<float>::NPB, true>(d, a, st);
 }
 
 int backward(const ma_attn_desc* d, const void* const* ptrs, float* stats, const void* fo, const float* lse,

@@ -456,9 +456,8 @@ struct FlRow {
 //
 // One workgroup (NW waves) per 16 NQ NW queries of one stream; a wave holds
 // NQ groups of 16 queries, so that every K and V operand it reads from LDS
-// feeds NQ MFMAs.  Key blocks of KB rows go through LDS (DB: two buffers, the
-// next block's loads in flight while this one computes; otherwise one buffer,
-// refilled between two barriers), softmax online in registers, rescaled only
+// feeds NQ MFMAs.  Key blocks of KB rows go through LDS (one buffer, refilled
+// between two barriers from loads issued a block earlier), softmax online in registers, rescaled only
 // when a row's maximum rose.  The running maximum is kept times scale log2(e),
 // rounded: a row whose maximum stayed is rescaled by 2^0 exactly (a difference
 // formed from the raw maximum inside one fma would leave that product's
@@ -513,16 +512,16 @@ __device__ __forceinline__ void fl_fwd_rows(const FlArgs& a, const FlPos& ps, __
 
 constexpr float kSlack = 8.0f;
 
-// GL (Longformer windows; one residue class, one buffer): after the window's
+// GL (Longformer windows; one residue class): after the window's
 // blocks one more holds the global keys, of which a row takes those before its
 // window.  Rows below `globals` are not written: they attend every key and
 // another kernel splits them.
-template <typename T, int ND, int NQ, int NW, int KB, int NPB, bool DB, int OCC, bool GL>
+template <typename T, int ND, int NQ, int NW, int KB, int NPB, int OCC, bool GL>
 __global__ __launch_bounds__(64 * NW, OCC) void flash_fwd_kernel(FlArgs a) {
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
   using St = FlStage<T, ND, KB, NW>;
   using Sc = FlScale<T, NPB>;
-  constexpr int RS = St::RS, PL = St::kPlane, MAT = St::kMat, BUF = 2 * MAT;
+  constexpr int RS = St::RS, PL = St::kPlane, MAT = St::kMat;
   constexpr int NU = KB / 16;
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -573,7 +572,6 @@ __global__ __launch_bounds__(64 * NW, OCC) void flash_fwd_kernel(FlArgs a) {
       vs.load(Vr, next, tid, tb, D);
     }
     __builtin_amdgcn_sched_barrier(0);
-    const uint8_t* buf = lds + (DB && (e & 1) ? BUF : 0);
     const bool glob = GL && e == nwin;
     const int key0 = glob ? 0 : k0 + e * KB;
     // sub-tiles [u0, u1] of the block meet some window of the wave
@@ -589,7 +587,7 @@ __global__ __launch_bounds__(64 * NW, OCC) void flash_fwd_kernel(FlArgs a) {
 #pragma unroll
       for (int u = 0; u < NU; ++u) {
         if (u >= u0 && u <= u1) {
-          fl_rowdot<T, ND, PL, NQ>(buf + u * 16 * RS + kl, qf, sc[u]);
+          fl_rowdot<T, ND, PL, NQ>(lds + u * 16 * RS + kl, qf, sc[u]);
           const int key = key0 + 16 * u;
 #pragma unroll
           for (int n = 0; n < NQ; ++n) {
@@ -654,17 +652,10 @@ __global__ __launch_bounds__(64 * NW, OCC) void flash_fwd_kernel(FlArgs a) {
           }
           pb[n].set(p0, p1);
         }
-        fl_trmul<T, ND, PL, NQ, NPB>(buf + u * 16 * RS + vl, buf + (u + 1) * 16 * RS + vl, pb, acc);
+        fl_trmul<T, ND, PL, NQ, NPB>(lds + u * 16 * RS + vl, lds + (u + 1) * 16 * RS + vl, pb, acc);
       }
     }
-    if constexpr (DB) {
-      if (e + 1 < nb) {
-        uint8_t* nx = lds + (e & 1 ? 0 : BUF);
-        ks.store(nx, tid);
-        vs.store(nx + MAT, tid);
-      }
-      __syncthreads();
-    } else if (e + 1 < nb) {
+    if (e + 1 < nb) {
       __syncthreads();
       ks.store(lds, tid);
       vs.store(lds + MAT, tid);
