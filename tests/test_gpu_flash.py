@@ -273,6 +273,23 @@ def test_flash_float32_long_rows(ext, N, D):
         assert err <= 2.0 ** -19, name
 
 
+@pytest.mark.parametrize("D", [16, 64])
+@pytest.mark.parametrize("left,right", [(100, 20), (300, 300), (5000, 0)])
+def test_flash_float32_window_error(ext, kernel_env, D, left, right):
+    """float32 windows of hundreds of keys against float64: scores, weights'
+    exponents (rounded at up to 2^-22, 2^-24 rms) and a sum rounded once per 32
+    keys each come to under 2^-23 of the result's norm, and 2^-22 together; sums
+    rounded six times per 32 keys, at 3.9e-7, do not fit."""
+    kernel_env("MA_ATTN_KERNEL", "flash")
+    N = 4096
+    q, k, v = (torch.from_numpy(a).cuda() for a in qkv((1, N, 1, D), 8995 + D))
+    y = ext.sliding_forward(q, k, v, left, right)[0, :, 0].cpu().double()
+    ref = _double(q, k, v, q, left, right)[0]
+    err = float((y - ref).norm() / ref.norm())
+    print(f"  relative error {err:.2e}", flush=True)
+    assert err <= 2.0 ** -22
+
+
 # N, head_dim, left, right (left None: every key), dO's size, rows of dO 2^10 times as large
 SMALL_GRADS = [(2048, 128, None, 0, 1e-3, None), (2048, 32, None, 0, 1e-3, None), (1500, 128, 600, 0, 1e-4, None),
                (700, 40, 100, 100, 1e-3, slice(400, 410)), (1000, 8, None, 0, 1.0, None)]
