@@ -101,7 +101,7 @@ int run_pair(const ma_attn_desc* d, FlArgs a, hipStream_t st) {
 // waves share a block once there are workgroups enough for every CU (two-sided
 // 129-key window, 8 heads of 32768 rows: 82 us against 102 with 4 waves; 2
 // heads of 600 rows: 14.7 against 11.8), and two query groups per wave pay on
-// very long rows (causal, 8 heads of 16384 rows: 1275 us against 1387; 8000
+// very long dense rows (causal, 8 heads of 16384 rows: 1275 us against 1387; 8000
 // rows: 558 against 415).  Sequences of one 64-row tile would leave half of the 8
 // waves idle.
 template <typename T, int ND>
@@ -113,7 +113,7 @@ int fwd_nd(const ma_attn_desc* d, const FlArgs& a, hipStream_t st) {
   const int64_t tiles128 = d->batch * d->num_heads * b.dil * ((b.nr + 127) / 128);
   if (a.desc && b.nr > 128 && tiles128 <= 256 && (f32 || d->head_dim != 64)) return run_pair<T, ND, 8, KB>(d, a, st);
   if constexpr (f32 && ND == 2) {
-    if (b.left >= b.nr && tiles128 >= 1024) return run_fwd<T, ND, 2, 8, KB, 2>(d, a, st);
+    if (d->pattern == MA_ATTN_DENSE && tiles128 >= 1024) return run_fwd<T, ND, 2, 8, KB, 2>(d, a, st);
     if (b.nr > 64 && tiles128 >= 256) return run_fwd<T, ND, 1, 8, KB, 2>(d, a, st);
   }
   // head_dim 64 in 16 bits: P in 16 bits, as in the stream kernel that these

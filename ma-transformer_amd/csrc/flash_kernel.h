@@ -276,9 +276,11 @@ __device__ __forceinline__ uint32_t fl_tr_lane(int c, int g) {
 // LOCAL (float32): the six products of a pair of sub-tiles are summed from zero
 // and added to acc once, so that acc is rounded once per 32 rows instead of six
 // times.  The forward up to head_dim 64 takes it: relative error at head_dim 64 of
-// [i-300, i+300] 3.9e-7 -> 1.7e-7 and of causal rows of 4096 3.9e-7 -> 1.6e-7
-// (fp32 FMA kernels before: 2.7e-7 both), for 2 to 5 % of the time; above head_dim
-// 64 the sums were closer than those kernels' already (4.0e-7 against 5.9e-7).
+// [i-300, i+300] 3.9e-7 -> 1.7e-7 and of windows over all of 4096 earlier rows
+// 3.9e-7 -> 1.6e-7 (fp32 FMA kernels before: 2.7e-7 both), for 0 to 4 % of the time.
+// Where the kernels before were further off already it is left out: above head_dim
+// 64 (4.0e-7 against 5.9e-7) and for the long dense rows of two query groups (8 heads
+// of 16384 rows 1243 us, with it 1302).
 template <typename T, int ND, int PL, int NF, int NPB = FlElt<T>::NPB, bool LOCAL = false>
 __device__ __forceinline__ void fl_trmul(const uint8_t* m0, const uint8_t* m1, const FlB<T, NPB> (&b)[NF],
                                          f32x4 (&acc)[NF][2 * ND]) {
@@ -663,7 +665,7 @@ __global__ __launch_bounds__(64 * NW, OCC) void flash_fwd_kernel(FlArgs a) {
           }
           pb[n].set(p0, p1);
         }
-        fl_trmul<T, ND, PL, NQ, NPB, ND <= 2>(lds + u * 16 * RS + vl, lds + (u + 1) * 16 * RS + vl, pb, acc);
+        fl_trmul<T, ND, PL, NQ, NPB, ND <= 2 && NQ == 1>(lds + u * 16 * RS + vl, lds + (u + 1) * 16 * RS + vl, pb, acc);
       }
     }
     if (e + 1 < nb) {
