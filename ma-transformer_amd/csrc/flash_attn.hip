@@ -82,12 +82,12 @@ int run_pair(const ma_attn_desc* d, FlArgs a, hipStream_t st) {
 
 // One query group per wave, 4 waves, 64-key blocks in one buffer: measured
 // best of 1 or 2 groups, 4 or 8 waves, 32- or 64-key blocks and one or two
-// buffers at head_dim 32 and 128 (causal 128-key window, bf16, head_dim 128,
-// 8 heads, 32768 rows: 83 us against 87-104; two-sided 64-key window, head_dim
-// 32, 4 x 8 heads, 8191 rows: f16 26 us against 28-31, f32 43 us against
-// 43-70).  16-bit windows of at most 128 keys at head_dim 32 take 128-key
-// blocks: a 64-query tile of a 64-key window is then one block (22 us against
-// 24 on the f16 window above).  float32 above head_dim 64 takes 32-key blocks
+// buffers at head_dim 32 and 128, in a first version (causal 128-key window, bf16,
+// head_dim 128, 8 heads, 32768 rows: 83 us against 87-104, 75 now; two-sided
+// 64-key window, head_dim 32, 4 x 8 heads, 8191 rows: f16 26 us against 28-31, f32
+// 43 us against 43-70, 39 now).  16-bit windows of at most 128 keys at head_dim 32
+// take 128-key blocks: a 64-query tile of a 64-key window is then one block (22 us
+// against 24 on the f16 window above, 19.5 now).  float32 above head_dim 64 takes 32-key blocks
 // (three planes of 64 rows would leave one workgroup per CU, or spill).
 //
 // Causal rows whose 128-row tiles are at most one per CU run in pairs, longest
@@ -158,9 +158,9 @@ int run_bwd(const ma_attn_desc* d, FlArgs a, hipStream_t st) {
 
 // 4 waves and 64-row blocks (float32 above head_dim 64: 32-row): measured best
 // of 4 or 8 waves and 32- or 64-row blocks (causal 128-key window, bf16,
-// head_dim 128, 2 x 8 heads, 4096 rows: 74 us against 79-88).  Two workgroups a
-// CU: registers for three cost more than they bring (same case, dQ 38 -> 41 us,
-// dK/dV 35 -> 63).
+// head_dim 128, 2 x 8 heads, 4096 rows: 74 us against 79-88; with P and dS in three
+// planes 76).  Two workgroups a CU: registers for three cost more than they bring
+// (same case, dQ 38 -> 41 us, dK/dV 35 -> 63).
 //
 // Causal rows in pairs of tiles, as in the forward: float32 above head_dim 32 on
 // at most one 128-row tile per CU (8 heads of 4096 rows: head_dim 64 628 -> 561

@@ -1641,17 +1641,18 @@ bool bwd_two_blocks(int64_t L, int64_t R) {
 //
 // Head_dims other than 64 (8 to 128, a multiple of 8): in both directions.  In
 // bf16 at head_dim 128 the row kernels took 2740 us for a causal 128-key window
-// over 8 heads of 32768 rows, these take 71 us (backward over 2 x 8 heads of
-// 4096 rows: 3017 -> 74 us); at head_dim 32 the narrow kernel took 174 us for a
-// two-sided 64-key window over 4 x 8 heads of 8191 rows (f16), these 21 us, and
-// 8.9 against 7.6 us on 4 heads of 1024 rows of 16.
+// over 8 heads of 32768 rows, these take 75 us (backward over 2 x 8 heads of
+// 4096 rows: 3017 -> 76 us); at head_dim 32 the narrow kernel took 172 us for a
+// two-sided 64-key window over 4 x 8 heads of 8191 rows (f16), these 19.5 us, and
+// 8.9 against 7.4 us on 4 heads of 1024 rows of 16.
 //
 // float32 at head_dim 64: dense rows, windows of more than 65 keys forward, and
 // windows past two 64-row blocks backward; shorter ones stay on the stream
 // kernels, which read every row once and keep a tile's scores in registers
 // (8 heads of 32768 rows, stream / these: [i-63, i] forward 65 / 62 us,
 // backward 234 / 263; [i-100, i] 114 / 80 and 466 / 344; [i-64, i+64] 121 / 82
-// and 490 / 361; dense causal, 8 heads of 4000 rows: 211 / 136 and 924 / 594).
+// and 490 / 361; dense causal, 8 heads of 4000 rows: 208 / 137 and 922 / 544; the
+// windows' forwards before their sums were taken apart, 2 to 4 % more since).
 //
 // 16-bit at head_dim 64: forward windows with a right side, past 48 keys, and
 // causal ones past 256, where the stream kernel's ring of 64-row slots leaves
@@ -2280,8 +2281,8 @@ int ma_attn_forward_noalloc(const ma_attn_desc* desc, const void* q, const void*
 namespace {
 
 // lse: optional per-row softmax statistics (ma_attn_forward_lse), written by
-// the block-row, tiled and Longformer stream kernels; other kernels refuse
-// it.
+// the block-row, tiled and Longformer stream kernels and, for float32 dense
+// rows, by the kernels of flash_kernel.h; other kernels refuse it.
 int forward_launch(const ma_attn_desc* desc, const void* q, const void* k, const void* v, void* o, float* lse,
                    void* workspace, size_t workspace_bytes, hipStream_t st) {
   (void)hipGetLastError();  // launch errors below must be ours
