@@ -6,11 +6,12 @@
 // x2 the successive bf16 roundings of what is left (24 bits in all, float32's
 // exponent range), and a product takes the six partial products whose bf16
 // planes p, p' have p + p' <= 2, smallest first; the three left out come to
-// 2^-24 of it at most (x1 reaches 2^-8 of x, x2 2^-16), 2^-27 on average.  Six 16x16x32 MFMAs take 6/16 of the time of the sixteen
-// 16x16x4 fp32 MFMAs they replace, and 64-term dot products came out closer to
-// 64-bit ones (relative error 4.6e-8 against 1.44e-7 on normal data; 7.7e-8
-// against 1.24e-7 on data spread over e^(+-9)): each MFMA rounds once per 32
-// terms instead of once per term.
+// 2^-24 of it at most (x1 reaches 2^-8 of x, x2 2^-17), 2^-27.5 rms over uniform
+// mantissas.  Six 16x16x32 MFMAs take 6/16 of the time of the sixteen 16x16x4 fp32
+// MFMAs they replace, and 64-term dot products came out closer to 64-bit ones
+// (relative error 4.6e-8 against 1.44e-7 on normal data; 7.7e-8 against 1.24e-7 on
+// data spread over e^(+-9)): each MFMA rounds once per 32 terms instead of once per
+// term.
 //
 // 16-bit inputs multiply exactly (one plane).  Probabilities and dS are float32
 // and enter their products in planes too, so that nothing but the stored
@@ -988,8 +989,8 @@ __device__ __forceinline__ void fl_dkv_rows(const FlArgs& a, const FlPos& ps, __
 // row are (dK and dV all NaN in either computation), or whose delta is NaN where
 // dV's sums are finite (v_ok; dK all NaN).
 template <typename T, int ND>
-__device__ __forceinline__ bool fl_dkv_nan(const FlArgs& a, const FlPos& ps, __amdgpu_buffer_rsrc_t Gr, int r0, int lane,
-                                           bool v_ok) {
+__device__ __forceinline__ bool fl_dkv_nan(const FlArgs& a, const FlPos& ps, __amdgpu_buffer_rsrc_t Gr, int r0,
+                                           int lane, bool v_ok) {
   bool nan_l = false;
   int w = -1;
   for (int i = max(0, r0 + 15 - a.right) + lane; i <= min(ps.Nr - 1, r0 + a.left); i += 64) {
