@@ -516,3 +516,10 @@ def test_flash_dispatch_short_calls(ext, kernel_env, B, N, H, D, left, right, di
     other = time()
     print(f"  {50 * t:.1f} us, other kernels {50 * other:.1f}", flush=True)
     assert t <= 1.5 * other
+
+
+def test_flash_launch_limit_forced(ext, kernel_env):
+    """As test_flash_launch_limit, with the banded kernels asked for: the limit,
+    not the length of the sequences, leaves the call to the row kernels."""
+    kernel_env("MA_ATTN_KERNEL", "flash")
+    test_flash_launch_limit(ext)
